@@ -453,10 +453,7 @@ int h3a_qknorm_rope(const h3a_qknorm_rope_args* a, void* stream) {
         return fail(H3A_EUNSUPPORTED, "h3a_qknorm_rope: batch %lld x seqlen %lld x %d x heads %lld rows (limits 2^31, batch 65535)",
                     (long long)a->batch, (long long)a->seqlen, n, (long long)a->heads);
     p.rows = a->batch * a->seqlen * n * a->heads;
-    p.div_heads = h3a::make_fast_div((uint32_t)a->heads);
-    p.div_tensors = h3a::make_fast_div((uint32_t)n);
-    p.div_seqlen = h3a::make_fast_div((uint32_t)a->seqlen);
-    p.div_hpg = p.div_heads;  // ungrouped output heads
+    p.div_hpg = h3a::make_fast_div((uint32_t)a->heads);  // ungrouped output heads
     hipError_t e = h3a::launch_qknorm_rope(p, (hipStream_t)stream);
     if (e != hipSuccess) return fail(H3A_ELAUNCH, "h3a_qknorm_rope: launch failed: %s", hipGetErrorString(e));
     return H3A_OK;
@@ -600,13 +597,7 @@ int h3a_qknorm_rope_pack(const h3a_qknorm_rope_pack_args* a, void* stream) {
     p.seqlen = (int32_t)a->rows; p.heads = (int32_t)a->heads; p.n_tensors = 2;
     p.head_dim = (int32_t)D; p.rotary_dim = (int32_t)R; p.w_f32 = a->w_dtype == H3A_DTYPE_F32;
     p.rows = a->rows * 2 * a->heads;
-    p.div_heads = h3a::make_fast_div((uint32_t)a->heads);
-    p.div_tensors = h3a::make_fast_div(2u);
-    p.div_seqlen = h3a::make_fast_div((uint32_t)a->rows);
     p.div_hpg = h3a::make_fast_div((uint32_t)hl);
-    // Rotary widths that are not a multiple of 16, or tables without 16-byte
-    // rows, take the generic kernel (one row per lane group, element-wise
-    // partner and table reads) in the same output layout.
     hipError_t e = h3a::launch_qknorm_rope(p, (hipStream_t)stream);
     if (e != hipSuccess) return fail(H3A_ELAUNCH, "h3a_qknorm_rope_pack: launch failed: %s", hipGetErrorString(e));
     return H3A_OK;

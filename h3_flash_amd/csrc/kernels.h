@@ -132,7 +132,7 @@ struct QkNormRopeParams {
     const float* sin;
     int64_t table_stride;
     int64_t rows;  // batch * seqlen * n_tensors * heads, < 2^31
-    FastDiv div_heads, div_tensors, div_seqlen;
+    int32_t head_first;  // first head of the launch's grid (0; set by the launcher)
     int32_t seqlen;
     int32_t heads;
     int32_t n_tensors;  // 1 (q only) or 2 (q and k)
@@ -152,8 +152,6 @@ struct QkNormRopeParams {
 };
 
 hipError_t launch_qknorm_rope(const QkNormRopeParams& p, hipStream_t stream);
-// Whether launch_qknorm_rope takes the fast (lane-group-per-token) path.
-bool qknorm_rope_fast_path(const QkNormRopeParams& p);
 
 // Destination-major q/k/v pack. Byte strides; row_bytes = head_dim * element size.
 struct PackQkvParams {

@@ -65,36 +65,26 @@ __device__ __forceinline__ int64_t head_ofs(const QkNormRopeParams& p, int h, in
     return (int64_t)g * sg + (int64_t)((uint32_t)h - g * p.div_hpg.d) * sh;
 }
 
-struct RowRef {
-    const uint16_t* x;
-    uint16_t* y;
-    uint32_t s, h, b;
-    int which;
-    bool ok;
-};
+// LDS bytes of a lane group's row in the any-R form: the row, then the start
+// of its rotary part again (at most 1.5 * 16 L bytes), then the overrun of the
+// partner reads; rows stay 16-byte aligned.
+constexpr int any_r_row_bytes(int lanes) { return (24 * lanes + 32 + 15) / 16 * 16; }
 
-__device__ __forceinline__ RowRef locate(const QkNormRopeParams& p, uint32_t row) {
-    RowRef r;
-    r.ok = row < (uint32_t)p.rows;
-    const uint32_t rr = r.ok ? row : 0u;
-    const uint32_t t = fdiv(rr, p.div_heads);
-    r.h = rr - t * p.div_heads.d;
-    const uint32_t t2 = fdiv(t, p.div_tensors);
-    r.which = (int)(t - t2 * p.div_tensors.d);
-    r.b = fdiv(t2, p.div_seqlen);
-    r.s = t2 - r.b * p.div_seqlen.d;
-    const bool second = r.which != 0;
-    r.x = (const uint16_t*)(second ? p.x[1] : p.x[0]) + (int64_t)r.b * (second ? p.x_sb[1] : p.x_sb[0]) +
-          (int64_t)r.s * (second ? p.x_ss[1] : p.x_ss[0]) + (int64_t)r.h * (second ? p.x_sh[1] : p.x_sh[0]);
-    r.y = (uint16_t*)(second ? p.y[1] : p.y[0]) + (int64_t)r.b * (second ? p.y_sb[1] : p.y_sb[0]) +
-          (int64_t)r.s * (second ? p.y_ss[1] : p.y_ss[0]) +
-          head_ofs(p, (int)r.h, second ? p.y_sh[1] : p.y_sh[0], second ? p.y_sg[1] : p.y_sg[0]);
-    return r;
-}
-
-// Fast path: R % 16 == 0 and 16-byte aligned tables, so a lane's 8 columns
+// kAnyR false: R % 16 == 0 and 16-byte aligned tables, so a lane's 8 columns
 // are either all rotary or all pass-through, its partner columns are the 8
 // columns of lane (j +- R/16), and cos/sin come in two 16-byte loads.
+// kAnyR true (any other even R, or tables at any 4-byte alignment): a lane's
+// partner columns lie across two other lanes, at any even offset. Partner of
+// c is (c + R/2) mod R, so each row goes through LDS once with the first R/2
+// columns written again from column R on: a lane's eight partners are then
+// the 16 bytes at byte 16j + R, read as five aligned dwords and shifted into
+// place by v_alignbit when R/2 is odd. A group's LDS accesses are one wave's,
+// which run in order, so rows need no barrier. Columns past R take cos 1,
+// sin -0 and a zero partner, which leaves n as it is, -0 included. The tables
+// and the partner's weights are per-lane registers shared by the block's
+// heads. Against one row per lane group with element-wise partner and table
+// loads (six dependent 2- and 4-byte loads per output), the pack of 6,240 rows
+// x 40 heads at R = 126 went from 385 to 78 us (389 MB).
 // One lane group per (token, chunk of kChunk heads): it reads the token's
 // cos/sin once and walks its heads tensor by tensor, each tensor's loads
 // issued first (with a copied third tensor, all loads of the block first);
@@ -102,7 +92,7 @@ __device__ __forceinline__ RowRef locate(const QkNormRopeParams& p, uint32_t row
 // Splitting heads over blockIdx.y keeps the grid wide for short shards with
 // many heads (a Ulysses rank's 6,240 rows x 40 heads). Every byte of x and y
 // is touched once: non-temporal accesses.
-template <int L, bool kCopy>
+template <int L, bool kCopy, bool kAnyR>
 __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(QkNormRopeParams p) {
     constexpr int kGroups = kThreads / L;
     constexpr int kChunk = kCopy ? kHeadChunkCopy : kHeadChunk;
@@ -111,7 +101,7 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
     const int s = (int)blockIdx.x * kGroups + tid / L;  // token
     const int64_t b = blockIdx.z;
     const int D = p.head_dim, R = p.rotary_dim, half = R >> 1;
-    const int hb = (int)blockIdx.y * kChunk;  // this block's heads: [hb, H)
+    const int hb = p.head_first + (int)blockIdx.y * kChunk;  // this block's heads: [hb, H)
     const int H = min(p.heads, hb + kChunk);
     const int col0 = j * 8;
     const bool on = s < p.seqlen && col0 < D;
@@ -124,7 +114,34 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
     const bool d_pow2 = (D & (D - 1)) == 0;  // then ss * inv_d == ss / D exactly
 
     float cv[8], sv[8];
-    if (on && rot) {
+    uint32_t pmask[4];  // kAnyR: partner pairs of the rotary columns
+    if constexpr (kAnyR) {
+        // Pairs of columns (R is even: a pair is rotary or not as a whole);
+        // pairs past R load the last one and drop it.
+        const int64_t trow = (int64_t)(on ? s : 0) * p.table_stride;
+        const bool pairs = (((uintptr_t)p.cos | (uintptr_t)p.sin) & 7) == 0 && (p.table_stride & 1) == 0;  // uniform
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int c = min(col0 + 2 * i, R - 2);
+            const float* cp = p.cos + trow + c;
+            const float* sp = p.sin + trow + c;
+            f32x2 cw, sw;
+            if (pairs) {
+                cw = *(const f32x2*)cp;
+                sw = *(const f32x2*)sp;
+            } else {
+                cw = f32x2{cp[0], cp[1]};
+                sw = f32x2{sp[0], sp[1]};
+            }
+            const bool in = col0 + 2 * i < R;
+            pmask[i] = in ? 0xffffffffu : 0u;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                cv[2 * i + e] = in ? cw[e] : 1.f;
+                sv[2 * i + e] = !in ? -0.f : col0 + 2 * i + e < half ? -sw[e] : sw[e];
+            }
+        }
+    } else if (on && rot) {
         const float* cp = p.cos + (int64_t)s * p.table_stride + col0;
         const float* sp = p.sin + (int64_t)s * p.table_stride + col0;
         const f32x4 c0 = *(const f32x4*)cp, c1 = *(const f32x4*)(cp + 4);
@@ -133,6 +150,18 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
         sv[0] = s0.x; sv[1] = s0.y; sv[2] = s0.z; sv[3] = s0.w; sv[4] = s1.x; sv[5] = s1.y; sv[6] = s1.z; sv[7] = s1.w;
     }
 
+    // Norm weights of the lane's partner columns.
+    auto load_wp = [&](const void* w, float* wp) __attribute__((always_inline)) {
+        if constexpr (kAnyR) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int c = min(col0 + e, R - 1);
+                wp[e] = load_w(w, c < half ? c + half : c - half, wf);
+            }
+        } else if (on && rot) {
+            load_w8(w, src * 8, wf, wp);
+        }
+    };
     // Normalise, rotate and store one row chunk (all L lanes of the group join
     // the reductions and the partner shuffle).
     auto row = [&](const i32x4& x, const float* wv, const float* wp, float eps, uint16_t* dst) __attribute__((always_inline)) {
@@ -151,7 +180,29 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
         // Partner chunk lives in lane src of the same row; with R = D = 128
         // that is lane j ^ 8 of the 16, a DPP rotation of the row.
         i32x4 praw;
-        if (L == 16 && ror8) {
+        if constexpr (kAnyR) {
+            typedef __attribute__((address_space(3))) char lds_char;
+            typedef __attribute__((address_space(3))) i32x4 lds_i32x4;
+            typedef __attribute__((address_space(3))) uint32_t lds_u32;
+            constexpr int kRowB = any_r_row_bytes(L);
+            __shared__ __attribute__((aligned(16))) char rows[kGroups * kRowB];
+            lds_char* const buf = (lds_char*)rows + tid / L * kRowB;
+            asm volatile("" ::: "memory");
+            *(lds_i32x4*)(buf + 16 * j) = x;
+            asm volatile("" ::: "memory");  // the second copy lands after the first, and over it
+            if (col0 < half) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) *(lds_u32*)(buf + 2 * R + 16 * j + 4 * i) = (uint32_t)x[i];
+            }
+            asm volatile("" ::: "memory");
+            const lds_char* const src8 = buf + ((16 * j + R) & ~3);
+            uint32_t d[5];
+#pragma unroll
+            for (int i = 0; i < 5; ++i) d[i] = *(const lds_u32*)(src8 + 4 * i);
+            const uint32_t sh = (uint32_t)(R & 2) * 8u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) praw[i] = (int)(__builtin_amdgcn_alignbit(d[i + 1], d[i], sh) & pmask[i]);
+        } else if (L == 16 && ror8) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) praw[e] = dpp<kDppRor8>(x[e]);
         } else {
@@ -160,7 +211,16 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
         }
         if (!on) return;
         float out[8];
-        if (rot) {
+        if constexpr (kAnyR) {
+            float xp[8];
+            unpack8(praw, xp);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float n = xv[e] * r * wv[e];
+                const float pn = xp[e] * r * wp[e];
+                out[e] = n * cv[e] + pn * sv[e];
+            }
+        } else if (rot) {
             float xp[8];
             unpack8(praw, xp);
 #pragma unroll
@@ -208,7 +268,7 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
         for (int which = 0; which < 2; ++which) {
             float wv[8], wp[8];
             if (on) load_w8(p.w[which], col0, wf, wv);
-            if (on && rot) load_w8(p.w[which], src * 8, wf, wp);
+            load_wp(p.w[which], wp);
 #pragma unroll
             for (int i = 0; i < kChunk; ++i) {
                 if (i >= nh) break;  // uniform
@@ -235,7 +295,7 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
                            (int64_t)s * (second ? p.y_ss[1] : p.y_ss[0]) + col0;
             float wv[8], wp[8];
             if (on) load_w8(w, col0, wf, wv);
-            if (on && rot) load_w8(w, src * 8, wf, wp);
+            load_wp(w, wp);
             i32x4 raw[kChunk];
 #pragma unroll
             for (int i = 0; i < kChunk; ++i) {
@@ -251,89 +311,29 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
     }
 }
 
-// Generic path (any even R <= D, any table alignment): one row per lane
-// group, element-wise partner and table reads. Output heads may be grouped
-// (the pack layout), and a copied third tensor goes along with the first
-// tensor's rows (each (batch, token, head) once).
-template <int L>
-__global__ __launch_bounds__(kThreads) void qknorm_rope_generic_kernel(QkNormRopeParams p) {
-    const int tid = threadIdx.x;
-    const int j = tid % L;
-    const RowRef ref = locate(p, blockIdx.x * (uint32_t)(kThreads / L) + (uint32_t)(tid / L));
-    const int D = p.head_dim, R = p.rotary_dim, half = R >> 1;
-    const int col0 = j * 8;
-    const bool active = ref.ok && col0 < D;
-    const void* w = ref.which ? p.w[1] : p.w[0];
-    const bool wf = p.w_f32 != 0;
-    float xv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (active) unpack8(*(const i32x4*)(ref.x + col0), xv);
-    float ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss += xv[e] * xv[e];
-    if constexpr (L <= 16) {
-        ss = group_sum<L>(ss);
-    } else {
-#pragma unroll
-        for (int off = L / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, L);
-    }
-    if (!active) return;
-    const float r = rsqrtf(ss / (float)D + (ref.which ? p.eps[1] : p.eps[0]));
-    float out[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int col = col0 + e;
-        float o = 0.f;
-        if (col < D) {
-            const float n = xv[e] * r * load_w(w, col, wf);
-            if (col < R) {
-                const bool first = col < half;
-                const int pc = first ? col + half : col - half;
-                const float pn = bf16_to_f32(ref.x[pc]) * r * load_w(w, pc, wf);
-                const float rt = first ? -pn : pn;
-                const float cv = p.cos[(int64_t)ref.s * p.table_stride + col];
-                const float sv = p.sin[(int64_t)ref.s * p.table_stride + col];
-                o = n * cv + rt * sv;
-            } else {
-                o = n;
-            }
-        }
-        out[e] = o;
-    }
-    i32x4 packed;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) packed[e] = (int)pack_bf16x2(out[2 * e], out[2 * e + 1]);
-    *(i32x4*)(ref.y + col0) = packed;
-    if (p.xc != nullptr && ref.which == 0) {
-        const uint16_t* xc = (const uint16_t*)p.xc + (int64_t)ref.b * p.xc_sb + (int64_t)ref.s * p.xc_ss +
-                             (int64_t)ref.h * p.xc_sh + col0;
-        uint16_t* yc = (uint16_t*)p.yc + (int64_t)ref.b * p.yc_sb + (int64_t)ref.s * p.yc_ss +
-                       head_ofs(p, (int)ref.h, p.yc_sh, p.yc_sg) + col0;
-        *(i32x4*)yc = *(const i32x4*)xc;
-    }
-}
-
-template <int L>
-hipError_t launch_l(const QkNormRopeParams& p, bool fast, hipStream_t stream) {
-    if (fast) {
-        const int64_t batch = p.rows / ((int64_t)p.seqlen * p.n_tensors * p.heads);
-        const int chunk = p.xc != nullptr ? kHeadChunkCopy : kHeadChunk;
-        const dim3 grid((unsigned)((p.seqlen + kThreads / L - 1) / (kThreads / L)), (unsigned)((p.heads + chunk - 1) / chunk),
+template <int L, bool kAnyR>
+hipError_t launch_l(QkNormRopeParams p, hipStream_t stream) {
+    const int64_t batch = p.rows / ((int64_t)p.seqlen * p.n_tensors * p.heads);
+    const int chunk = p.xc != nullptr ? kHeadChunkCopy : kHeadChunk;
+    const int chunks = (p.heads + chunk - 1) / chunk;
+    // (Head chunks past the grid's 65,535 in y go into further launches.)
+    for (int first = 0; first < chunks; first += 65535) {
+        p.head_first = first * chunk;
+        const dim3 grid((unsigned)((p.seqlen + kThreads / L - 1) / (kThreads / L)), (unsigned)min(chunks - first, 65535),
                         (unsigned)batch);
         if (p.xc != nullptr)
-            hipLaunchKernelGGL((qknorm_rope_kernel<L, true>), grid, dim3(kThreads), 0, stream, p);
+            hipLaunchKernelGGL((qknorm_rope_kernel<L, true, kAnyR>), grid, dim3(kThreads), 0, stream, p);
         else
-            hipLaunchKernelGGL((qknorm_rope_kernel<L, false>), grid, dim3(kThreads), 0, stream, p);
-    } else {
-        const int64_t per_block = kThreads / L;
-        const unsigned blocks = (unsigned)((p.rows + per_block - 1) / per_block);
-        hipLaunchKernelGGL((qknorm_rope_generic_kernel<L>), dim3(blocks), dim3(kThreads), 0, stream, p);
+            hipLaunchKernelGGL((qknorm_rope_kernel<L, false, kAnyR>), grid, dim3(kThreads), 0, stream, p);
     }
     return hipGetLastError();
 }
 
 }  // namespace
 
-bool qknorm_rope_fast_path(const QkNormRopeParams& p) {
+// Whether a lane's columns, partners and table values come in whole 16-byte
+// pieces (the form without LDS).
+static bool rotary_in_lanes(const QkNormRopeParams& p) {
     if (p.rotary_dim == 0) return true;
     const bool aligned = ((uintptr_t)p.cos % 16 == 0) && ((uintptr_t)p.sin % 16 == 0) && (p.table_stride % 4 == 0);
     return (p.rotary_dim % 16 == 0) && aligned;
@@ -341,17 +341,17 @@ bool qknorm_rope_fast_path(const QkNormRopeParams& p) {
 
 hipError_t launch_qknorm_rope(const QkNormRopeParams& p, hipStream_t stream) {
     if (p.rows <= 0) return hipSuccess;
-    const bool fast = qknorm_rope_fast_path(p);
+    const bool lanes16 = rotary_in_lanes(p);
     int lanes = 1;
     while (lanes * 8 < p.head_dim) lanes <<= 1;
     switch (lanes) {
-        case 1: return launch_l<1>(p, fast, stream);
-        case 2: return launch_l<2>(p, fast, stream);
-        case 4: return launch_l<4>(p, fast, stream);
-        case 8: return launch_l<8>(p, fast, stream);
-        case 16: return launch_l<16>(p, fast, stream);
-        case 32: return launch_l<32>(p, fast, stream);
-        case 64: return launch_l<64>(p, fast, stream);
+        case 1: return lanes16 ? launch_l<1, false>(p, stream) : launch_l<1, true>(p, stream);
+        case 2: return lanes16 ? launch_l<2, false>(p, stream) : launch_l<2, true>(p, stream);
+        case 4: return lanes16 ? launch_l<4, false>(p, stream) : launch_l<4, true>(p, stream);
+        case 8: return lanes16 ? launch_l<8, false>(p, stream) : launch_l<8, true>(p, stream);
+        case 16: return lanes16 ? launch_l<16, false>(p, stream) : launch_l<16, true>(p, stream);
+        case 32: return lanes16 ? launch_l<32, false>(p, stream) : launch_l<32, true>(p, stream);
+        case 64: return lanes16 ? launch_l<64, false>(p, stream) : launch_l<64, true>(p, stream);
         default: return hipErrorInvalidValue;
     }
 }

@@ -165,3 +165,29 @@ def test_full_size_workload(name):
     for got, x in ((oq, raw["q_raw"]), (ok, raw["k_raw"])):
         ref = qknorm_rope_reference(x, raw["w_q"], raw["cos"], raw["sin"], raw["eps"])
         assert_rounding_parity(got, ref, name)
+
+
+# Widths whose partners lie across lanes: half even and odd, every lane count,
+# one lane, a lane straddling R/2 or R, columns past the head in the last lane
+# group; tables read in pairs and (odd row stride, or a base one float off)
+# one value at a time. 13 heads: two head chunks, the second partial.
+@pytest.mark.parametrize(
+    "D,R", [(8, 2), (8, 6), (8, 8), (16, 14), (24, 10), (24, 24), (64, 40), (128, 4), (128, 66), (128, 126), (136, 130),
+            (256, 254), (512, 510)]
+)
+@pytest.mark.parametrize("tables", ["pairs", "odd stride", "odd base"])
+def test_partners_across_lanes(D, R, tables):
+    B, S, H = 2, 21, 13
+    x = _rand((B, S, H, D), D + R, 1.5)
+    w = torch.randn(D, generator=torch.Generator().manual_seed(R)).to(torch.bfloat16)
+    ang = torch.randn((S, R), generator=torch.Generator().manual_seed(12))
+    cos, sin = ang.cos().to(DEV), ang.sin().to(DEV)
+    if tables != "pairs":
+        pad = 1 if tables == "odd stride" else 2
+        wide = [torch.full((S, R + pad), float("nan"), device=DEV) for _ in range(2)]
+        at = pad - 1
+        for dst, src in zip(wide, (cos, sin)):
+            dst[:, at : at + R] = src
+        cos, sin = (t[:, at : at + R] for t in wide)
+    y = fused_qknorm_rope(x.to(DEV), w.to(DEV), cos, sin, 1e-5)
+    assert_rounding_parity(y, qknorm_rope_reference(x, w, cos.cpu(), sin.cpu(), 1e-5), (D, R, tables))
