@@ -799,10 +799,9 @@ int h3a_proj_gemm(const h3a_proj_args* a, void* stream) {
         d.w_rs = s.weight_stride * 2;
         d.y_rs = s.y_stride * 2;
         d.n = (int32_t)s.n;
-        d.tiles = (int32_t)((s.n + tile - 1) / tile);
         d.mode = s.mode;
         d.eps = s.eps;
-        n_tiles += d.tiles;
+        n_tiles += (s.n + tile - 1) / tile;
     }
     if (any_norm && R > 0) {
         if (!a->cos || !a->sin) return fail(H3A_EINVAL, "%s: NULL cos/sin table", fn);
@@ -827,20 +826,9 @@ int h3a_proj_gemm(const h3a_proj_args* a, void* stream) {
         p.rotary_dim = 0;
         p.seqlen = 1;
     }
-    // Sections without RoPE store their rows straight from registers, unless
-    // the launch has RoPE sections or writes rows of 16 KiB or more: then
-    // they stage them in LDS and write whole 256-byte pieces past the
-    // caches, like the RoPE sections (the 40-head q/k/v launch 0.6% faster,
-    // three plain 5,120-wide sections 3.8%; one such section measured 0.8%
-    // slower staged).
-    int64_t out_row_bytes = 0;
-    for (int i = 0; i < a->num_sections; ++i) out_row_bytes += a->sections[i].n * 2;
-    p.stage_plain = (any_norm && R > 0) || out_row_bytes >= 16384 ? 1 : 0;
     if (a->m == 0) return H3A_OK;
-    p.m_tiles = (int32_t)((a->m + tile - 1) / tile);
-    p.n_tiles = (int32_t)n_tiles;
-    if ((int64_t)p.m_tiles * n_tiles >= ((int64_t)1 << 31)) return fail(H3A_EUNSUPPORTED, "%s: grid too large", fn);
-    hipError_t e = h3a::launch_proj_gemm(p, (hipStream_t)stream);
+    if ((a->m + tile - 1) / tile * n_tiles >= ((int64_t)1 << 31)) return fail(H3A_EUNSUPPORTED, "%s: grid too large", fn);
+    hipError_t e = h3a::launch_proj_gemm(p, device_cus(), (hipStream_t)stream);
     if (e != hipSuccess) return fail(H3A_ELAUNCH, "%s: launch failed: %s", fn, hipGetErrorString(e));
     return H3A_OK;
 }

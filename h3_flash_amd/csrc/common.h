@@ -91,4 +91,38 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, b);
 }
 
+// Rotary partners of a row of up to 8 * lanes bf16 columns held 16 bytes per
+// lane (lane j of the group: columns 8j .. 8j+7), for any even rotary width R.
+// The partner of column c < R is column (c + R/2) mod R, so the row goes to
+// the group's LDS buffer with its first R/2 columns written again from column
+// R on: the eight partners of lane j are then the 16 bytes at byte 16j + R,
+// read as five aligned dwords and shifted into place by v_alignbit when R/2
+// is odd. (Lanes past R get bytes without meaning.) A group lies in one wave,
+// whose LDS accesses run in order: no barrier, and the buffer can be reused at
+// once; the memory clobbers keep the compiler from reordering across them.
+constexpr int any_r_row_bytes(int lanes) { return (24 * lanes + 32 + 15) / 16 * 16; }
+typedef __attribute__((address_space(3))) char lds_bytes;
+
+__device__ __forceinline__ i32x4 any_r_partners(lds_bytes* buf, const i32x4& x, int j, int R) {
+    typedef __attribute__((address_space(3))) i32x4 lds_i32x4;
+    typedef __attribute__((address_space(3))) uint32_t lds_u32;
+    asm volatile("" ::: "memory");
+    *(lds_i32x4*)(buf + 16 * j) = x;
+    asm volatile("" ::: "memory");  // the second copy lands after the first, and over it
+    if (16 * j < R) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *(lds_u32*)(buf + 2 * R + 16 * j + 4 * i) = (uint32_t)x[i];
+    }
+    asm volatile("" ::: "memory");
+    const lds_bytes* const src = buf + ((16 * j + R) & ~3);
+    uint32_t d[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) d[i] = *(const lds_u32*)(src + 4 * i);
+    const uint32_t sh = (uint32_t)(R & 2) * 8u;
+    i32x4 p;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) p[i] = (int)__builtin_amdgcn_alignbit(d[i + 1], d[i], sh);
+    return p;
+}
+
 }  // namespace h3a

@@ -236,7 +236,7 @@ struct ProjSection {
     void* y;             // bf16 (m, n), y_rs bytes per row
     int64_t w_rs, y_rs;
     int32_t n;           // features, a multiple of 128
-    int32_t tiles;       // ceil(n / 256)
+    int32_t tiles;       // feature tiles (set by the launcher)
     int32_t mode;
     float eps;
 };
@@ -245,7 +245,9 @@ struct ProjGemmParams {
     const void* x;  // bf16 (m, k), x_rs bytes per row
     int64_t x_rs;
     int32_t m, k;   // k a multiple of proj_gemm_k_multiple()
-    int32_t m_tiles, n_tiles;  // n_tiles = sum of the sections' tiles
+    // Set by the launcher: token tiles, the sections' feature tiles together,
+    // and the token tiles of a group of the tile order.
+    int32_t m_tiles, n_tiles, group_m;
     int32_t n_sections;
     ProjSection sec[kProjMaxSections];
     const float* cos;  // fp32 (seqlen, table_stride) tables (norm sections with rotary_dim > 0)
@@ -253,16 +255,14 @@ struct ProjGemmParams {
     int64_t table_stride;
     int32_t rotary_dim;
     int32_t seqlen;  // token m uses table row m % seqlen
-    int32_t stage_plain;  // 1: sections without RoPE stage their rows in LDS like the RoPE sections
-    // 1: the RoPE epilogue reads cos / sin at every rotated column and takes
-    // the partners from the token's other lanes (any even rotary_dim, tables
-    // in any form, 4-byte aligned); 0: rotary_dim a multiple of 32 with
-    // rotate-half tables, 16-byte aligned, read at their first half only.
+    // 1: cos / sin are read at every rotated column (any even rotary_dim,
+    // tables in any form); 0: rotate-half tables (columns c and c +
+    // rotary_dim / 2 equal), of which the first half is enough.
     int32_t rope_full_tables;
 };
-int proj_gemm_tile();
+int proj_gemm_tile();        // the largest tile's extent in features and in tokens
 int proj_gemm_k_multiple();  // k must be a multiple of this
-hipError_t launch_proj_gemm(const ProjGemmParams& p, hipStream_t stream);
+hipError_t launch_proj_gemm(ProjGemmParams p, int cus, hipStream_t stream);
 
 // Clock sample (clock.hip): H3A_CLOCK_RECORDS records of 4 uint64 at out.
 hipError_t launch_clock_sample(uint64_t* out, hipStream_t stream);

@@ -15,23 +15,22 @@
 // 32 K) and the X fragment the B operand (32 K x 16 tokens), so every lane of
 // the result holds one token and 4 consecutive features per 16-feature block.
 //
-// Tiling: one workgroup = 4 waves = 256 features x 256 tokens, one wave per
-// SIMD. Wave (wn, wm) owns features wn*128 .. +128 (one head) and tokens
-// wm*128 .. +128: 8 x 8 MFMA blocks, 256 fp32 accumulators per lane (the
-// accumulation registers), 16 fragment reads of 1 KB per 64 MFMAs.
+// Tiling: one workgroup of 4 waves per CU computes TF features x 16*NT tokens
+// (proj_gemm_kernel<TF, NT, SW, SX>), one wave per SIMD. Large tiles split the waves
+// 2 x 2 (128 features x 8*NT tokens each), small ones 4 x 1 (TF/4 features x
+// all tokens), whichever reads fewer LDS bytes per MFMA; the accumulators are
+// held in the accumulation registers (256 per lane at TF = 256, NT = 16).
 //
-// K advances 64 at a time through two LDS buffers of 32 KB per operand,
-// filled HBM -> LDS by buffer_load ... lds (16 bytes per lane, no VGPR
+// K advances 64 at a time through rings of SW (W rows) and SX (X rows) LDS
+// stages, as many as fit in 160 KB, filled HBM -> LDS by buffer_load ... lds (16 bytes per lane, no VGPR
 // staging; each load covers whole 128-byte lines of 8 rows). LDS rows are 128
 // bytes; the 16-byte chunk c of row r sits at c ^ ((r >> 1) & 7), so the 16
 // rows a quarter-wave's fragment read touches hit 16 distinct bank groups.
-// One barrier per K step of 64, in its middle: before it the wave waits for
-// its own DMA of the next K step (issued during the previous step's second
-// half, about 2,000 MFMA cycles earlier) and for its reads of the current
-// buffer; after it the next step's fragments are read, and the step after
-// next is loaded into the buffer just released, under the second half's
-// MFMAs.
+// One barrier per K step of 64, in its middle (see the step below).
 #include <math.h>
+
+#include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "kernels.h"
@@ -39,28 +38,15 @@
 namespace h3a {
 namespace {
 
-constexpr int kPT = 256;                  // tile extent in features and in tokens
 constexpr int kPK = 64;                   // K per stage (two MFMA K steps of 32)
-constexpr int kPStages = 2;
 constexpr int kPWaves = 4;
 constexpr int kPThreads = kPWaves * 64;
 constexpr int kPRow = kPK * 2;            // LDS bytes per tile row
-constexpr int kPTile = kPT * kPRow;       // 32 KB per operand per stage
-constexpr int kPXBase = kPStages * kPTile;  // X stages follow the W stages
-constexpr int kPLds = 2 * kPStages * kPTile;
-constexpr int kPDmaPerOp = kPT * kPRow / 1024 / kPWaves;  // 1 KB loads per wave per operand and stage
-static_assert(kPDmaPerOp == 8, "DMA map below assumes eight loads per operand");
 
 typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
-typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
-typedef __attribute__((address_space(3))) float lds_f32;
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
+typedef __attribute__((address_space(3))) i32x4 lds_i32x4;
+typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
 
 // vmcnt(N) and lgkmcnt(0): the wave's own DMA loads beyond the newest N have
 // landed and its LDS reads have completed.
@@ -79,33 +65,38 @@ __device__ __forceinline__ void mfma_acc(f32x4& acc, const bf16x8& a, const bf16
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
-// acc = A B (the first K step of a tile: no accumulator to read).
-__device__ __forceinline__ void mfma_first(f32x4& acc, const bf16x8& a, const bf16x8& b) {
-    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
+// f(0), ..., f(N - 1) with compile-time indices.
+template <int... I, typename F>
+__device__ __forceinline__ void static_for_seq(std::integer_sequence<int, I...>, F&& f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_seq(std::make_integer_sequence<int, N>{}, f);
 }
 
 // Section i of the launch, selected field by field (indexing the kernel
 // argument with a runtime index would copy the whole argument block into
 // private memory).
 __device__ __forceinline__ ProjSection section(const ProjGemmParams& p, int i) {
-    ProjSection s = p.sec[0];
-    if (i == 1) s = p.sec[1];
-    if (i == 2) s = p.sec[2];
-    return s;
+    auto pick = [&](auto f0, auto f1, auto f2) { return i == 0 ? f0 : i == 1 ? f1 : f2; };
+#define H3A_FIELD(f) pick(p.sec[0].f, p.sec[1].f, p.sec[2].f)
+    return ProjSection{H3A_FIELD(w),    H3A_FIELD(bias), H3A_FIELD(norm_w), H3A_FIELD(y),    H3A_FIELD(w_rs),
+                       H3A_FIELD(y_rs), H3A_FIELD(n),    H3A_FIELD(tiles),  H3A_FIELD(mode), H3A_FIELD(eps)};
+#undef H3A_FIELD
 }
 
-// Tile t of the grouped order: groups of kGroupM token tiles x every feature
+// Tile t of the grouped order: groups of p.group_m token tiles x every feature
 // tile, token tile fastest.
 struct TileCoord {
-    int sec;   // section of the feature tile
-    int f0;    // first feature of the tile, within the section
-    int m0;    // first token of the tile
+    int sec;  // section of the feature tile
+    int f0;   // first feature of the tile, within the section
+    int m0;   // first token of the tile
 };
-constexpr int kGroupM = 2;
-__device__ __forceinline__ TileCoord tile_coord(const ProjGemmParams& p, int tile) {
-    const int in_group = kGroupM * p.n_tiles;
-    const int first_m = (tile / in_group) * kGroupM;
-    const int group_m = min(p.m_tiles - first_m, kGroupM);
+__device__ __forceinline__ TileCoord tile_coord(const ProjGemmParams& p, int tile, int tile_f, int tile_m) {
+    const int in_group = p.group_m * p.n_tiles;
+    const int first_m = (tile / in_group) * p.group_m;
+    const int group_m = min(p.m_tiles - first_m, p.group_m);
     const int mt = first_m + (tile % in_group) % group_m;
     int nt = (tile % in_group) / group_m;
     int sec = 0;
@@ -117,414 +108,316 @@ __device__ __forceinline__ TileCoord tile_coord(const ProjGemmParams& p, int til
             sec = 2;
         }
     }
-    return TileCoord{sec, nt * kPT, mt * kPT};
+    return TileCoord{sec, nt * tile_f, mt * tile_m};
 }
 
-// Where one tile's operands come from: the W and X buffer resources (based at
-// the tile's first row; rows past the section or the token range are outside
-// their records and load as zeros) and the per-lane part of the W offsets.
-struct TileSrc {
-    i32x4 rw, rx;
-    uint32_t dw[2];
-    int32_t w_rs;
+__device__ __forceinline__ void unpack8(const i32x4& raw, float* f) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        f[2 * i] = __uint_as_float((uint32_t)raw[i] << 16);
+        f[2 * i + 1] = __uint_as_float((uint32_t)raw[i] & 0xffff0000u);
+    }
+}
+
+// A tile shape: TF features x 16*NT tokens; SW stages of W rows, SX of X rows.
+template <int TF, int NT, int SW, int SX>
+struct Tile {
+    static constexpr int kTokens = 16 * NT;
+    // Waves over features x tokens. LDS reads per MFMA K step: 2 x 2 reads
+    // 4 * (8 + NT/2) KB, 4 x 1 reads 4 * (TF/64 + NT) KB.
+    static constexpr int WN = TF == 256 && NT >= 10 ? 2 : 4, WM = kPWaves / WN;
+    static constexpr int NA = TF / 16 / WN, NB = NT / WM;  // 16 x 16 MFMA blocks of a wave
+    static constexpr int kWBytes = TF * kPRow, kXBytes = kTokens * kPRow;
+    static constexpr int kXBase = SW * kWBytes, kStages = kXBase + SX * kXBytes;  // X stages follow the W stages
+    // DMA loads (1 KB: 8 rows) per wave and stage
+    static constexpr int kLoadsW = TF / 8 / kPWaves, kLoadsX = kTokens / 8 / kPWaves;
+    // Epilogue: the tile's bf16 output rows over the (then idle) stages, and
+    // a row buffer per 16-lane group for RoPE partners across lanes.
+    static constexpr int kOutRow = TF * 2;
+    static constexpr int kOutBytes = kTokens * kOutRow;
+    static constexpr int kPartner = any_r_row_bytes(16);
+    static constexpr int kEpiBytes = kOutBytes + kPThreads / 16 * kPartner;
+    static constexpr int kLds = kStages > kEpiBytes ? kStages : kEpiBytes;
+    static_assert(NT % 2 == 0 && TF % 128 == 0, "DMA map: whole loads per wave");
+    static_assert(NB * WM == NT && NA * NB >= 4, "wave map; an accumulator is next used 4 MFMAs later at the least");
+    static_assert(SX >= 2 && SW > SX, "the waits below count loads in this order");
+    static_assert(kLds <= 160 * 1024, "LDS of one workgroup");
 };
 
-// Epilogue LDS use: the output rows of RoPE sections, over the stage memory
-// once the K loop is done: per wave 128 tokens x 256 bytes, the 8-byte chunk
-// c of row r at c ^ (r mod 32), so that the 16 rows of a quarter-wave's
-// writes fall in distinct bank pairs.
-constexpr int kPOutWave = 128 * 256;
-// RoPE epilogue with partners in other lanes: per wave, one token block's
-// bf16 projection rows (16 tokens x 256 bytes), past the stage memory.
-constexpr int kPRowsWave = 16 * 256;
-constexpr int kPSmem = kPLds + kPWaves * kPRowsWave;
-static_assert(kPWaves * kPOutWave <= kPLds, "output rows fit the stage memory");
-static_assert(kPSmem <= 160 * 1024, "LDS of one workgroup");
-
-// Epilogue of one tile: bias, then per section mode the plain value or the
-// RMSNorm + norm weight + RoPE of each 128-feature head, rounded once to
-// bf16. RoPE sections, and every section of a launch with RoPE sections or
-// 16 KiB output rows (p.stage_plain), put their values into the wave's LDS
-// rows first, which then go out as non-temporal 16-byte stores (4 token rows
-// of 256 bytes per instruction); the others store straight from registers
-// (lane pairs trade halves so each lane holds 8 consecutive features). The waves work
-// independently (no barrier); `active` is false for the wave whose head
-// lies past the section. The RoPE tables are in the rotate-half form
-// (columns c and c + R/2 equal), so only their first R/2 columns are read,
-// each lane loading its own token's values into registers one token block
-// ahead.
-__device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoord& tc, const f32x4 (&acc)[8][8],
-                                         int wave, int wn, int wm, int lane, char* smem) {
+// Epilogue of one tile, in two passes. First every wave adds the bias to its
+// accumulators, rounds to bf16 (as the module's linear outputs it) and writes
+// the values into the tile's output rows in LDS: token t, head h of the tile
+// (128 features) at byte t * 2 TF + 256 h, its 16-byte chunk c at c ^ (t & 15)
+// (both passes bank-conflict free). Then 16 lanes take one (token, head) row
+// at a time, 16 bytes each: plain rows go out as they are; norm rows are
+// RMS-normalised in fp32 (sum of squares over the 16 lanes by DPP), scaled by
+// the norm weight, rotated and rounded once more, as the reference's separate
+// steps do (dense_fa4.py:123-140, transformer.py:146-173; normalising the
+// unrounded accumulator moves the LSE of the attention that follows by up to
+// about 2e-3 against that order). Rows go out as whole 256-byte pieces,
+// non-temporal (no later tile reads them). RoPE partners c +- R/2: with R a
+// multiple of 16 another lane's 8 columns, read from the row in LDS;
+// otherwise any_r_partners. cos / sin of the next token are loaded before the
+// current one is computed, once for the heads of the tile.
+// Bound by VALU issue (one wave per SIMD, the matrix cores idle): row-wise it
+// needs about 90 instructions per four rows, roughly 5 us of a 256 x 256 tile
+// at R = 128 where a head's columns in the accumulator layout (4 lanes x 32
+// columns) took 13, and R = 126 costs little more (element-wise partner and
+// table reads there: 332 us for the q/k/v launch of 1,296 tokens x 40 heads,
+// now 200 with the tile shape of that launch). The longest launches hardly
+// gain (6,240 tokens: 741 -> 742 us): there the clock follows the power drawn.
+template <typename T>
+__device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoord& tc, const f32x4 (&acc)[T::NA][T::NB],
+                                         int wn, int wm, int tid, char* smem) {
+    constexpr int kHeads = T::kOutRow / 256;
     // Opaque here, so that no lane-derived value of the epilogue is hoisted
     // and held (or spilled) across the K loop.
-    asm volatile("" : "+v"(lane));
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
     const ProjSection sec = section(p, tc.sec);
-    // Lane l holds, for token block b (token wm*128 + 16b + (l & 15)) and
-    // feature block a, features wn*128 + 16a + 4*(l >> 4) + e in acc[a][b][e]:
-    // 32 of a head's 128 features; lanes l ^ 16, l ^ 32 and l ^ 48 hold the
-    // other 96.
-    const int f_head = tc.f0 + wn * 128;  // first feature of this wave's head, within the section
-    const bool active = f_head < sec.n;   // false: the half of a 128-feature last tile past the section
-    const bool norm = sec.mode != 0;
-    const int R = norm ? p.rotary_dim : 0;
-    const int fl = 4 * (lane >> 4);
-    const int j16 = lane & 15;
-    const int f_safe = active ? f_head : 0;
-    const int seqlen = p.seqlen;
-    const int m_head = tc.m0 + wm * 128;  // first token of the wave
-
-    // RoPE tables straight into registers: for token block b the lane loads,
-    // from its token's rows (wrapped per sequence), the first-half columns
-    // 16*ta + fl .. +3 of cos and sin for each rotated block pair ta. The
-    // loads of block b+1 are issued before block b is computed; the RoPE
-    // path issues no stores until its rows are complete, so each wait is for
-    // the tables alone (one counter covers loads and stores).
-    const uint32_t tab_bytes = (uint32_t)((int64_t)seqlen * p.table_stride * 4);
-    const auto rcos = make_rsrc(p.cos, tab_bytes);
-    const auto rsin = make_rsrc(p.sin, tab_bytes);
-    const uint32_t row_bytes = (uint32_t)(p.table_stride * 4);
-    auto tab_offset = [&](int b) __attribute__((always_inline)) {
-        int s = m_head + 16 * b + j16;
-        s = s < seqlen ? s : s % seqlen;
-        return (uint32_t)s * row_bytes + (uint32_t)fl * 4u;
-    };
-    const bool rope = R > 0;
-    const bool staged = rope || p.stage_plain != 0;  // rows go out through LDS
-
-    // Bias and norm weight of the lane's features (bf16, widened to fp32).
-    const bool has_bias = sec.bias != nullptr;
-    float bias[8][4], nw[8][4];
+    lds_char* const out = (lds_char*)smem;
+    {
+        // Lane l holds, for token block b (token 16 (NB wm + b) + (l & 15)) and
+        // feature block a, features 16 (NA wn + a) + 4 * (l >> 4) + e.
+        const int f_wave = 16 * T::NA * wn, q = lane >> 4;
+        const bool has_bias = sec.bias != nullptr;
+        lds_char* const row = out + (16 * T::NB * wm + (lane & 15)) * T::kOutRow + (f_wave >> 7) * 256 + (q & 1) * 8;
+        const int swz = ((lane & 15) ^ (q >> 1)) << 4;
 #pragma unroll
-    for (int a = 0; a < 8; ++a) {
-        const i32x2 br = has_bias ? *(const i32x2*)((const uint16_t*)sec.bias + f_safe + 16 * a + fl) : i32x2{0, 0};
-        const i32x2 wr = norm ? *(const i32x2*)((const uint16_t*)sec.norm_w + 16 * a + fl) : i32x2{0, 0};
-        bias[a][0] = __uint_as_float((uint32_t)br.x << 16);
-        bias[a][1] = __uint_as_float((uint32_t)br.x & 0xffff0000u);
-        bias[a][2] = __uint_as_float((uint32_t)br.y << 16);
-        bias[a][3] = __uint_as_float((uint32_t)br.y & 0xffff0000u);
-        nw[a][0] = __uint_as_float((uint32_t)wr.x << 16);
-        nw[a][1] = __uint_as_float((uint32_t)wr.x & 0xffff0000u);
-        nw[a][2] = __uint_as_float((uint32_t)wr.y << 16);
-        nw[a][3] = __uint_as_float((uint32_t)wr.y & 0xffff0000u);
-    }
-
-    // bias, then RMSNorm over the head (sum of squares in-lane, then over
-    // lanes l ^ 16 and l ^ 32) and the norm weight. Norm sections first round
-    // the projection to bf16, as the module's linear outputs it, so the norm
-    // and RoPE see the values the reference's separate steps see
-    // (dense_fa4.py:123-140, transformer.py:146-173); rounding only once, at
-    // the end, moves the LSE of the attention that follows by up to about
-    // 2e-3 against that order.
-    auto normed = [&](int b, float (&v)[8][4], auto norm_c) __attribute__((always_inline)) {
+        for (int a = 0; a < T::NA; ++a) {
+            // (Features past the section, in the second half of a last tile,
+            // read the section's first ones; their rows are not stored.)
+            const int f = tc.f0 + f_wave + 16 * a + 4 * q;
+            const i32x2 br = has_bias ? *(const i32x2*)((const uint16_t*)sec.bias + (f < sec.n ? f : 0)) : i32x2{0, 0};
+            const float b0 = __uint_as_float((uint32_t)br.x << 16), b1 = __uint_as_float((uint32_t)br.x & 0xffff0000u);
+            const float b2 = __uint_as_float((uint32_t)br.y << 16), b3 = __uint_as_float((uint32_t)br.y & 0xffff0000u);
+            const int c = (((f_wave & 127) >> 3) + 2 * a) << 4;
 #pragma unroll
-        for (int a = 0; a < 8; ++a)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[a][e] = acc[a][b][e] + bias[a][e];
-        if constexpr (decltype(norm_c)::value) {
-#pragma unroll
-            for (int a = 0; a < 8; ++a)
-#pragma unroll
-                for (int e = 0; e < 4; e += 2) {
-                    const uint32_t r = pack_bf16x2(v[a][e], v[a][e + 1]);
-                    v[a][e] = __uint_as_float(r << 16);
-                    v[a][e + 1] = __uint_as_float(r & 0xffff0000u);
-                }
-            // Four partial sums (over e), added at the end: short dependency
-            // chains for a lone wave.
-            float s4[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int a = 0; a < 8; ++a)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) s4[e] += v[a][e] * v[a][e];
-            float ss = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-            auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(ss), __float_as_uint(ss), false, false);
-            ss = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
-            const f32x2 h = halves(ss);
-            ss = h[0] + h[1];
-            const float r = rsqrtf(ss * (1.0f / 128.0f) + sec.eps);
-#pragma unroll
-            for (int a = 0; a < 8; ++a)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[a][e] = (v[a][e] * r) * nw[a][e];
+            for (int b = 0; b < T::NB; ++b) {
+                const f32x4 v = acc[a][b];
+                *(lds_i32x2*)(row + b * 16 * T::kOutRow + (swz ^ c)) =
+                    i32x2{(int)pack_bf16x2(v.x + b0, v.y + b1), (int)pack_bf16x2(v.z + b2, v.w + b3)};
+            }
         }
+    }
+    __syncthreads();
+
+    const int g = tid >> 4, j = tid & 15;  // row group, lane of the row
+    const int heads = min(kHeads, (sec.n - tc.f0) >> 7);
+    const int tokens = min(T::kTokens, p.m - tc.m0);
+    char* const yb = (char*)sec.y + (int64_t)tc.m0 * sec.y_rs + (int64_t)tc.f0 * 2 + j * 16;
+    auto load_row = [&](int t, int h, int chunk) {
+        return *(const lds_i32x4*)(out + t * T::kOutRow + h * 256 + ((chunk ^ (t & 15)) << 4));
     };
-    lds_char* const orow = (lds_char*)smem + wave * kPOutWave;
-    // Direct stores (sections without RoPE) go through a resource over this
-    // wave's 128 token rows of its head: rows past the launch's tokens lie
-    // outside its records and are dropped, and a wave whose head is past the
-    // section gets no records at all, so no store needs a branch. f_pair:
-    // byte offset of the lane's 8 features within a 32-feature group.
-    // (Base and size go through readfirstlane: uniform, but the compiler
-    // would otherwise keep the resource in VGPRs and wrap every store in a
-    // waterfall loop.)
-    const int rows_valid = active ? max(0, min(128, p.m - m_head)) : 0;
-    const uint64_t ybase = (uint64_t)(uintptr_t)((const char*)sec.y + (int64_t)m_head * sec.y_rs + (int64_t)f_safe * 2);
-    const uint32_t ybytes = rows_valid > 0 ? (uint32_t)((rows_valid - 1) * sec.y_rs + 256) : 0u;
-    const auto yout = make_rsrc(
-        (const void*)(uintptr_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(ybase >> 32)) << 32) |
-                                 (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)ybase)),
-        (uint32_t)__builtin_amdgcn_readfirstlane((int)ybytes));
-    const uint32_t f_pair = (uint32_t)((((lane >> 4) & 1) ? 16 : 0) + 4 * ((lane >> 4) & 2)) * 2u;
-    // R a multiple of 32: every RoPE partner (c +- R/2, R/2 a multiple of 16)
-    // is held by the same lane, feature block a pairing with a +- R/32, and
-    // both use the table columns of block a mod R/32.
-    auto in_lane = [&](auto rh_c, auto norm_c) __attribute__((always_inline)) {
-        constexpr int rh = decltype(rh_c)::value, ra = 2 * rh;  // half of the rotated blocks, all of them
-        constexpr int nt = rh > 0 ? rh : 1;
-        f32x4 tcv[2][nt], tsv[2][nt];
-        auto load_regs = [&](int b) __attribute__((always_inline)) {
-            const uint32_t o = tab_offset(b);
+    auto store_row = [&](int t, int h, const i32x4& v) {
+        __builtin_nontemporal_store(v, (i32x4*)(yb + (int64_t)t * sec.y_rs + h * 256));
+    };
+    const int R = sec.mode != 0 ? p.rotary_dim : 0;
+    if (sec.mode == 0) {
+#pragma unroll 4
+        for (int t = g; t < tokens; t += 16)
 #pragma unroll
-            for (int ta = 0; ta < rh; ++ta) {
-                tcv[b & 1][ta] = __builtin_bit_cast(f32x4, buf_load16(rcos, o + 64u * ta));
-                tsv[b & 1][ta] = __builtin_bit_cast(f32x4, buf_load16(rsin, o + 64u * ta));
+            for (int h = 0; h < kHeads; ++h)
+                if (h < heads) store_row(t, h, load_row(t, h, j));
+        return;
+    }
+    const int half = R >> 1, col0 = 8 * j;
+    const float eps = sec.eps;
+    float wv[8], wp[8];
+    unpack8(*(const i32x4*)((const uint16_t*)sec.norm_w + col0), wv);
+
+    // Norm and RoPE of the tile's rows: kForm 0: no rotary columns, 1: R a
+    // multiple of 16 and tables with 16-byte rows, 2: any even R.
+    auto rows = [&](auto form_c) __attribute__((always_inline)) {
+        constexpr int kForm = decltype(form_c)::value;
+        const bool rot = kForm == 1 && col0 < R;
+        const bool first = col0 < half;
+        const int pj = rot ? (first ? j + (half >> 3) : j - (half >> 3)) : j;  // partner lane (kForm 1)
+        uint32_t pmask[4];
+        if constexpr (kForm == 1) unpack8(*(const i32x4*)((const uint16_t*)sec.norm_w + 8 * pj), wp);
+        if constexpr (kForm == 2) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int c = min(col0 + e, R - 1);
+                wp[e] = bf16_to_f32(((const uint16_t*)sec.norm_w)[c < half ? c + half : c - half]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pmask[i] = col0 + 2 * i < R ? 0xffffffffu : 0u;
+        }
+        // Tables of a rotate-half pair are equal in both halves: reading the
+        // first alone halves their cache traffic.
+        const int tcol = kForm != 1 ? 0 : !rot ? 0 : (p.rope_full_tables == 0 && !first) ? col0 - half : col0;
+        const bool pairs = (((uintptr_t)p.cos | (uintptr_t)p.sin) & 7) == 0 && (p.table_stride & 1) == 0;  // uniform
+        struct Tabs {
+            f32x4 c[2], s[2];  // cos and sin of the lane's 8 columns
+        };
+        auto load_tables = [&](int t) __attribute__((always_inline)) {
+            Tabs w{};
+            if constexpr (kForm != 0) {
+                int s = tc.m0 + min(t, tokens - 1);
+                s = s < p.seqlen ? s : s % p.seqlen;
+                const float* const cr = p.cos + (int64_t)s * p.table_stride;
+                const float* const sr = p.sin + (int64_t)s * p.table_stride;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    if constexpr (kForm == 1) {
+                        w.c[i] = *(const f32x4*)(cr + tcol + 4 * i);
+                        w.s[i] = *(const f32x4*)(sr + tcol + 4 * i);
+                    } else {
+                        const int c0 = min(col0 + 4 * i, R - 2), c1 = min(col0 + 4 * i + 2, R - 2);
+                        if (pairs) {
+                            const f32x2 a = *(const f32x2*)(cr + c0), b = *(const f32x2*)(cr + c1);
+                            const f32x2 c = *(const f32x2*)(sr + c0), d = *(const f32x2*)(sr + c1);
+                            w.c[i] = f32x4{a.x, a.y, b.x, b.y};
+                            w.s[i] = f32x4{c.x, c.y, d.x, d.y};
+                        } else {
+                            w.c[i] = f32x4{cr[c0], cr[c0 + 1], cr[c1], cr[c1 + 1]};
+                            w.s[i] = f32x4{sr[c0], sr[c0 + 1], sr[c1], sr[c1 + 1]};
+                        }
+                    }
+                }
+            }
+            return w;
+        };
+        // A wave's four groups are four consecutive tokens: the loop bound is
+        // the wave's, so every lane joins the row sums and partner reads.
+        const int t_end = (tokens - 4 * (g >> 2) + 15) / 16;  // iterations of this wave
+        auto token = [&](int t, const Tabs& tab) __attribute__((always_inline)) {
+#pragma unroll
+            for (int h = 0; h < kHeads; ++h) {
+                if (h >= heads) break;
+                const i32x4 x = load_row(t, h, j);
+                float xv[8], o[8];
+                unpack8(x, xv);
+                float ss = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) ss += xv[e] * xv[e];
+                const float r = rsqrtf(group_sum<16>(ss) * (1.0f / 128.0f) + eps);
+                if constexpr (kForm == 0) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) o[e] = (xv[e] * r) * wv[e];
+                } else {
+                    i32x4 px;
+                    if constexpr (kForm == 1) {
+                        px = load_row(t, h, pj);
+                    } else {
+                        px = any_r_partners(out + T::kOutBytes + g * T::kPartner, x, j, R);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) px[i] &= (int)pmask[i];
+                    }
+                    float xp[8];
+                    unpack8(px, xp);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float n = (xv[e] * r) * wv[e];
+                        const float pn = (xp[e] * r) * wp[e];
+                        if constexpr (kForm == 1) {
+                            o[e] = rot ? n * tab.c[e >> 2][e & 3] + (first ? -pn : pn) * tab.s[e >> 2][e & 3] : n;
+                        } else {
+                            const bool in = col0 + e < R;
+                            const float c = in ? tab.c[e >> 2][e & 3] : 1.f, sn = tab.s[e >> 2][e & 3];
+                            const float s = !in ? -0.f : col0 + e < half ? -sn : sn;
+                            o[e] = n * c + pn * s;
+                        }
+                    }
+                }
+                i32x4 w;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[e] = (int)pack_bf16x2(o[2 * e], o[2 * e + 1]);
+                if (t < tokens) store_row(t, h, w);
             }
         };
-        if constexpr (ra > 0) load_regs(0);
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            if constexpr (ra > 0) {
-                if (b + 1 < 8) load_regs(b + 1);
-            }
-            float v[8][4];
-            normed(b, v, norm_c);
-            const int r = 16 * b + j16;
-            if (ra == 0 && !staged) {
-                // No tables to wait for: stores go out directly. Lanes l and
-                // l ^ 16 (feature groups q, q ^ 1) trade one of two feature
-                // blocks 2j, 2j+1 (permlane16_swap exchanges the first
-                // operand of the odd lane with the second of the even one),
-                // so that the even lane holds 8 consecutive features of
-                // block 2j and the odd lane of block 2j+1: one 16-byte store
-                // each, 64 contiguous bytes per token.
-                const uint32_t row_off = (uint32_t)r * (uint32_t)sec.y_rs;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t p0x = pack_bf16x2(v[2 * j][0], v[2 * j][1]), p0y = pack_bf16x2(v[2 * j][2], v[2 * j][3]);
-                    const uint32_t p1x = pack_bf16x2(v[2 * j + 1][0], v[2 * j + 1][1]);
-                    const uint32_t p1y = pack_bf16x2(v[2 * j + 1][2], v[2 * j + 1][3]);
-                    const auto sx = __builtin_amdgcn_permlane16_swap(p0x, p1x, false, false);
-                    const auto sy = __builtin_amdgcn_permlane16_swap(p0y, p1y, false, false);
-                    const i32x4 w{(int)sx[0], (int)sy[0], (int)sx[1], (int)sy[1]};
-                    __builtin_amdgcn_raw_buffer_store_b128(w, yout, (int)(row_off + (uint32_t)(64 * j) + f_pair), 0, 0);
-                }
-                continue;
-            }
-#pragma unroll
-            for (int a = 0; a < 8; ++a) {
-                float y[4];
-                if (a < ra) {
-                    const int pa = a < rh ? a + rh : a - rh;
-                    const int ta = a < rh ? a : a - rh;
-                    const f32x4 cw = tcv[b & 1][ta], sw = tsv[b & 1][ta];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float rot = a < rh ? -v[pa][e] : v[pa][e];
-                        y[e] = v[a][e] * cw[e] + rot * sw[e];
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) y[e] = v[a][e];
-                }
-                const i32x2 w{(int)pack_bf16x2(y[0], y[1]), (int)pack_bf16x2(y[2], y[3])};
-                *(__attribute__((address_space(3))) i32x2*)(orow + r * 256 + ((((4 * a + (lane >> 4)) ^ r) & 31) << 3)) = w;
-            }
+        Tabs t0 = load_tables(g);
+        int it = 0, t = g;
+        for (; it + 2 <= t_end; it += 2, t += 32) {
+            const Tabs t1 = load_tables(t + 16);
+            token(t, t0);
+            t0 = load_tables(t + 32);
+            token(t + 16, t1);
         }
+        if (it < t_end) token(t, t0);
     };
-    // Any other even R, or tables read at every rotated column: the partner
-    // c +- R/2 of feature c is in general held by another lane of the token,
-    // at another position. The norm starts from the bf16-rounded projection,
-    // so the token's projection row is exact in bf16: it goes into the
-    // wave's LDS row of the token (feature f at byte 2f, past the stage
-    // memory), each lane reads its partners' values back, normalises them
-    // with the token's r (the same in the 4 lanes of a token) and the
-    // partner's norm weight, and reads cos / sin at its own columns. A
-    // wave's LDS operations run in order: every lane's row writes precede
-    // the reads, and a block's reads precede the next block's writes (the
-    // memory clobbers keep the compiler from moving one past the other).
-    lds_char* const prows = (lds_char*)smem + kPLds + wave * kPRowsWave;
-    auto cross_lane = [&]() __attribute__((always_inline)) {
-        const int rh = R >> 1;
-        float wpart[8][4];  // norm weight at the partner column
-#pragma unroll
-        for (int a = 0; a < 8; ++a)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int c = 16 * a + fl + e;
-                const int pc = c < rh ? c + rh : c - rh;
-                wpart[a][e] = c < R ? bf16_to_f32(((const uint16_t*)sec.norm_w)[pc]) : 0.f;
-            }
-        // (Unrolled: the accumulators are registers, indexed by constants.)
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            float v[8][4];
-#pragma unroll
-            for (int a = 0; a < 8; ++a)
-#pragma unroll
-                for (int e = 0; e < 4; e += 2) {
-                    const uint32_t h2 = pack_bf16x2(acc[a][b][e] + bias[a][e], acc[a][b][e + 1] + bias[a][e + 1]);
-                    v[a][e] = __uint_as_float(h2 << 16);
-                    v[a][e + 1] = __uint_as_float(h2 & 0xffff0000u);
-                }
-            const int r = 16 * b + j16;
-            lds_char* const prow = prows + j16 * 256;
-            asm volatile("" ::: "memory");
-#pragma unroll
-            for (int a = 0; a < 8; ++a)
-                *(__attribute__((address_space(3))) i32x2*)(prow + (16 * a + fl) * 2) =
-                    i32x2{(int)pack_bf16x2(v[a][0], v[a][1]), (int)pack_bf16x2(v[a][2], v[a][3])};
-            asm volatile("" ::: "memory");
-            float s4[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int a = 0; a < 8; ++a)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) s4[e] += v[a][e] * v[a][e];
-            float ss = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-            auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(ss), __float_as_uint(ss), false, false);
-            ss = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
-            const f32x2 hs = halves(ss);
-            ss = hs[0] + hs[1];
-            const float rn = rsqrtf(ss * (1.0f / 128.0f) + sec.eps);
-            int tok = m_head + r;
-            tok = tok < seqlen ? tok : tok % seqlen;
-            const uint32_t trow = (uint32_t)tok * row_bytes;
-#pragma unroll
-            for (int a = 0; a < 8; ++a) {
-                float y[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int c = 16 * a + fl + e;
-                    const float n = (v[a][e] * rn) * nw[a][e];
-                    y[e] = n;
-                    if (c < R) {
-                        const int pc = c < rh ? c + rh : c - rh;
-                        const float pp = bf16_to_f32(*(const __attribute__((address_space(3))) uint16_t*)(prow + pc * 2));
-                        const float pn = (pp * rn) * wpart[a][e];
-                        const uint32_t to = trow + (uint32_t)c * 4u;
-                        const float cv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rcos, (int)to, 0, 0));
-                        const float sv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsin, (int)to, 0, 0));
-                        y[e] = n * cv + (c < rh ? -pn : pn) * sv;
-                    }
-                }
-                const i32x2 w{(int)pack_bf16x2(y[0], y[1]), (int)pack_bf16x2(y[2], y[3])};
-                *(__attribute__((address_space(3))) i32x2*)(orow + r * 256 + ((((4 * a + (lane >> 4)) ^ r) & 31) << 3)) = w;
-            }
-        }
-    };
-    using Y = std::true_type;
-    if (!norm) {
-        in_lane(std::integral_constant<int, 0>{}, std::false_type{});
-    } else if (R > 0 && p.rope_full_tables != 0) {
-        cross_lane();
-    } else {
-        switch (R) {
-            case 0: in_lane(std::integral_constant<int, 0>{}, Y{}); break;
-            case 32: in_lane(std::integral_constant<int, 1>{}, Y{}); break;
-            case 64: in_lane(std::integral_constant<int, 2>{}, Y{}); break;
-            case 96: in_lane(std::integral_constant<int, 3>{}, Y{}); break;
-            default: in_lane(std::integral_constant<int, 4>{}, Y{}); break;  // 128 (other widths: cross_lane)
-        }
-    }
-    if (!active || !staged) return;  // the rows went out directly
-    // Lane l moves bytes 16*(l & 15) .. +16 of token row 4*it + (l >> 4) (the
-    // wave's LDS ops are ordered, so its own writes are visible here).
-    char* const yb = (char*)sec.y + (int64_t)f_head * 2 + j16 * 16;
-#pragma unroll 8
-    for (int it = 0; it < 32; ++it) {
-        const int r = 4 * it + (lane >> 4);
-        const lds_char* const src = (const lds_char*)orow + r * 256;
-        const i32x2 lo = *(const __attribute__((address_space(3))) i32x2*)(src + ((((2 * j16) ^ r) & 31) << 3));
-        const i32x2 hi = *(const __attribute__((address_space(3))) i32x2*)(src + ((((2 * j16 + 1) ^ r) & 31) << 3));
-        const int m = m_head + r;
-        // Non-temporal: whole 256-byte row pieces that no later tile reads
-        // (q and k of the 40-head block 3.5% faster; the direct stores'
-        // 64-byte pieces measured slower this way and stay ordinary).
-        if (m < p.m) __builtin_nontemporal_store(i32x4{lo.x, lo.y, hi.x, hi.y}, (i32x4*)(yb + (int64_t)m * sec.y_rs));
-    }
+    const bool tab16 = (((uintptr_t)p.cos | (uintptr_t)p.sin) & 15) == 0 && (p.table_stride & 3) == 0;
+    if (R == 0)
+        rows(std::integral_constant<int, 0>{});
+    else if ((R & 15) == 0 && tab16)
+        rows(std::integral_constant<int, 1>{});
+    else
+        rows(std::integral_constant<int, 2>{});
 }
 
+template <int TF, int NT, int SW, int SX>
 __global__ __launch_bounds__(kPThreads, 1) void proj_gemm_kernel(ProjGemmParams p) {
-    __shared__ __attribute__((aligned(1024))) char smem[kPSmem];
-    const lds_char* const lds = (const lds_char*)smem;
+    using T = Tile<TF, NT, SW, SX>;
+    __shared__ __attribute__((aligned(1024))) char smem[T::kLds];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wn = wave >> 1, wm = wave & 1;
+    const int wn = wave / T::WM, wm = wave % T::WM;
 
     // One workgroup per tile. Workgroup b runs on XCD b mod 8 (round-robin
     // dispatch) as that XCD's (b / 8)-th; each XCD owns one contiguous range
     // of the grouped tile order, so the ~32 tiles an XCD runs at a time are
-    // consecutive in it (about 2 token tiles x 16 feature tiles sharing their
-    // X and W panels in the XCD's L2). (A persistent grid of one workgroup
-    // per CU looping over its XCD's range measured from 1% faster to 4%
-    // slower, and is not used.)
+    // consecutive in it and share their X and W panels in the XCD's L2. (A
+    // persistent grid of one workgroup per CU looping over its XCD's range
+    // measured from 1% faster to 4% slower, and is not used.)
     const int total = p.m_tiles * p.n_tiles;
     const int bid = blockIdx.x;
     const int xcd = bid & 7, local = bid >> 3;
     const int per = total >> 3, rem = total & 7;
-    const int first = xcd * per + min(xcd, rem), end = first + per + (xcd < rem ? 1 : 0);
-    const int tile = first + local;
-    if (tile >= end) return;  // the grid is the tile count: never taken
+    const int tile = xcd * per + min(xcd, rem) + local;
+    const TileCoord tc = tile_coord(p, tile, TF, T::kTokens);
 
-    // DMA map: load i of a wave fills rows (8*wave + i)*8 .. +8 of an operand
-    // tile; lane L writes LDS chunk (L & 7) of row r0 + (L >> 3), which holds
-    // the row's 16-byte chunk (L & 7) ^ swz(row), swz(r) = (r >> 1) & 7 =
-    // 4*(i & 1) + (L >> 4) for these rows. The per-lane part of the source
-    // offset depends on the parity of i; the load's first row and the K step
-    // go into the scalar offset.
-    int chunk[2];
-#pragma unroll
-    for (int par = 0; par < 2; ++par) chunk[par] = ((lane & 7) ^ ((4 * par + (lane >> 4)) & 7)) << 4;
-    uint32_t dx[2];
-#pragma unroll
-    for (int par = 0; par < 2; ++par) dx[par] = (uint32_t)((lane >> 3) * p.x_rs + chunk[par]);
-    auto source = [&](const TileCoord& tc) __attribute__((always_inline)) {
-        const ProjSection sec = section(p, tc.sec);
-        const int n_rows = min(kPT, sec.n - tc.f0), m_rows = min(kPT, p.m - tc.m0);
-        const char* const wb = (const char*)sec.w + (int64_t)tc.f0 * sec.w_rs;
-        const char* const xb = (const char*)p.x + (int64_t)tc.m0 * p.x_rs;
-        TileSrc s;
-        s.rw = make_rsrc_words(wb, (uint32_t)((int64_t)(n_rows - 1) * sec.w_rs + p.k * 2));
-        s.rx = make_rsrc_words(xb, (uint32_t)((int64_t)(m_rows - 1) * p.x_rs + p.k * 2));
-        s.w_rs = (int32_t)sec.w_rs;
-#pragma unroll
-        for (int par = 0; par < 2; ++par) s.dw[par] = (uint32_t)((lane >> 3) * sec.w_rs + chunk[par]);
-        return s;
-    };
-    const int nk = p.k / kPK;
-    // Load j (0..15) of this wave's share of K step kt of a tile into
-    // `stage`: j < 8 are W rows, j >= 8 X rows. buffer_load ... lds writes 16
+    // Operand resources, based at the tile's first row: rows past the section
+    // or the token range are outside their records and load as zeros.
+    const ProjSection sec = section(p, tc.sec);
+    const int32_t w_rs = (int32_t)sec.w_rs, x_rs = (int32_t)p.x_rs;
+    i32x4 rw = make_rsrc_words((const char*)sec.w + (int64_t)tc.f0 * sec.w_rs,
+                                     (uint32_t)((int64_t)(min(TF, sec.n - tc.f0) - 1) * sec.w_rs + p.k * 2));
+    i32x4 rx = make_rsrc_words((const char*)p.x + (int64_t)tc.m0 * p.x_rs,
+                                     (uint32_t)((int64_t)(min(T::kTokens, p.m - tc.m0) - 1) * p.x_rs + p.k * 2));
+    // DMA map: load i of wave w fills rows 8 (4i + w) .. +8 of an operand's
+    // stage; lane L writes LDS chunk (L & 7) of row r = 8 (4i + w) + (L >> 3),
+    // which holds the row's 16-byte chunk (L & 7) ^ ((r >> 1) & 7) =
+    // (L & 7) ^ (4 (w & 1) + (L >> 4)). Everything that depends on the lane is
+    // the same for every load; i and the K step go into the scalar offset.
+    const int chunk = ((lane & 7) ^ (4 * (wave & 1) + (lane >> 4))) << 4;
+    const int row0 = 8 * wave + (lane >> 3);
+    const uint32_t dw = (uint32_t)(row0 * w_rs + chunk), dx = (uint32_t)(row0 * x_rs + chunk);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(const lds_char*)smem;
+    const uint32_t lds_wave = lds0 + (uint32_t)wave * 1024u;
+    // Load j of this wave's share of a K step's rows (32 j rows on from the
+    // wave's first), into LDS at dst + 4096 j. buffer_load ... lds writes 16
     // bytes per lane to LDS address M0 + 16*lane; M0 needs one wait state
-    // before the load reads it (the two scalar offset instructions give it).
-    // The scalar offsets are formed in the asm itself, per load: hoisted out
-    // of the loop they would hold 32 scalar registers.
-    const uint32_t lds_wave = (uint32_t)(uintptr_t)(lds + wave * kPDmaPerOp * 8 * kPRow);
-    auto dma1 = [&](i32x4 rw, i32x4 rx, uint32_t dw0, uint32_t dw1, int w_rs, int kt, int stage, int j)
-                    __attribute__((always_inline)) {
-        const int i = j & 7;
-        const bool is_w = j < 8;
-        const uint32_t row8 = (uint32_t)(8 * (is_w ? w_rs : (int)p.x_rs));  // bytes of 8 rows
-        const uint32_t base = (uint32_t)(wave * kPDmaPerOp) * row8 + (uint32_t)(kt * kPRow);
-        const uint32_t voff = is_w ? ((i & 1) ? dw1 : dw0) : dx[i & 1];
-        uint32_t soff;
-        if (is_w)
-            asm volatile(
-                "s_add_u32 m0, %1, %2\n\ts_mul_i32 %0, %3, %4\n\ts_add_u32 %0, %0, %5\n\t"
-                "buffer_load_dwordx4 %6, %7, %0 offen lds"
-                : "=&s"(soff)
-                : "s"(lds_wave), "i"(stage * kPTile + i * 8 * kPRow), "s"(row8), "i"(i), "s"(base), "v"(voff), "s"(rw)
-                : "memory");
-        else
-            asm volatile(
-                "s_add_u32 m0, %1, %2\n\ts_mul_i32 %0, %3, %4\n\ts_add_u32 %0, %0, %5\n\t"
-                "buffer_load_dwordx4 %6, %7, %0 offen lds"
-                : "=&s"(soff)
-                : "s"(lds_wave), "i"(kPXBase + stage * kPTile + i * 8 * kPRow), "s"(row8), "i"(i), "s"(base),
-                  "v"(voff), "s"(rx)
-                : "memory");
+    // before the load reads it. The row offsets stay in scalar registers and
+    // the resources' bases move along K: three instructions a load, which fit
+    // between two MFMAs (offsets formed per load took six, and held up the
+    // lone wave's MFMAs).
+    auto dma1 = [&](const i32x4& rsrc, uint32_t voff, uint32_t soff, uint32_t dst, int j) __attribute__((always_inline)) {
+        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
+                     :
+                     : "s"(dst), "i"(j * 4096), "v"(voff), "s"(rsrc), "s"(soff)
+                     : "memory", "scc");
     };
-    auto dma_src = [&](const TileSrc& s, int kt, int stage, int j) __attribute__((always_inline)) {
-        dma1(s.rw, s.rx, s.dw[0], s.dw[1], s.w_rs, kt, stage, j);
+    uint32_t sow[T::kLoadsW], sox[T::kLoadsX];
+#pragma unroll
+    for (int j = 0; j < T::kLoadsW; ++j) sow[j] = (uint32_t)(32 * j * w_rs);
+#pragma unroll
+    for (int j = 0; j < T::kLoadsX; ++j) sox[j] = (uint32_t)(32 * j * x_rs);
+    auto dma_w1 = [&](const i32x4& r, uint32_t stage, int j) __attribute__((always_inline)) {
+        dma1(r, dw, sow[j], lds_wave + stage, j);
+    };
+    auto dma_x1 = [&](const i32x4& r, uint32_t stage, int j) __attribute__((always_inline)) {
+        dma1(r, dx, sox[j], lds_wave + T::kXBase + stage, j);
+    };
+    // The resource one K step further along its rows. The records stay: a
+    // lane's offset in its row is under 128 bytes and a row is at least the
+    // reduction long, so the row after the last one is out of range at every
+    // base.
+    auto advance = [](i32x4& r) __attribute__((always_inline)) {
+        const uint64_t base = ((uint64_t)(uint32_t)r.y << 32 | (uint32_t)r.x) + kPRow;
+        r.x = (int)(uint32_t)base;
+        r.y = (int)((uint32_t)(base >> 32) & 0xffffu);
     };
 
     // Fragment reads: lane l takes row (16*block + (l & 15)) of the wave's
@@ -533,112 +426,197 @@ __global__ __launch_bounds__(kPThreads, 1) void proj_gemm_kernel(ProjGemmParams 
     const int sl = (lane >> 1) & 7;
     const int fo0 = (lane & 15) * kPRow + (((lane >> 4) ^ sl) << 4);
     const int fo1 = (lane & 15) * kPRow + (((4 + (lane >> 4)) ^ sl) << 4);
-    const lds_char* const wfr0 = lds + wn * 128 * kPRow + fo0;
-    const lds_char* const wfr1 = lds + wn * 128 * kPRow + fo1;
-    const lds_char* const xfr0 = lds + kPXBase + wm * 128 * kPRow + fo0;
-    const lds_char* const xfr1 = lds + kPXBase + wm * 128 * kPRow + fo1;
+    const lds_char* const lds = (const lds_char*)smem;
+    const lds_char* const wfr0 = lds + wn * 16 * T::NA * kPRow + fo0;
+    const lds_char* const wfr1 = lds + wn * 16 * T::NA * kPRow + fo1;
+    const lds_char* const xfr0 = lds + T::kXBase + wm * 16 * T::NB * kPRow + fo0;
+    const lds_char* const xfr1 = lds + T::kXBase + wm * 16 * T::NB * kPRow + fo1;
 
-    f32x4 acc[8][8];
-    bf16x8 fw[2][8], fx[2][8];
+    f32x4 acc[T::NA][T::NB];
+    bf16x8 fw[2][T::NA], fx[2][T::NB];
+    constexpr int kReads = T::NA + T::NB, kMfmas = T::NA * T::NB;
 
-    // Fragments of MFMA K step h of the stage in LDS buffer `st` into set h.
-    auto read1 = [&](int st, int h, int j) __attribute__((always_inline)) {
-        const lds_char* const xf = h ? xfr1 : xfr0;
-        const lds_char* const wf = h ? wfr1 : wfr0;
-        if (j < 8)
-            fx[h][j] = *(const lds_bf16x8*)(xf + st * kPTile + j * 16 * kPRow);
+    // Fragment j of MFMA K step h of the stages at byte offsets sw, sx.
+    auto read1 = [&](uint32_t sw, uint32_t sx, int h, int j) __attribute__((always_inline)) {
+        const lds_char* const xf = (h ? xfr1 : xfr0) + sx;
+        const lds_char* const wf = (h ? wfr1 : wfr0) + sw;
+        if (j < T::NB)
+            fx[h][j] = *(const lds_bf16x8*)(xf + j * 16 * kPRow);
         else
-            fw[h][j - 8] = *(const lds_bf16x8*)(wf + st * kPTile + (j - 8) * 16 * kPRow);
+            fw[h][j - T::NB] = *(const lds_bf16x8*)(wf + (j - T::NB) * 16 * kPRow);
     };
-    // 64 MFMAs of fragment set h, feature block major, token blocks snaking,
-    // with `extra(t)` issued after MFMA t; `first`: the tile's first K step.
-    auto mfma64 = [&](int h, bool first, auto&& extra) __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < 64; ++t) {
-            const int a = t >> 3, b = (a & 1) ? 7 - (t & 7) : (t & 7);
-            if (first)
-                mfma_first(acc[a][b], fw[h][a], fx[h][b]);
-            else
-                mfma_acc(acc[a][b], fw[h][a], fx[h][b]);
-            extra(t);
+    // The MFMAs of fragment set h, feature block major, token blocks snaking,
+    // with `extra(t)` issued after MFMA t.
+    auto mfmas = [&](int h, auto&& extra) __attribute__((always_inline)) {
+        static_for<kMfmas>([&](auto tc_) __attribute__((always_inline)) {
+            constexpr int t = decltype(tc_)::value, a = t / T::NB, r = t % T::NB, b = (a & 1) ? T::NB - 1 - r : r;
+            mfma_acc(acc[a][b], fw[h][a], fx[h][b]);
+            extra(tc_);
             __builtin_amdgcn_sched_barrier(0);
-        }
+        });
     };
+    // n items spread over the first `over` MFMAs: those that follow MFMA t.
+    auto spread = [](auto tc_, auto n_c, auto over_c, auto&& item) __attribute__((always_inline)) {
+        constexpr int t = decltype(tc_)::value, n = decltype(n_c)::value, over = decltype(over_c)::value;
+        constexpr int lo = t < over ? t * n / over : n, hi = t < over ? (t + 1) * n / over : n;
+        static_for<hi - lo>([&](auto i) __attribute__((always_inline)) { item(lo + decltype(i)::value); });
+    };
+    using Reads = std::integral_constant<int, kReads>;
+    using LoadsW = std::integral_constant<int, T::kLoadsW>;
+    using LoadsX = std::integral_constant<int, T::kLoadsX>;
+    using Most = std::integral_constant<int, kMfmas * 3 / 4>;
+    using All = std::integral_constant<int, kMfmas>;
 
-    {
-        const TileCoord tc = tile_coord(p, tile);
-        const TileSrc cur = source(tc);
-        // The tile's first two K steps.
+    const int nk = p.k / kPK;
+    // K step i of W is loaded in the first half of step i + 1 - SW, of X in the
+    // second half of step i - SX. Those before step 0 come here, in that order
+    // (steps past the end of a short reduction through an empty resource: they
+    // load zeros, so that the waits count the same).
+    const i32x4 none{0, 0, 0, kBufferWord3};
 #pragma unroll
-        for (int j = 0; j < 16; ++j) dma_src(cur, 0, 0, j);
+    for (int i = 0; i < SW - 1; ++i) {
+        const int ix = i + 1 - SW + SX;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) dma_src(cur, 1, 1, j);
-        wait_vm_lgkm<16>();  // K step 0 (own loads) landed
-        barrier();
+        for (int j = 0; j < T::kLoadsW; ++j) dma_w1(i < nk ? rw : none, (uint32_t)(i * T::kWBytes), j);
+        advance(rw);
+        if (ix < 0) continue;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) read1(0, 0, j);
-
-        // K step kt in LDS buffer st = kt mod 2, its first-half fragments in
-        // set 0. First half: MFMAs of set 0 while set 1 is read from the same
-        // stage. Then the wave's DMA of K step kt+1 (issued during the
-        // previous step) is waited for, with its reads of stage st; after the
-        // barrier every wave's part of K step kt+1 is in LDS and buffer st is
-        // no longer read by anyone. Second half: MFMAs of set 1 while K step
-        // kt+1's first-half fragments are read into set 0 and K step kt2 =
-        // kt+2 is loaded into buffer st. The tile's last two steps load
-        // nothing, and the last reads nothing.
-        auto step = [&](auto st_c, auto dma_c, auto last_c, bool first, int kt2) __attribute__((always_inline)) {
-            constexpr int st = decltype(st_c)::value;
-            constexpr int nst = st ^ 1;
-            constexpr bool dma = decltype(dma_c)::value, last = decltype(last_c)::value;
-            mfma64(0, first, [&](int t) __attribute__((always_inline)) {
-                if ((t & 1) == 1 && t < 32) read1(st, 1, t >> 1);
-            });
-            wait_vm_lgkm<0>();
-            barrier();
-            mfma64(1, false, [&](int t) __attribute__((always_inline)) {
-                if (!last && (t & 3) == 1) read1(nst, 0, t >> 2);
-                if (dma && (t & 3) == 0) dma_src(cur, kt2, st, t >> 2);
-            });
-        };
-        using I0 = std::integral_constant<int, 0>;
-        using I1 = std::integral_constant<int, 1>;
-        using T = std::true_type;
-        using F = std::false_type;
-        // K is a multiple of two steps (checked by the caller), so the buffer
-        // of every step is a compile-time constant.
-        if (nk == 2) {
-            step(I0{}, F{}, F{}, true, 0);
-            step(I1{}, F{}, T{}, false, 0);
-        } else {
-            step(I0{}, T{}, F{}, true, 2);
-            step(I1{}, T{}, F{}, false, 3);
-            for (int kt = 2; kt < nk - 2; kt += 2) {
-                step(I0{}, T{}, F{}, false, kt + 2);
-                step(I1{}, T{}, F{}, false, kt + 3);
-            }
-            step(I0{}, F{}, F{}, false, 0);
-            step(I1{}, F{}, T{}, false, 0);
-        }
-        // No load is in flight and no wave reads the stages any more (the
-        // last step's barrier followed every wave's last fragment read). The
-        // MFMAs are inline asm, outside the compiler's hazard tracking: give
-        // the last ones time to write their results before they are read.
-        asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
-        epilogue(p, tc, acc, wave, wn, wm, lane, smem);
+        for (int j = 0; j < T::kLoadsX; ++j) dma_x1(ix < nk ? rx : none, (uint32_t)(ix * T::kXBytes), j);
+        advance(rx);
     }
+#pragma unroll
+    for (int a = 0; a < T::NA; ++a)
+#pragma unroll
+        for (int b = 0; b < T::NB; ++b) {
+            acc[a][b] = f32x4{};
+            asm volatile("" : "+a"(acc[a][b]));
+        }
+    wait_vm_lgkm<(SX - 1) * (T::kLoadsW + T::kLoadsX)>();  // K step 0 (own loads) landed
+    barrier();
+#pragma unroll
+    for (int j = 0; j < kReads; ++j) read1(0, 0, 0, j);
+
+    // K step kt in the stages at `cw` and `cx`, its first-half fragments in set
+    // 0. First half: MFMAs of set 0 while set 1 is read from the same stages,
+    // and the W rows of step kt+SW-1 go into the W stage before `cw`. Then the
+    // wave's own loads of step kt+1 are waited for (later ones stay in flight),
+    // with its reads of the stages; after the barrier every wave's part of
+    // step kt+1 is in LDS and step kt's stages are no longer read by anyone.
+    // Second half: MFMAs of set 1 while step kt+1's first-half fragments are
+    // read into set 0 and the X rows of step kt+SX go into `cx`. The loads of a
+    // step are thus spread over it (the CU's address path takes 64 bytes a
+    // clock, and a lone wave that finds it busy holds up its MFMAs), and W, the
+    // operand that comes from HBM, has SW - 1 steps to land.
+    // `left` K steps follow; the last steps run out of loads, the last one
+    // reads nothing.
+    uint32_t cw = 0, pw = (SW - 1) * T::kWBytes, cx = 0;
+    int kt = 0;
+    auto step = [&](auto left_c) __attribute__((always_inline)) {
+        constexpr int left = decltype(left_c)::value;  // SW: that many or more
+        constexpr int kAheadW = left - (SW - SX) < SX - 1 ? left - (SW - SX) : SX - 1;
+        constexpr int kAheadX = left - 1 < SX - 2 ? left - 1 : SX - 2;
+        const uint32_t nw = cw == (SW - 1) * T::kWBytes ? 0u : cw + T::kWBytes;
+        const uint32_t nx = cx == (SX - 1) * T::kXBytes ? 0u : cx + T::kXBytes;
+        mfmas(0, [&](auto t) __attribute__((always_inline)) {
+            spread(t, Reads{}, Most{}, [&](int i) __attribute__((always_inline)) { read1(cw, cx, 1, i); });
+            if constexpr (left >= SW - 1)
+                spread(t, LoadsW{}, All{}, [&](int i) __attribute__((always_inline)) { dma_w1(rw, pw, i); });
+        });
+        wait_vm_lgkm<(kAheadW > 0 ? kAheadW : 0) * T::kLoadsW + (kAheadX > 0 ? kAheadX : 0) * T::kLoadsX>();
+        barrier();
+        mfmas(1, [&](auto t) __attribute__((always_inline)) {
+            if constexpr (left > 0)
+                spread(t, Reads{}, All{}, [&](int i) __attribute__((always_inline)) { read1(nw, nx, 0, i); });
+            if constexpr (left >= SX)
+                spread(t, LoadsX{}, Most{}, [&](int i) __attribute__((always_inline)) { dma_x1(rx, cx, i); });
+        });
+        advance(rw);
+        advance(rx);
+        pw = cw;
+        cw = nw;
+        cx = nx;
+        ++kt;
+    };
+    while (kt < nk - SW) step(std::integral_constant<int, SW>{});
+    // The last min(SW, nk) steps.
+    auto tail = [&](auto self, auto left_c) __attribute__((always_inline)) -> void {
+        constexpr int left = decltype(left_c)::value;
+        if (left < nk) step(left_c);
+        if constexpr (left > 0) self(self, std::integral_constant<int, left - 1>{});
+    };
+    tail(tail, std::integral_constant<int, SW - 1>{});
+    // No load is in flight and no wave reads the stages any more (the last
+    // step's barrier followed every wave's last fragment read). The MFMAs are
+    // inline asm, outside the compiler's hazard tracking: give the last ones
+    // time to write their results before they are read.
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+    epilogue<T>(p, tc, acc, wn, wm, tid, smem);
+}
+
+template <int TF, int NT, int SW, int SX>
+hipError_t launch_tile(ProjGemmParams& p, hipStream_t stream) {
+    using T = Tile<TF, NT, SW, SX>;
+    p.m_tiles = (p.m + T::kTokens - 1) / T::kTokens;
+    p.n_tiles = 0;
+    for (int i = 0; i < p.n_sections; ++i) p.n_tiles += p.sec[i].tiles = (p.sec[i].n + TF - 1) / TF;
+    // Token tiles of a group: all of a short launch (every W row is then read
+    // from HBM once), else about 1,024 tokens. 1,296 x 5,120 x 5,120 at 128
+    // tokens a tile: 69.9 us with groups of 2, 63.6 with 8, 61.5 with all 11;
+    // 6,240 x 15,360 x 5,120 at 256: 742 (1), 698 (2), 697 (4), 703 (8), 739 (16).
+    p.group_m = p.m_tiles <= 12 ? p.m_tiles : 1024 / T::kTokens;
+    hipLaunchKernelGGL((proj_gemm_kernel<TF, NT, SW, SX>), dim3((unsigned)(p.m_tiles * p.n_tiles)), dim3(kPThreads), 0, stream, p);
+    return hipGetLastError();
+}
+
+// The tile shapes, with the time of one K step of 64 when most CUs run one
+// (measured: 6,240 x 15,360 x 5,120 q/k/v launches, time per round of tiles
+// over 80 steps). Small tiles read more operand bytes per MFMA, so a step costs
+// more than its share; they win where larger ones leave CUs idle: a launch of
+// few tiles, or a last round that is nearly empty. Below about 128 tokens the
+// step time is that of the W rows alone (a CU gets about 60 GB/s from HBM), so
+// 128-feature tiles on twice as many CUs win.
+struct Shape {
+    int tf, nt;
+    float step_us;
+    hipError_t (*launch)(ProjGemmParams&, hipStream_t);
+};
+constexpr Shape kShapes[] = {
+    {256, 16, 1.33f, launch_tile<256, 16, 3, 2>}, {256, 14, 1.21f, launch_tile<256, 14, 3, 2>},
+    {256, 12, 1.07f, launch_tile<256, 12, 3, 2>}, {256, 10, 0.95f, launch_tile<256, 10, 3, 2>},
+    {256, 8, 0.78f, launch_tile<256, 8, 4, 2>},   {256, 6, 0.70f, launch_tile<256, 6, 4, 2>},
+    {128, 8, 0.49f, launch_tile<128, 8, 6, 4>},   {128, 4, 0.33f, launch_tile<128, 4, 7, 5>},
+    {128, 2, 0.27f, launch_tile<128, 2, 8, 6>},
+};
+
+// The shape with the least expected time: rounds of tiles over the CUs, times
+// a tile's K steps and its start and epilogue. Past three rounds the tiles no
+// longer run in step, and the last round costs about half of one.
+const Shape& pick_shape(const ProjGemmParams& p, int cus) {
+    const Shape* best = &kShapes[0];
+    float best_us = 0.f;
+    for (const Shape& s : kShapes) {
+        int64_t tiles = 0;
+        for (int i = 0; i < p.n_sections; ++i) tiles += (p.sec[i].n + s.tf - 1) / s.tf;
+        tiles *= (p.m + 16 * s.nt - 1) / (16 * s.nt);
+        if (tiles >= ((int64_t)1 << 31)) continue;
+        const float r = (float)tiles / (float)cus;
+        const float rounds = r > 3.f ? r + 0.5f : ceilf(r);
+        const float us = rounds * ((float)(p.k / kPK) * s.step_us + 3.f + (float)(s.nt * s.tf) / 1024.f);
+        if (s.nt == 16 || us < best_us) {
+            best = &s;
+            best_us = us;
+        }
+    }
+    return *best;
 }
 
 }  // namespace
 
-hipError_t launch_proj_gemm(const ProjGemmParams& p, hipStream_t stream) {
-    const int64_t tiles = (int64_t)p.m_tiles * p.n_tiles;
-    if (tiles <= 0) return hipSuccess;
-    hipLaunchKernelGGL(proj_gemm_kernel, dim3((unsigned)tiles), dim3(kPThreads), 0, stream, p);
-    return hipGetLastError();
+hipError_t launch_proj_gemm(ProjGemmParams p, int cus, hipStream_t stream) {
+    return pick_shape(p, cus > 0 ? cus : 256).launch(p, stream);
 }
 
-int proj_gemm_tile() { return kPT; }
-int proj_gemm_k_multiple() { return kPK * kPStages; }
+int proj_gemm_tile() { return 256; }
+int proj_gemm_k_multiple() { return 2 * kPK; }
 
 }  // namespace h3a

@@ -65,26 +65,17 @@ __device__ __forceinline__ int64_t head_ofs(const QkNormRopeParams& p, int h, in
     return (int64_t)g * sg + (int64_t)((uint32_t)h - g * p.div_hpg.d) * sh;
 }
 
-// LDS bytes of a lane group's row in the any-R form: the row, then the start
-// of its rotary part again (at most 1.5 * 16 L bytes), then the overrun of the
-// partner reads; rows stay 16-byte aligned.
-constexpr int any_r_row_bytes(int lanes) { return (24 * lanes + 32 + 15) / 16 * 16; }
-
 // kAnyR false: R % 16 == 0 and 16-byte aligned tables, so a lane's 8 columns
 // are either all rotary or all pass-through, its partner columns are the 8
 // columns of lane (j +- R/16), and cos/sin come in two 16-byte loads.
 // kAnyR true (any other even R, or tables at any 4-byte alignment): a lane's
-// partner columns lie across two other lanes, at any even offset. Partner of
-// c is (c + R/2) mod R, so each row goes through LDS once with the first R/2
-// columns written again from column R on: a lane's eight partners are then
-// the 16 bytes at byte 16j + R, read as five aligned dwords and shifted into
-// place by v_alignbit when R/2 is odd. A group's LDS accesses are one wave's,
-// which run in order, so rows need no barrier. Columns past R take cos 1,
-// sin -0 and a zero partner, which leaves n as it is, -0 included. The tables
-// and the partner's weights are per-lane registers shared by the block's
-// heads. Against one row per lane group with element-wise partner and table
-// loads (six dependent 2- and 4-byte loads per output), the pack of 6,240 rows
-// x 40 heads at R = 126 went from 385 to 78 us (389 MB).
+// partner columns lie across two other lanes, at any even offset, and come
+// through LDS (any_r_partners). Columns past R take cos 1, sin -0 and a zero
+// partner, which leaves n as it is, -0 included. The tables and the partners'
+// weights are per-lane registers shared by the block's heads. Against one row
+// per lane group with element-wise partner and table loads (six dependent 2-
+// and 4-byte loads per output), the pack of 6,240 rows x 40 heads at R = 126
+// went from 385 to 78 us (389 MB).
 // One lane group per (token, chunk of kChunk heads): it reads the token's
 // cos/sin once and walks its heads tensor by tensor, each tensor's loads
 // issued first (with a copied third tensor, all loads of the block first);
@@ -181,27 +172,10 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
         // that is lane j ^ 8 of the 16, a DPP rotation of the row.
         i32x4 praw;
         if constexpr (kAnyR) {
-            typedef __attribute__((address_space(3))) char lds_char;
-            typedef __attribute__((address_space(3))) i32x4 lds_i32x4;
-            typedef __attribute__((address_space(3))) uint32_t lds_u32;
-            constexpr int kRowB = any_r_row_bytes(L);
-            __shared__ __attribute__((aligned(16))) char rows[kGroups * kRowB];
-            lds_char* const buf = (lds_char*)rows + tid / L * kRowB;
-            asm volatile("" ::: "memory");
-            *(lds_i32x4*)(buf + 16 * j) = x;
-            asm volatile("" ::: "memory");  // the second copy lands after the first, and over it
-            if (col0 < half) {
+            __shared__ __attribute__((aligned(16))) char rows[kGroups * any_r_row_bytes(L)];
+            praw = any_r_partners((lds_bytes*)rows + tid / L * any_r_row_bytes(L), x, j, R);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) *(lds_u32*)(buf + 2 * R + 16 * j + 4 * i) = (uint32_t)x[i];
-            }
-            asm volatile("" ::: "memory");
-            const lds_char* const src8 = buf + ((16 * j + R) & ~3);
-            uint32_t d[5];
-#pragma unroll
-            for (int i = 0; i < 5; ++i) d[i] = *(const lds_u32*)(src8 + 4 * i);
-            const uint32_t sh = (uint32_t)(R & 2) * 8u;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) praw[i] = (int)(__builtin_amdgcn_alignbit(d[i + 1], d[i], sh) & pmask[i]);
+            for (int i = 0; i < 4; ++i) praw[i] &= (int)pmask[i];
         } else if (L == 16 && ror8) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) praw[e] = dpp<kDppRor8>(x[e]);

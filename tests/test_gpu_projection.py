@@ -119,6 +119,24 @@ def test_qkv_sections_match_the_oracle(M, K, heads, R, bias, seqlen):
     check_qkv(x, w, b, nwq, nwk, cos, sin, seqlen, y)
 
 
+# One launch per tile shape (features x tokens, from 128 x 32 to 256 x 256),
+# with a ragged last token tile, a half-width last feature tile where the head
+# count is odd, and reductions shorter and longer than the shape's stage rings.
+@pytest.mark.parametrize(
+    "M, K, heads, R",
+    [
+        (1, 128, 1, 128), (45, 1280, 1, 126), (500, 256, 8, 96), (1290, 128, 5, 42), (1290, 640, 5, 128), (1990, 384, 8, 126),
+        (2990, 128, 5, 64), (2990, 640, 8, 128), (1290, 256, 20, 126), (4490, 128, 8, 128), (4490, 256, 8, 48),
+        (1990, 128, 20, 126), (1990, 384, 20, 128),
+    ],
+)
+def test_every_tile_shape(M, K, heads, R):
+    x, w, b, nwq, nwk = make(M, K, heads, R, True, seed=M + K)
+    cos, sin = tables(M, R)
+    y = run_qkv(x, w, b, nwq, nwk, cos, sin, M)
+    check_qkv(x, w, b, nwq, nwk, cos, sin, M, y)
+
+
 def test_3d_rope_tables_of_the_480p_grid():
     grid = (2, 10, 16)
     S = grid[0] * grid[1] * grid[2]
