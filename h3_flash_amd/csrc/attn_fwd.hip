@@ -661,7 +661,7 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
         }
     };
 
-    // Pipeline: K_t and V_t live in LDS stage t % 4. Iteration j issues the
+    // Pipeline: K_t and V_t live in LDS stage (t + off) % 4. Iteration j issues the
     // QK^T of tile j+2, the softmax of tile j+1 and the PV of tile j, and the
     // DMA of K_{j+5} (into K_{j+1}'s stage) and V_{j+3} (into V_{j-1}'s); its
     // last PV steps already read the first K fragments of tile j+3. At its
@@ -677,16 +677,58 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
     constexpr std::integral_constant<int, 0> kNoSoftmax{};
     constexpr std::integral_constant<int, 1> kSoftmax{};
     constexpr std::integral_constant<int, 2> kFirstSoftmax{};
-    const int nsteps = (ntiles + 3) & ~3;
+    // The loop's steps come in groups of four with fixed stages (step U of a
+    // group: key tile jj with jj + off = U mod 4). Key tiles are padded to an
+    // even count: off = 2 shifts every tile by two stages, so that the steps
+    // start in the middle of a group and the last one still has U = 3. (The
+    // wide forms, whose V window moves with the groups, and persistent
+    // launches, whose next-tile loads go to fixed stages, pad to a multiple of
+    // four. 40 heads of 1,296 x 1,296, 21 key tiles: 22 steps against 24.)
+    constexpr bool kEven = !kWide && !kPersist;
+    const int nsteps = kEven ? (ntiles + 1) & ~1 : (ntiles + 3) & ~3;
+    const int off = kEven ? nsteps & 2 : 0;
+    // Whether this wave's 32 rows lie past the last query row: it only keeps
+    // its share of the DMA and the barriers going, so that the SIMDs and the
+    // power it would take go to the other waves.
+    if (kEven && m0 + wave * 32 >= sq && ntiles > 0) {
+        auto stage = [&](int t) { return (t + off) & 3; };
+        if (issue) {
+            dma_k(0, stage(0));
+            dma_k(1, stage(1));
+            dma_v(0, stage(0));
+            dma_k(2, stage(2));
+            dma_v(1, stage(1));
+            dma_k(3, stage(3));
+            dma_v(2, stage(2));
+        }
+        wait_vmcnt<6 * kDmaPerTile>();
+        barrier();
+        barrier();
+        dma_k(4, stage(4));
+        wait_vmcnt<6 * kDmaPerTile>();
+        barrier();
+        wait_vmcnt<2 * kDmaPerTile>();
+        barrier();
+        for (int jj = 0; jj < nsteps; ++jj) {
+            if (jj < nsteps - 2) {
+                dma_k(jj + 5, stage(jj + 1));
+                dma_v(jj + 3, stage(jj + 3));
+            }
+            wait_vmcnt<2 * kDmaPerTile>();
+            barrier();
+        }
+        wait_vmcnt<0>();
+        return false;
+    }
     if (ntiles > 0) {
         if (issue) {
-            dma_k(0, 0);
-            dma_k(1, 1);
-            dma_v(0, 0);
-            dma_k(2, 2);
-            dma_v(1, 1);
-            dma_k(3, 3);
-            dma_v(2, 2);
+            dma_k(0, off);
+            dma_k(1, 1 + off);
+            dma_v(0, off);
+            dma_k(2, 2 ^ off);
+            dma_v(1, 1 + off);
+            dma_k(3, 3 ^ off);
+            dma_v(2, 2 ^ off);
         }
         // Prefetched by the previous tile, in this order, before that
         // tile's O stores: the stores are younger, so each wait below only
@@ -696,19 +738,19 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
         for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]));  // no Q use before the wait
         barrier();
 #pragma unroll
-        for (int t = 0; t < 4; ++t) kf[t] = kread(0, t);
-        iterate(std::true_type{}, kNoSoftmax, std::false_type{}, 0, 0, 0, sb, sa, pfb, pfb, -1, no_hook);
-        barrier();  // K stage 0 is free
-        dma_k(4, 0);
+        for (int t = 0; t < 4; ++t) kf[t] = kread(off, t);
+        iterate(std::true_type{}, kNoSoftmax, std::false_type{}, off, 0, 0, sb, sa, pfb, pfb, -1, no_hook);
+        barrier();  // K_0's stage is free
+        dma_k(4, off);
         wait_vmcnt<6 * kDmaPerTile>();  // K_1 has landed
         barrier();
 #pragma unroll
-        for (int t = 0; t < 4; ++t) kf[t] = kread(1, t);
-        iterate(std::true_type{}, kFirstSoftmax, std::false_type{}, 1, 0, 0, sa, sb, pfb, pfa, -1, no_hook);
+        for (int t = 0; t < 4; ++t) kf[t] = kread(1 + off, t);
+        iterate(std::true_type{}, kFirstSoftmax, std::false_type{}, 1 + off, 0, 0, sa, sb, pfb, pfa, -1, no_hook);
         wait_vmcnt<2 * kDmaPerTile>();  // V_0, K_2, V_1 and K_3 too
-        barrier();                      // and K stage 1 is free
+        barrier();                      // and K_1's stage is free
 #pragma unroll
-        for (int t = 0; t < 4; ++t) kf[t] = kread(2, t);
+        for (int t = 0; t < 4; ++t) kf[t] = kread(2 ^ off, t);
     }
     // Persistent launches: the first PV-only iteration issues the next
     // tile's Q loads (Q's registers are dead after the last QK^T) and its
@@ -809,6 +851,13 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
         barrier();
     };
     int j = 0;
+    if constexpr (kEven) {
+        if (off != 0 && nsteps > 2) {
+            step(std::integral_constant<int, 2>{}, 0, std::false_type{});
+            step(std::integral_constant<int, 3>{}, 1, std::false_type{});
+            j = 2;
+        }
+    }
     for (; j < nsteps - 4; j += 4) {
         step(std::integral_constant<int, 0>{}, j, std::false_type{});
         step(std::integral_constant<int, 1>{}, j + 1, std::false_type{});
@@ -823,10 +872,13 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
         l32 = lane & 31;
     }
     if (nsteps > 0) {
-        step(std::integral_constant<int, 0>{}, j, std::false_type{});
-        step(std::integral_constant<int, 1>{}, j + 1, std::false_type{});
-        step(std::integral_constant<int, 2>{}, j + 2, std::true_type{});
-        step(std::integral_constant<int, 3>{}, j + 3, std::true_type{});
+        if (!kEven || nsteps > 2) {
+            step(std::integral_constant<int, 0>{}, j, std::false_type{});
+            step(std::integral_constant<int, 1>{}, j + 1, std::false_type{});
+            j += 2;
+        }
+        step(std::integral_constant<int, 2>{}, j, std::true_type{});
+        step(std::integral_constant<int, 3>{}, j + 1, std::true_type{});
     }
     if (!pref) wait_vmcnt<0>();  // no LDS DMA may still land after the workgroup ends (a prefetch lands for the next tile)
 
