@@ -19,6 +19,8 @@ H3A_OK = 0
 H3A_EINVAL = -1
 H3A_EUNSUPPORTED = -2
 H3A_ELAUNCH = -3
+H3A_NEED_WORKSPACE = 1
+H3A_WORKSPACE_ASK = -(1 << 63)
 
 H3A_DTYPE_BF16 = 0
 H3A_DTYPE_F32 = 1

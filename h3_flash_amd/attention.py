@@ -101,8 +101,10 @@ def flash_attn_func(
     key-range pieces (taken from a counter as CUs free up when there are
     more tiles than CUs; statically assigned when a single round would
     leave most CUs idle), merged by a second kernel; the workspace comes
-    from torch's stream-ordered caching allocator. ``False`` runs every
-    tile whole (results differ by rounding).
+    from torch's stream-ordered caching allocator. Short attention, and at
+    most 32 rows past the whole tiles, run as units of 32 rows with the keys
+    split over a workgroup's waves (no workspace). ``False`` runs every tile
+    whole (results differ by rounding).
 
     Raises RuntimeError for semantics the dense path does not serve (causal,
     GQA) and for a missing library, mirroring dense_fa4.py:19-20,72-73.
@@ -174,12 +176,16 @@ def flash_attn_func(
     lib = _ext.load_library()
     workspace = None
     with torch.cuda.device(q.device):
-        need = lib.h3a_attn_fwd_workspace_size(ctypes.byref(args)) if split_tail else 0
-        if need > 0:
+        stream = ctypes.c_void_p(_stream_handle(q.device))
+        if split_tail:
+            args.workspace_bytes = _ext.H3A_WORKSPACE_ASK
+        rc = lib.h3a_attn_fwd(ctypes.byref(args), stream)
+        if rc == _ext.H3A_NEED_WORKSPACE:
             # Stream-ordered caching allocation: reused, not freed, after the call.
+            need = lib.h3a_attn_fwd_workspace_size(ctypes.byref(args))
             workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
             args.workspace, args.workspace_bytes = workspace.data_ptr(), need
-        rc = lib.h3a_attn_fwd(ctypes.byref(args), ctypes.c_void_p(_stream_handle(q.device)))
+            rc = lib.h3a_attn_fwd(ctypes.byref(args), stream)
     if rc != _ext.H3A_OK:
         message = _ext.last_error(lib)
         if rc == _ext.H3A_EINVAL:

@@ -82,6 +82,10 @@ constexpr int kQueueMinKeyTiles = 48;
 // Key tiles from which a 4-way queued split is graded (its small pieces keep
 // 32 key tiles or more).
 constexpr int kGradedMinKeyTiles = 256;
+// Times in a launch's last round (plan_attn_split), in us: the fixed part of a
+// tile or piece, and the launches that pieces add. At most kMaxPieces pieces.
+constexpr double kTileUs = 9.7, kPiecesUs = 14.0;
+constexpr int kMaxPieces = 8;
 
 static_assert(kDmaPerTile == 2, "vmcnt accounting below assumes 2 K + 2 V loads per iteration");
 static_assert(kStages == 4, "the pipeline below is unrolled over four stages");
@@ -942,6 +946,255 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
     return pref;
 }
 
+// Short attention: 32 query rows of one head per workgroup, the keys split
+// over its eight waves. Wave w takes key blocks w, w + 8, ... of 32 keys
+// through a K and a V buffer of its own (8 KB each, the same swizzle as the
+// tile's), so the loop has no barrier: K of the next block is loaded once this
+// block's K fragments are in registers, V once its V fragments are. Each wave
+// keeps an exact running max; at the end the eight partial results (fp32 O, max
+// and sum) are merged through LDS and stored: no second launch, no workspace.
+// Bound by latency: a few dependent loads and 16 MFMAs per block. Against the
+// 256-row tiles 5 heads of 640 x 640 went from 14.5 to 9.0 us, 14 segments of 1
+// to 278 rows at 8 heads from 28.4 to 9.4.
+constexpr int kUnitRows = 32;
+constexpr int kUnitKeys = 32;
+constexpr int kUnitBuf = kUnitKeys * kRow;  // 8 KB
+
+struct UnitView {
+    const char *q, *k, *v;  // first query row of the unit, first key of its sequence
+    char* o;
+    float* lse;             // NULL: not wanted
+    int rows, sk;           // query rows (at most 32 count) and keys
+};
+
+template <typename Params>
+__device__ __forceinline__ void attn_unit(Params& p, const UnitView& u) {
+    char* const smem = attn_lds();
+    __shared__ float stat[kWaves][2][kUnitRows];
+    const int tid = threadIdx.x, lane = tid & 63, hi = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    char* const kbuf = smem + wave * 2 * kUnitBuf;
+    const int nblk = (u.sk + kUnitKeys - 1) / kUnitKeys;
+    const i32x4 rk = make_rsrc_words(u.k, span_bytes(u.sk, p.k_rs));
+    const i32x4 rv = make_rsrc_words(u.v, span_bytes(u.sk, p.v_rs));
+    // DMA map: load i fills rows 4i .. 4i+3 of a block; lane L writes LDS chunk
+    // (L & 15) of row 4i + (L >> 4), which holds the row's chunk (L & 15) ^
+    // swz(row), swz(row) = 4 (L >> 4) ^ (i & 3).
+    const int chunk = (lane & 15) ^ ((lane >> 4) << 2);
+    uint32_t dk[4], dv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        dk[i] = (uint32_t)((lane >> 4) * p.k_rs + ((chunk ^ i) << 4));
+        dv[i] = (uint32_t)((lane >> 4) * p.v_rs + ((chunk ^ i) << 4));
+    }
+    const uint32_t lds_k = (uint32_t)(uintptr_t)(const lds_char*)kbuf;
+    // Rows past the last key are outside the records (the scalar offset
+    // counts in the range check): zeros.
+    auto dma = [&](const i32x4& r, const uint32_t* voff, int rs, uint32_t dst, int blk) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                         :
+                         : "s"(dst + i * 1024), "v"(voff[i & 3]), "s"(r), "s"((uint32_t)((blk * kUnitKeys + 4 * i) * rs))
+                         : "memory");
+    };
+    const int l15 = lane & 15, jr = l15 >> 2;
+    const int vbase = (4 * hi + jr) * kRow + ((32 * ((lane >> 4) & 1)) ^ (16 * ((l15 & 3) >> 1)) ^ (64 * jr) ^ (16 * hi)) + (l15 & 1) * 8;
+    const lds_char* const kl = (const lds_char*)kbuf;
+    const lds_char* const vl = kl + kUnitBuf;
+
+    // Q (the B operand of S^T = K Q^T): rows past the view load as zeros.
+    const __amdgpu_buffer_rsrc_t rq = make_rsrc(u.q, span_bytes(min(u.rows, kUnitRows), p.q_rs));
+    bf16x8 qf[8];
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+        qf[ks] = __builtin_bit_cast(bf16x8, buf_load16(rq, (uint32_t)(l32 * p.q_rs + ks * 32 + hi * 16)));
+    const float c = p.scale_log2;
+    f32x16 oacc[4] = {f32x16{}, f32x16{}, f32x16{}, f32x16{}};
+    float mc = -INFINITY, l_run = 0.f;  // max (log2 units) and this lane's part of the sum
+    int blk = wave;
+    if (blk < nblk) {
+        dma(rk, dk, p.k_rs, lds_k, blk);
+        dma(rv, dv, p.v_rs, lds_k + kUnitBuf, blk);
+    }
+    for (; blk < nblk; blk += kWaves) {
+        const int next = blk + kWaves;
+        wait_vmcnt<8>();  // K has landed (V, issued after it, may be in flight)
+        asm volatile("" ::: "memory");
+        f32x16 s{};
+        {
+            bf16x8 kf[8];
+#pragma unroll
+            for (int ks = 0; ks < 8; ++ks)
+                kf[ks] = *(const lds_bf16x8*)(kl + l32 * kRow + (((2 * ks + hi) ^ swz(l32)) << 4));
+#pragma unroll
+            for (int ks = 0; ks < 8; ++ks) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qf[ks], s, 0, 0, 0);
+        }
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): K's buffer is read
+        asm volatile("" ::: "memory");
+        const bool more = next < nblk;
+        if (more) dma(rk, dk, p.k_rs, lds_k, next);
+        if ((blk + 1) * kUnitKeys > u.sk) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (blk * kUnitKeys + (r >> 2) * 8 + hi * 4 + (r & 3) >= u.sk) s[r] = -INFINITY;
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+        const f32x2 hm = halves(mx);
+        const float m_new = fmaxf(mc, fmaxf(hm.x, hm.y) * c);
+        if (__builtin_amdgcn_ballot_w64(m_new > mc)) {
+            const float alpha = fast_exp2(mc - m_new);
+            mc = m_new;
+            l_run *= alpha;
+#pragma unroll
+            for (int db = 0; db < 4; ++db)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
+        }
+        // (A block of scores that overflowed to -inf leaves the max there; its
+        // p are zero, as against any finite offset.)
+        const float mo = mc == -INFINITY ? 0.f : mc;
+        bf16x8 pf[2];
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc) {
+            i32x4 w;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float a = fast_exp2(__builtin_fmaf(s[8 * cc + 2 * i], c, -mo));
+                const float b = fast_exp2(__builtin_fmaf(s[8 * cc + 2 * i + 1], c, -mo));
+                l_run += a + b;
+                w[i] = (int)pack_bf16x2(a, b);
+            }
+            pf[cc] = __builtin_bit_cast(bf16x8, w);
+        }
+        if (more)
+            wait_vmcnt<8>();  // V has landed (the next K may be in flight)
+        else
+            wait_vmcnt<0>();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+            for (int db = 0; db < 4; ++db) {
+                const lds_char* const a = vl + cc * 16 * kRow;
+                const i32x2 lo = read_tr(a + (vbase ^ (64 * db)));
+                const i32x2 up = read_tr(a + 8 * kRow + (vbase ^ (64 * db) ^ 32));
+                oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    __builtin_bit_cast(bf16x8, i32x4{lo.x, lo.y, up.x, up.y}), pf[cc], oacc[db], 0, 0, 0);
+            }
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): V's buffer is read
+        asm volatile("" ::: "memory");
+        if (more) dma(rv, dv, p.v_rs, lds_k + kUnitBuf, next);
+    }
+    {
+        const f32x2 pr = halves(l_run);
+        l_run = pr.x + pr.y;
+    }
+    // Partial O over the wave's own buffers (16 KB: 32 rows of 128 fp32): row
+    // l32, 16-byte chunk d/4 at chunk ^ row.
+    typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+    lds_char* const part = (lds_char*)kbuf;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *(lds_f32x4*)(part + l32 * 512 + (((8 * db + 2 * i + hi) ^ l32) << 4)) =
+                f32x4{oacc[db][4 * i], oacc[db][4 * i + 1], oacc[db][4 * i + 2], oacc[db][4 * i + 3]};
+    if (hi == 0) {
+        stat[wave][0][l32] = mc;
+        stat[wave][1][l32] = l_run;
+    }
+    __syncthreads();
+    // Sixteen lanes per row, eight head dims each.
+    const int row = tid >> 4, j = tid & 15;
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) top = fmaxf(top, stat[w][0][row]);
+    float sum = 0.f;
+    f32x4 acc[2] = {f32x4{}, f32x4{}};
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        const float m = stat[w][0][row];
+        const float e = m == -INFINITY ? 0.f : fast_exp2(m - top);  // a wave without keys weighs nothing
+        sum += e * stat[w][1][row];
+        const lds_char* const src = (const lds_char*)smem + w * 2 * kUnitBuf + row * 512;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[i] += e * *(const lds_f32x4*)(src + (((2 * j + i) ^ row) << 4));
+    }
+    if (row < u.rows) {
+        const float inv = sum > 0.f ? 1.0f / sum : 0.f;
+        i32x4 w;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            w[i] = (int)pack_bf16x2(acc[i >> 1][2 * (i & 1)] * inv, acc[i >> 1][2 * (i & 1) + 1] * inv);
+        *(i32x4*)(u.o + (int64_t)row * p.o_rs + j * 16) = w;
+        if (u.lse != nullptr && j == 0) u.lse[row] = sum > 0.f ? (top + __log2f(sum)) * 0.69314718055994531f : -INFINITY;
+    }
+}
+
+// The unit of rows [m0, m0 + 32) of head h of batch (or packed segment) grp.
+template <typename Params>
+__device__ __forceinline__ void attn_unit_at(Params& p, int grp, int h, int m0) {
+    int b = grp, q0 = 0, k0 = 0, sq = p.seqlen_q, sk = p.seqlen_k;
+    if (p.cu_q != nullptr) {
+        b = 0;
+        q0 = min(max(p.cu_q[grp], 0), p.seqlen_q);
+        sq = min(max(p.cu_q[grp + 1], q0), p.seqlen_q) - q0;
+        k0 = min(max(p.cu_k[grp], 0), p.seqlen_k);
+        sk = min(max(p.cu_k[grp + 1], k0), p.seqlen_k) - k0;
+    }
+    if (m0 >= sq) return;  // the whole workgroup: past this segment
+    attn_unit(p, UnitView{(const char*)p.q + 2 * (b * p.q_sb + h * p.q_sh) + (int64_t)(q0 + m0) * p.q_rs,
+                          (const char*)p.k + 2 * (b * p.k_sb + h * p.k_sh) + (int64_t)k0 * p.k_rs,
+                          (const char*)p.v + 2 * (b * p.v_sb + h * p.v_sh) + (int64_t)k0 * p.v_rs,
+                          (char*)p.o + 2 * (b * p.o_sb + h * p.o_sh) + (int64_t)(q0 + m0) * p.o_rs,
+                          p.lse == nullptr ? nullptr : p.lse + b * p.lse_sb + h * p.lse_sh + q0 + m0, sq - m0, sk});
+}
+
+// A launch of units alone, contiguous per XCD (a head's units share its K/V in
+// that XCD's L2). Dense: n_units per (batch, head). Packed: the units of the
+// segments one after another, a segment's heads outermost; which segment a
+// workgroup's unit lies in is found from the offsets (64 segments at a time, a
+// lane each), so no workgroup goes to the rows that shorter segments lack (a
+// grid of n_units per segment: 14 segments of 1 to 486 rows, 8 heads, 51 us;
+// this one 36). Workgroups past the last unit end at once.
+__global__ __launch_bounds__(kThreads, 2) void attn_short_kernel(AttnParams p) {
+    const int nb = gridDim.x, bid = blockIdx.x;
+    const int xcd = bid & 7, per = nb >> 3, rem = nb & 7;
+    int unit = xcd * per + min(xcd, rem) + (bid >> 3);
+    if (p.cu_q == nullptr) {
+        const int rest = unit / p.n_units;
+        attn_unit_at(p, rest / p.heads, rest % p.heads, unit % p.n_units * kUnitRows);
+        return;
+    }
+    const int lane = threadIdx.x & 63;
+    for (int s0 = 0; s0 < p.n_groups; s0 += 64) {
+        const int s = s0 + lane;
+        int n = 0;
+        if (s < p.n_groups) {
+            const int q0 = min(max(p.cu_q[s], 0), p.seqlen_q), q1 = min(max(p.cu_q[s + 1], q0), p.seqlen_q);
+            n = min((q1 - q0 + kUnitRows - 1) / kUnitRows, p.n_units);
+        }
+        int incl = n * p.heads;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int up = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += up;
+        }
+        const uint64_t past = __builtin_amdgcn_ballot_w64(incl > unit);
+        if (past != 0) {
+            const int at = __builtin_ctzll(past);
+            const int units = __builtin_amdgcn_readlane(n, at);
+            unit -= __builtin_amdgcn_readlane(incl, at) - units * p.heads;
+            attn_unit_at(p, s0 + at, unit / units, unit % units * kUnitRows);
+            return;
+        }
+        unit -= __builtin_amdgcn_readlane(incl, 63);
+    }
+}
+
 // The dynamic tail: the last round's tiles are cut into key-range pieces
 // that the workgroups after the whole tiles take from a counter in the
 // workspace as they free up, so CUs that ran their whole tiles faster (XCD
@@ -965,6 +1218,20 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
     // XCDs nearly only empty tiles: the 49,920 + 1,296 two-segment batch ran
     // at half speed).
     const int bid = blockIdx.x;
+    // Dense launches whose last query tile would hold at most 32 rows run
+    // those as units, one per (batch, head), on the last rag_blocks workgroups:
+    // a tile for them keeps a CU as long as one or two rows of tiles do (40
+    // heads of 1,560 x 1,560, 240 whole tiles on 256 CUs: 66.9 -> 53.8 us).
+    const int n_blocks = (int)gridDim.x - p.rag_blocks;
+    if constexpr (!kWide) {
+        if (bid >= n_blocks) {
+            for (int u = bid - n_blocks; u < p.heads * p.n_groups; u += p.rag_blocks) {
+                attn_unit_at(p, u / p.heads, u % p.heads, p.n_qtiles * kBM);
+                __syncthreads();  // the merge has read the buffers that the next unit fills
+            }
+            return;
+        }
+    }
     // First work item of this wave (wide forms: read once, kept as a scalar).
     const int wave_first = kWide ? __builtin_amdgcn_readfirstlane((int)threadIdx.x) & ~63 : 0;
     int tile = bid, chunk = -1, chunks = 1, slot = -1;
@@ -979,7 +1246,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
         if (bid >= p.vplan[kPlanFull]) return;
         tile = __builtin_amdgcn_readfirstlane(p.vlist[bid]);  // uniform: the addressing is scalar
     } else if (p.cu_q == nullptr && !queued) {
-        const int nb = p.queue != nullptr ? p.n_full : (int)gridDim.x;
+        const int nb = p.queue != nullptr ? p.n_full : n_blocks;
         const int xcd = bid & 7, local = bid >> 3, per = nb >> 3, rem = nb & 7;
         const int start = xcd * per + min(xcd, rem);  // first tile of this XCD's share
         tile = start + local;
@@ -1389,6 +1656,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
 
 }  // namespace
 
+int attn_fwd_unit_rows() { return kUnitRows; }
 int attn_fwd_block_m() { return kBM; }
 int attn_fwd_persist_max_rows() { return kPersistMaxQTiles * kBM; }
 int attn_fwd_tail_pieces() { return kQueuePieces; }
@@ -1396,6 +1664,18 @@ int64_t attn_fwd_piece_bytes() { return (int64_t)kBM * (kD * 2 + 4); }
 int attn_fwd_block_n() { return kBN; }
 int attn_fwd_window_rows() { return kWindowRows > kBM ? kWindowRows : kBM; }
 int attn_fwd_row_margin() { return kBM + kBN * (2 * kStages + 2); }
+
+int attn_rag_blocks(int64_t tiles, int64_t units, int64_t keys, int cus) {
+    // The units run one after another on the CUs that the last round of tiles
+    // leaves idle where they have the time for it, else one per workgroup. (As
+    // one workgroup each they would wait for a CU of the shader engine whose
+    // turn it is, though others are idle: 40 units beside 240 tiles took 13 us
+    // longer than 36 beside 216.)
+    const int64_t idle = cus > 0 ? (cus - tiles % cus) % cus : 0;
+    const double tile_us = kTileUs + 1.6 * (double)((keys + kBN - 1) / kBN);
+    const double unit_us = 5.0 + 1.6 * (double)((keys + kUnitKeys * kWaves - 1) / (kUnitKeys * kWaves));
+    return (int)(idle * (int64_t)(tile_us / unit_us) >= units && idle < units ? idle : units);
+}
 
 SplitPlan plan_attn_split(int64_t tiles, int64_t key_tiles, int cus, int64_t max_workspace) {
     SplitPlan plan{(int32_t)tiles, 0, 0, 0, 0, 0};
@@ -1412,6 +1692,27 @@ SplitPlan plan_attn_split(int64_t tiles, int64_t key_tiles, int cus, int64_t max
         auto bytes = [&](int n) { return ((int64_t)n * rest * piece_bytes + 255) / 256 * 256 + 256; };
         int n = kQueuePieces;
         while (n > 1 && (key_tiles / n < kQueueMinKeyTiles || bytes(n) > max_workspace)) --n;
+        if (n < 2) {
+            // Shorter key ranges: pieces pay where they fill a last round that
+            // would leave CUs idle, by the expected time: a tile's or piece's
+            // fixed part, its key tiles (slower the more CUs are busy: power),
+            // and what pieces cost besides (the counter's reset, the merge).
+            // Measured (us, whole -> pieces): 24 heads of 4,096 x 4,096 200 ->
+            // 185, 40 of 2,048 x 2,048 100 -> 92, 20 of 3,500 x 3,500 162 ->
+            // 125; 8 of 10,240 x 1,024 58 -> 60, which the rule leaves whole.
+            auto last_round = [&](int64_t jobs, double kt) {
+                const double busy = jobs < cus ? (double)jobs / (double)cus : 1.0;
+                return (double)((jobs + cus - 1) / cus) * (kTileUs + kt * (1.0 + 0.6 * busy));
+            };
+            double best = last_round(rest, (double)key_tiles) - 2.0;
+            for (int c = 2; c <= kMaxPieces && key_tiles / c >= 2 && bytes(c) <= max_workspace; ++c) {
+                const double us = last_round(rest * c, (double)key_tiles / c) + kPiecesUs;
+                if (us < best) {
+                    best = us;
+                    n = c;
+                }
+            }
+        }
         if (n < 2) return plan;
         plan.n_full = (int32_t)full;
         plan.split_n = n;
@@ -1468,6 +1769,14 @@ hipError_t attn_static_scratch(void** ptr) {
 }
 
 hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t stream) {
+    if (p.n_units > 0) {
+        // Packed: no more than the rows and a part of a unit per segment give.
+        int64_t units = (int64_t)p.n_units * p.heads * p.n_groups;
+        const int64_t rows = p.heads * ((int64_t)p.seqlen_q / kUnitRows + p.n_groups);
+        if (p.cu_q != nullptr && rows < units) units = rows;
+        hipLaunchKernelGGL(attn_short_kernel, dim3((unsigned)units), dim3(kThreads), 0, stream, p);
+        return hipGetLastError();
+    }
     const int64_t tiles = (int64_t)p.n_qtiles * p.heads * p.n_groups;
     if (tiles <= 0) return hipSuccess;
     int64_t blocks = tiles;
@@ -1498,7 +1807,7 @@ hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t stream) {
         hipLaunchKernelGGL(attn_fwd_persist_kernel, dim3((unsigned)n), block, 0, stream, p);
         return hipGetLastError();
     }
-    const dim3 grid((unsigned)blocks);
+    const dim3 grid((unsigned)(blocks + p.rag_blocks));
     if (p.wide && p.vt != nullptr)
         hipLaunchKernelGGL((attn_fwd_kernel<true, true>), grid, block, 0, stream, p);
     else if (p.wide)

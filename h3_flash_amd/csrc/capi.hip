@@ -164,6 +164,47 @@ int device_cus() {
     return n;
 }
 
+// Dense launches with at most 32 rows past their whole tiles run those rows as
+// units beside the tiles.
+void take_rag_units(const h3a_attn_args* a, h3a::AttnParams& p) {
+    const int64_t rag = a->seqlen_q % h3a::attn_fwd_block_m();
+    if (p.cu_q != nullptr || p.wide != 0 || p.n_qtiles < 2 || rag == 0 || rag > h3a::attn_fwd_unit_rows()) return;
+    p.n_qtiles -= 1;
+    const int64_t units = (int64_t)p.heads * p.n_groups;
+    p.rag_blocks = h3a::attn_rag_blocks(units * p.n_qtiles, units, a->seqlen_k, device_cus());
+}
+
+// Units per (group, head) of a launch that runs as units of 32 rows (short
+// attention), or 0 where the 256-row tiles are faster.
+int32_t attn_units(const h3a_attn_args* a, const h3a::AttnParams& p) {
+    const int cus = device_cus();
+    if (p.wide != 0 || cus <= 0) return 0;
+    const int64_t rows = a->cu_seqlens_q != nullptr ? a->max_seqlen_q : a->seqlen_q;
+    const int64_t n = (rows + h3a::attn_fwd_unit_rows() - 1) / h3a::attn_fwd_unit_rows();
+    // Every unit reads all keys of its head, so units win while they all run
+    // at once, or in two rounds over few keys. Timed, heads x Sq x Sk (us, tiles
+    // -> units): 5 x 640 x 640 14.5 -> 9.0, 10 x 640 x 640 18.5 -> 9.4, 4 x
+    // 2,048 x 2,048 25.3 -> 18.5, 10 x 1,024 x 1,024 24.5 -> 22.1; 4 x 640 x
+    // 4,096 24.6 -> 25.1, 5 x 2,048 x 2,048 28.6 -> 32.7, 40 x 640 x 640 26.5
+    // -> 34.7.
+    if (a->cu_seqlens_q == nullptr) {
+        const int64_t units = n * p.heads * p.n_groups;
+        return (units <= cus && a->seqlen_k <= 2048) || (units <= 2 * cus && units * a->seqlen_k <= 400000) ? (int32_t)n : 0;
+    }
+    // Packed: by the expected time of either, from the units there can be (the
+    // host knows only the rows' total) and the longest key range (that of the
+    // queries when both share their offsets, else all keys at most). On 45
+    // mixes of 1 to 3,000 rows at 1 to 8 heads the tiles measured about 13 us +
+    // 0.9 per 64 keys + 0.018 per unit (planning launch, the longest tile, the
+    // work), rounds of units 4.3 us + 1.5 per 256 keys, a tenth more with
+    // ragged ends; this picked the faster one for all but one (0.84 of it).
+    const int64_t units = p.heads * (a->seqlen_q / h3a::attn_fwd_unit_rows() + (int64_t)a->num_segments);
+    const int64_t keys = a->cu_seqlens_k == a->cu_seqlens_q ? a->max_seqlen_q : a->seqlen_k;
+    const double tiles_us = 13.0 + 0.9 / 64.0 * (double)keys + 0.018 * (double)units;
+    const double units_us = 1.1 * (double)((units + cus - 1) / cus) * (4.3 + 1.5 * (double)((keys + 255) / 256));
+    return units_us < tiles_us ? (int32_t)n : 0;
+}
+
 // Split plan of a validated launch: dense inputs only (varlen tiles are not
 // uniform work).
 h3a::SplitPlan attn_plan(const h3a_attn_args* a, const h3a::AttnParams& p, int64_t max_workspace = INT64_MAX) {
@@ -191,6 +232,7 @@ struct AttnWorkspace {
 
 AttnWorkspace attn_workspace(const h3a_attn_args* a, const h3a::AttnParams& p, bool allow_vt,
                              int64_t max_workspace = INT64_MAX) {
+    if (p.n_units > 0) return AttnWorkspace{};
     AttnWorkspace w{attn_plan(a, p, max_workspace), 0, 0, 0, 0, 0, 0, false};
     w.total = w.plan.workspace_bytes;
     const int bn = h3a::attn_fwd_block_n();
@@ -325,7 +367,15 @@ int h3a_attn_fwd(const h3a_attn_args* a, void* stream) {
     bool empty = false;
     const int rc = prepare_attn(a, p, &empty);
     if (rc != H3A_OK || empty) return rc;
+    // Without a workspace every tile runs whole, unless the caller asks to be
+    // told where the launch takes one.
+    const bool ask = a->workspace == nullptr && a->workspace_bytes == H3A_WORKSPACE_ASK;
+    if (ask || a->workspace != nullptr) {
+        p.n_units = attn_units(a, p);
+        if (p.n_units == 0) take_rag_units(a, p);
+    }
     const AttnWorkspace w = attn_workspace(a, p, true);
+    if (ask && w.total > 0) return H3A_NEED_WORKSPACE;
     if (w.total > 0 && a->workspace != nullptr && a->workspace_bytes >= w.total && ((uintptr_t)a->workspace & 255u) == 0) {
         if (w.plan.split_n != 0) apply_plan(p, w.plan, a->workspace);
         if (w.persist) {
@@ -363,6 +413,13 @@ int h3a_attn_fwd_noalloc(const h3a_attn_args* a, void* stream) {
     bool empty = false;
     const int rc = prepare_attn(a, p, &empty);
     if (rc != H3A_OK || empty) return rc;
+    p.n_units = attn_units(a, p);
+    if (p.n_units > 0) {
+        const hipError_t e = h3a::launch_attn_fwd(p, (hipStream_t)stream);
+        if (e != hipSuccess) return fail(H3A_ELAUNCH, "h3a_attn_fwd_noalloc: launch failed: %s", hipGetErrorString(e));
+        return H3A_OK;
+    }
+    take_rag_units(a, p);
     void* scratch = nullptr;
     hipError_t e = h3a::attn_static_scratch(&scratch);
     if (e != hipSuccess)
@@ -397,7 +454,13 @@ int64_t h3a_attn_fwd_workspace_size(const h3a_attn_args* a) {
     bool empty = false;
     const int rc = prepare_attn(a, p, &empty);
     if (rc != H3A_OK) return rc;
-    return empty ? 0 : attn_workspace(a, p, true).total;
+    if (empty) return 0;
+    // What all tiles would take (a launch that runs as units leaves it unused),
+    // or the whole tiles alone beside their ragged rows' units.
+    const int64_t tiles = attn_workspace(a, p, true).total;
+    take_rag_units(a, p);
+    const int64_t whole = attn_workspace(a, p, true).total;
+    return tiles > whole ? tiles : whole;
 }
 
 int h3a_qknorm_rope(const h3a_qknorm_rope_args* a, void* stream) {

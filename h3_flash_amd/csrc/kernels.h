@@ -76,6 +76,12 @@ struct AttnParams {
     // workgroup per tile.
     int* persist_queue;
     int32_t persist_blocks;
+    // Units of 32 query rows per (group, head) when the launch runs them in
+    // place of tiles (short attention), else 0.
+    int32_t n_units;
+    // Workgroups after the tiles that run units: the at most 32 rows past the
+    // n_qtiles whole tiles of every (batch, head) (dense, not wide), or 0.
+    int32_t rag_blocks;
 };
 
 // Words of the planned-varlen header (vplan).
@@ -97,6 +103,9 @@ SplitPlan plan_attn_split(int64_t tiles, int64_t key_tiles, int cus, int64_t max
 constexpr int64_t kStaticScratchBytes = H3A_NOALLOC_SCRATCH_BYTES;
 hipError_t attn_static_scratch(void** ptr);
 
+// Workgroups for `units` ragged units beside `tiles` whole tiles.
+int attn_rag_blocks(int64_t tiles, int64_t units, int64_t keys, int cus);
+int attn_fwd_unit_rows();  // query rows of a unit of a short launch
 int attn_fwd_block_m();
 // Longest segment (max_seqlen_q) of a persistent packed launch.
 int attn_fwd_persist_max_rows();

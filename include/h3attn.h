@@ -65,6 +65,8 @@ extern "C" {
 #define H3A_EINVAL (-1)       /* invalid argument (shape, stride, pointer) */
 #define H3A_EUNSUPPORTED (-2) /* valid request the library does not implement */
 #define H3A_ELAUNCH (-3)      /* the HIP launch itself failed */
+#define H3A_NEED_WORKSPACE 1  /* h3a_attn_fwd, asked for by H3A_WORKSPACE_ASK: nothing launched */
+#define H3A_WORKSPACE_ASK INT64_MIN
 
 /* dtype codes: norm weights and modulation tables (bf16 / fp32), table indices (int32 / int64) */
 #define H3A_DTYPE_BF16 0
@@ -132,8 +134,17 @@ extern "C" {
  *     are few tiles per CU (heads x (seqlen_q / 256 + num_segments / 2) at
  *     most 3.2 per CU, or 9 with max_seqlen_q of 2,900 or more), such calls
  *     take the planned work list above instead.
- * With a NULL or smaller workspace every tile runs whole on V as given. The
- * results differ only by rounding. Calls sharing one workspace must be
+ * With a workspace given, short attention (up to about 256 units of 32 query
+ * rows of one head and 2,048 keys, or more units over fewer keys) runs without
+ * using it, as one workgroup per unit with the keys split over its waves; so
+ * do, beside the tiles, the rows past a dense call's whole tiles when they are
+ * at most 32.
+ * With a NULL workspace every tile runs whole on V as given (a smaller one
+ * keeps the units). The results differ only by rounding. A caller that would
+ * allocate the workspace only where the launch takes one passes NULL with
+ * workspace_bytes = H3A_WORKSPACE_ASK: the call launches as with a workspace
+ * where it needs none, else it launches nothing and returns
+ * H3A_NEED_WORKSPACE, and the caller allocates and calls again. Calls sharing one workspace must be
  * ordered (same stream).
  */
 typedef struct h3a_attn_args {

@@ -30,3 +30,67 @@ def test_key_tiles_and_idle_waves(Sq, Sk):
     torch.cuda.synchronize()
     ref_out, ref_lse = sdpa_reference(q, k, v)
     assert_parity(out.cpu(), lse.cpu(), ref_out, ref_lse, f"{Sq}x{Sk}")
+
+
+# At most 32 rows past the whole query tiles: one workgroup per (batch, head)
+# after the tiles, or (43 x 6 whole tiles on 256 CUs: 2 over) fewer workgroups
+# that take several; beside the queued and the static split, with strided
+# views, and with keys from fewer than one per wave to many rounds.
+@pytest.mark.parametrize(
+    "B, H, Sq, Sk, split",
+    [(1, 2, 257, 3, True), (2, 3, 288, 700, True), (1, 40, 1560, 300, True), (1, 43, 1552, 64, True),
+     (1, 40, 1537, 100, False), (3, 5, 520, 33, False), (1, 20, 3590, 640, True)],
+)
+def test_rows_past_the_whole_tiles(B, H, Sq, Sk, split):
+    q, k, v = _qkv(B, Sq, Sk, H, Sq + Sk)
+    view = torch.empty((B, Sq, H + 1, 128), dtype=torch.bfloat16, device=DEV)[:, :, 1:]
+    view.copy_(q)
+    out, lse = flash_attn_func(view, k.to(DEV), v.to(DEV), split_tail=split)
+    torch.cuda.synchronize()
+    rows = sorted({0, Sq // 256 * 256 - 1, *range(Sq // 256 * 256, Sq)})
+    ref_out, ref_lse = sdpa_reference(q[:, rows], k, v)
+    assert_parity(out.cpu()[:, rows], lse.cpu()[:, :, rows], ref_out, ref_lse, f"{B}x{H}x{Sq}x{Sk}")
+
+
+# Units alone: one key, fewer blocks than waves, a last block of one key, no
+# keys, many blocks; packed segments with empty ones and unequal key lengths.
+@pytest.mark.parametrize("B, H, Sq, Sk", [(1, 1, 1, 1), (2, 3, 33, 0), (1, 4, 31, 257), (1, 5, 640, 640), (3, 2, 70, 225), (1, 2, 32, 2048)])
+def test_short_attention(B, H, Sq, Sk):
+    q, k, v = _qkv(B, Sq, Sk, H, 7 * Sq + Sk)
+    out, lse = flash_attn_func(q.to(DEV), k.to(DEV), v.to(DEV))
+    torch.cuda.synchronize()
+    if Sk == 0:
+        assert (out == 0).all() and (lse == float("-inf")).all()
+        return
+    ref_out, ref_lse = sdpa_reference(q, k, v)
+    assert_parity(out.cpu(), lse.cpu(), ref_out, ref_lse, f"{B}x{H}x{Sq}x{Sk}")
+
+
+@pytest.mark.parametrize("qlens, klens", [([5, 0, 64, 33], [70, 9, 0, 300]), ([1], [1]), ([200, 31, 32], [200, 31, 32])])
+def test_short_packed_segments(qlens, klens):
+    H = 3
+    q, k, v = _qkv(1, sum(qlens), sum(klens), H, sum(qlens))
+    cq, ck = (torch.tensor([0, *torch.tensor(x).cumsum(0).tolist()], dtype=torch.int32) for x in (qlens, klens))
+    out, lse = flash_attn_func(
+        q.to(DEV), k.to(DEV), v.to(DEV), cu_seqlens_q=cq.to(DEV), cu_seqlens_k=ck.to(DEV), max_seqlen_q=max(qlens)
+    )
+    torch.cuda.synchronize()
+    for (a, b), (c, d) in zip(zip(cq[:-1], cq[1:]), zip(ck[:-1], ck[1:])):
+        if a == b:
+            continue
+        if c == d:
+            assert (out[:, a:b] == 0).all() and (lse[:, :, a:b] == float("-inf")).all()
+            continue
+        ref_out, ref_lse = sdpa_reference(q[:, a:b], k[:, c:d], v[:, c:d])
+        assert_parity(out[:, a:b].cpu(), lse[:, :, a:b].cpu(), ref_out, ref_lse, f"rows {a}:{b}")
+
+
+# Queued last rounds over short key ranges (pieces of a few key tiles).
+@pytest.mark.parametrize("H, Sq, Sk", [(20, 3500, 1500), (40, 2048, 2048), (70, 1024, 1300)])
+def test_last_round_pieces_of_short_key_ranges(H, Sq, Sk):
+    q, k, v = _qkv(1, Sq, Sk, H, Sk)
+    out, lse = flash_attn_func(q.to(DEV), k.to(DEV), v.to(DEV))
+    torch.cuda.synchronize()
+    h = [0, H - 1]
+    ref_out, ref_lse = sdpa_reference(q[:, :, h], k[:, :, h], v[:, :, h])
+    assert_parity(out.cpu()[:, :, h], lse.cpu()[:, h], ref_out, ref_lse, f"{H}x{Sq}x{Sk}")
