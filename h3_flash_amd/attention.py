@@ -25,7 +25,6 @@ Nothing here falls back to another backend.
 
 from __future__ import annotations
 
-import ctypes
 import math
 from collections.abc import Callable
 from typing import Any
@@ -50,24 +49,15 @@ __all__ = [
 HEAD_DIM = 128
 
 
-def _strides3(t: torch.Tensor) -> tuple[int, int, int]:
-    s = t.stride()
-    return (s[0], s[1], s[2])
-
-
 def _as_kernel_operand(t: torch.Tensor, name: str) -> torch.Tensor:
     if t.dtype != torch.bfloat16:
         raise TypeError(f"{name} must be bfloat16, got {t.dtype}")
     if t.dim() != 4:
         raise ValueError(f"{name} must be 4-D (batch, seq, heads, head_dim), got {tuple(t.shape)}")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise RuntimeError(f"{name} must be on a ROCm device, got {t.device}")
-    aligned = t.stride(-1) == 1 and all(s % 8 == 0 for s in t.stride()[:3]) and t.data_ptr() % 16 == 0
-    return t if aligned else t.contiguous()
-
-
-def _stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    b, s, h, d = t.stride()
+    return t if d == 1 and not (b | s | h) & 7 and not t.data_ptr() & 15 else t.contiguous()
 
 
 def flash_attn_func(
@@ -124,40 +114,30 @@ def flash_attn_func(
         raise ValueError(f"q {tuple(q.shape)} and k {tuple(k.shape)} are incompatible")
     if k.shape[2] != H:
         raise RuntimeError("H3 dense HIP attention does not support grouped-query attention")
-    if not (q.device == k.device == v.device):
+    device = q.device
+    if k.device != device or v.device != device:
         raise ValueError("q, k and v must be on the same device")
     Sk = k.shape[1]
     scale = 1.0 / math.sqrt(D) if softmax_scale is None else float(softmax_scale)
 
     if out is None:
-        out = torch.empty((B, Sq, H, D), dtype=torch.bfloat16, device=q.device)
-    elif out.shape != (B, Sq, H, D) or out.dtype != torch.bfloat16 or out.stride(-1) != 1 or out.device != q.device:
-        raise ValueError(f"out must be a bf16 (B, Sq, H, 128) tensor on {q.device} with a contiguous last dim")
+        out = q.new_empty((B, Sq, H, D))
+    elif out.shape != (B, Sq, H, D) or out.dtype != torch.bfloat16 or out.stride(-1) != 1 or out.device != device:
+        raise ValueError(f"out must be a bf16 (B, Sq, H, 128) tensor on {device} with a contiguous last dim")
     if lse is None:
-        lse = torch.empty((B, H, Sq), dtype=torch.float32, device=q.device)
-    elif lse.shape != (B, H, Sq) or lse.dtype != torch.float32 or lse.stride(-1) != 1 or lse.device != q.device:
-        raise ValueError(f"lse must be an fp32 (B, H, Sq) tensor on {q.device} with a contiguous last dim")
+        lse = q.new_empty((B, H, Sq), dtype=torch.float32)
+    elif lse.shape != (B, H, Sq) or lse.dtype != torch.float32 or lse.stride(-1) != 1 or lse.device != device:
+        raise ValueError(f"lse must be an fp32 (B, H, Sq) tensor on {device} with a contiguous last dim")
 
-    args = _ext.AttnArgs()
-    args.abi_version = _ext.ABI_VERSION
-    args.q, args.k, args.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
-    args.o, args.lse = out.data_ptr(), lse.data_ptr()
-    args.batch, args.heads, args.seqlen_q, args.seqlen_k, args.head_dim = B, H, Sq, Sk, D
-    args.q_stride[:] = _strides3(q)
-    args.k_stride[:] = _strides3(k)
-    args.v_stride[:] = _strides3(v)
-    args.o_stride[:] = _strides3(out)
-    args.lse_stride[:] = (lse.stride(0), lse.stride(1))
-    args.softmax_scale = scale
-    args.causal = 0
+    cu_q_ptr = cu_k_ptr = segments = longest = 0
     if cu_seqlens_q is not None or cu_seqlens_k is not None:
         if cu_seqlens_q is None:
             raise ValueError("cu_seqlens_k given without cu_seqlens_q")
         if cu_seqlens_k is None:
             cu_seqlens_k = cu_seqlens_q
         for name, cu in (("cu_seqlens_q", cu_seqlens_q), ("cu_seqlens_k", cu_seqlens_k)):
-            if cu.dtype != torch.int32 or cu.dim() != 1 or cu.device != q.device or not cu.is_contiguous():
-                raise ValueError(f"{name} must be a contiguous 1-D int32 tensor on {q.device}")
+            if cu.dtype != torch.int32 or cu.dim() != 1 or cu.device != device or not cu.is_contiguous():
+                raise ValueError(f"{name} must be a contiguous 1-D int32 tensor on {device}")
         if cu_seqlens_q.numel() != cu_seqlens_k.numel() or cu_seqlens_q.numel() < 2:
             raise ValueError("cu_seqlens_q and cu_seqlens_k must have the same length >= 2")
         if B != 1:
@@ -165,32 +145,25 @@ def flash_attn_func(
         if max_seqlen_q is None:
             # One host read of the offsets (synchronises the stream).
             max_seqlen_q = int((cu_seqlens_q[1:] - cu_seqlens_q[:-1]).max().item())
-        args.cu_seqlens_q = cu_seqlens_q.data_ptr()
-        args.cu_seqlens_k = cu_seqlens_k.data_ptr()
-        args.num_segments = cu_seqlens_q.numel() - 1
-        args.max_seqlen_q = int(max_seqlen_q)
-        if args.max_seqlen_q <= 0:
+        cu_q_ptr, cu_k_ptr = cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr()
+        segments, longest = cu_seqlens_q.numel() - 1, int(max_seqlen_q)
+        if longest <= 0:
             out.zero_()
             lse.fill_(float("-inf"))
             return out, lse
-    lib = _ext.load_library()
-    workspace = None
-    with torch.cuda.device(q.device):
-        stream = ctypes.c_void_p(_stream_handle(q.device))
-        if split_tail:
-            args.workspace_bytes = _ext.H3A_WORKSPACE_ASK
-        rc = lib.h3a_attn_fwd(ctypes.byref(args), stream)
-        if rc == _ext.H3A_NEED_WORKSPACE:
-            # Stream-ordered caching allocation: reused, not freed, after the call.
-            need = lib.h3a_attn_fwd_workspace_size(ctypes.byref(args))
-            workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-            args.workspace, args.workspace_bytes = workspace.data_ptr(), need
-            rc = lib.h3a_attn_fwd(ctypes.byref(args), stream)
+    args = (
+        _ext.ABI_VERSION, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), B, H, Sq, Sk, D,
+        *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3], *lse.stride()[:2],
+        scale, 0, cu_q_ptr, cu_k_ptr, segments, longest,
+    )
+    rc = _ext.attn_fwd(device, *args, 0, _ext.H3A_WORKSPACE_ASK if split_tail else 0)
+    if rc == _ext.H3A_NEED_WORKSPACE:
+        # Stream-ordered caching allocation: reused, not freed, after the call.
+        need = _ext.attn_fwd_workspace_size(device, *args, 0, 0)
+        workspace = torch.empty(need, dtype=torch.uint8, device=device)
+        rc = _ext.attn_fwd(device, *args, workspace.data_ptr(), need)
     if rc != _ext.H3A_OK:
-        message = _ext.last_error(lib)
-        if rc == _ext.H3A_EINVAL:
-            raise ValueError(message)
-        raise RuntimeError(message)
+        _ext.check(_ext.load_library(), rc)
     return out, lse
 
 

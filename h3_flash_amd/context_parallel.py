@@ -10,7 +10,6 @@ single-device form of the ring schedule built from it.
 
 from __future__ import annotations
 
-import ctypes
 from typing import Sequence
 
 import torch
@@ -19,14 +18,6 @@ from . import _ext
 from .attention import flash_attn_func
 
 __all__ = ["chunked_attention", "merge_attention"]
-
-
-def _raise(lib: ctypes.CDLL, rc: int) -> None:
-    if rc != _ext.H3A_OK:
-        message = _ext.last_error(lib)
-        if rc == _ext.H3A_EINVAL:
-            raise ValueError(message)
-        raise RuntimeError(message)
 
 
 def _dtype_code(dtype: torch.dtype) -> int:
@@ -124,23 +115,12 @@ def merge_attention(
         lse = torch.empty((B, H, S), dtype=torch.float32, device=ref.device)
     elif lse.shape != (B, H, S) or lse.dtype != torch.float32 or lse.stride(-1) != 1 or lse.device != ref.device:
         raise ValueError(f"lse must be fp32 (B, H, S) on {ref.device} with a contiguous last dim")
-    args = _ext.AttnMergeArgs()
-    args.abi_version = _ext.ABI_VERSION
-    args.n_parts = n
-    for i, (o, l) in enumerate(zip(parts, lparts)):
-        args.o_parts[i] = o.data_ptr()
-        args.lse_parts[i] = l.data_ptr()
-    args.part_dtype = _dtype_code(dtype)
-    args.o, args.out_dtype, args.lse = out.data_ptr(), _dtype_code(out_dtype), lse.data_ptr()
-    args.batch, args.heads, args.seqlen, args.head_dim = B, H, S, D
-    args.part_o_stride[:] = (parts[0].stride(0), parts[0].stride(1), parts[0].stride(2))
-    args.part_lse_stride[:] = (lparts[0].stride(0), lparts[0].stride(1))
-    args.o_stride[:] = (out.stride(0), out.stride(1), out.stride(2))
-    args.lse_stride[:] = (lse.stride(0), lse.stride(1))
-    lib = _ext.load_library()
-    with torch.cuda.device(ref.device):
-        stream = ctypes.c_void_p(torch.cuda.current_stream(ref.device).cuda_stream)
-        _raise(lib, lib.h3a_attn_merge(ctypes.byref(args), stream))
+    unused = (0,) * (_ext.H3A_MERGE_MAX_PARTS - n)
+    _ext.attn_merge.run(
+        ref.device, _ext.ABI_VERSION, n, *[o.data_ptr() for o in parts], *unused, *[l.data_ptr() for l in lparts], *unused,
+        _dtype_code(dtype), out.data_ptr(), _dtype_code(out_dtype), lse.data_ptr(), B, H, S, D,
+        *parts[0].stride()[:3], *lparts[0].stride()[:2], *out.stride()[:3], *lse.stride()[:2],
+    )
     return out, lse
 
 

@@ -16,8 +16,6 @@ bounds there). Every call is one HIP launch on the current stream.
 
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from . import _ext
@@ -29,18 +27,6 @@ __all__ = [
     "fused_rmsnorm_modulate",
     "fused_swiglu",
 ]
-
-
-def _raise(lib: ctypes.CDLL, rc: int) -> None:
-    if rc != _ext.H3A_OK:
-        message = _ext.last_error(lib)
-        if rc == _ext.H3A_EINVAL:
-            raise ValueError(message)
-        raise RuntimeError(message)
-
-
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
 def _rows(x: torch.Tensor, name: str, columns: int) -> torch.Tensor:
@@ -57,7 +43,9 @@ def _rows(x: torch.Tensor, name: str, columns: int) -> torch.Tensor:
 def _vector(t: torch.Tensor, columns: int, device: torch.device, name: str) -> torch.Tensor:
     if t.shape[-1] != columns or t.numel() != columns:
         raise ValueError(f"{name} must have {columns} elements, got shape {tuple(t.shape)}")
-    t = t.reshape(columns).to(device)
+    t = t.reshape(columns)
+    if t.device != device:
+        t = t.to(device)
     if t.dtype not in (torch.bfloat16, torch.float32):
         t = t.float()
     return t if t.is_contiguous() else t.contiguous()
@@ -68,9 +56,9 @@ def _tables(tables: list[torch.Tensor], columns: int, device: torch.device) -> l
     for t in tables:
         if t.dim() != 2 or t.shape[1] != columns:
             raise ValueError(f"modulation tables must be (rows, {columns}), got {tuple(t.shape)}")
-        out.append(t.to(device))
+        out.append(t if t.device == device else t.to(device))
     dtype = torch.bfloat16 if all(t.dtype == torch.bfloat16 for t in out) else torch.float32
-    out = [t.to(dtype) for t in out]
+    out = [t if t.dtype == dtype else t.to(dtype) for t in out]
     # _row_addressable (fusions.py:190-191): the last dimension must be
     # contiguous; broadcast rows (a row stride under the row, e.g. expand())
     # are written out, since the launch takes one row stride per table
@@ -78,7 +66,9 @@ def _tables(tables: list[torch.Tensor], columns: int, device: torch.device) -> l
 
 
 def _index(index: torch.Tensor, device: torch.device) -> torch.Tensor:
-    index = index.reshape(-1).to(device)
+    index = index.reshape(-1)
+    if index.device != device:
+        index = index.to(device)
     if index.numel() == 0:
         raise ValueError("index must not be empty")
     if index.dtype not in (torch.int32, torch.int64):
@@ -86,16 +76,12 @@ def _index(index: torch.Tensor, device: torch.device) -> torch.Tensor:
     return index if index.is_contiguous() else index.contiguous()
 
 
-def _fill_common(args, weight, tables, index, eps) -> None:
-    args.abi_version = _ext.ABI_VERSION
-    args.weight = weight.data_ptr()
-    args.w_dtype = _ext.H3A_DTYPE_F32 if weight.dtype == torch.float32 else _ext.H3A_DTYPE_BF16
-    args.table_dtype = _ext.H3A_DTYPE_F32 if tables[0].dtype == torch.float32 else _ext.H3A_DTYPE_BF16
-    args.table_rows = min(t.shape[0] for t in tables)
-    args.index = index.data_ptr()
-    args.index_dtype = _ext.H3A_DTYPE_I64 if index.dtype == torch.int64 else _ext.H3A_DTYPE_I32
-    args.n_index = index.numel()
-    args.eps = float(eps)
+def _dtype(t: torch.Tensor) -> int:
+    return _ext.H3A_DTYPE_F32 if t.dtype == torch.float32 else _ext.H3A_DTYPE_BF16
+
+
+def _index_args(index: torch.Tensor) -> tuple[int, int, int]:
+    return index.data_ptr(), _ext.H3A_DTYPE_I64 if index.dtype == torch.int64 else _ext.H3A_DTYPE_I32, index.numel()
 
 
 def fused_rmsnorm_modulate(x, weight, scale, shift, index, eps):
@@ -107,17 +93,13 @@ def fused_rmsnorm_modulate(x, weight, scale, shift, index, eps):
     weight = _vector(weight, columns, x.device, "weight")
     scale, shift = _tables([scale, shift], columns, x.device)
     index = _index(index, x.device)
-    output = torch.empty((flat.shape[0], columns), dtype=x.dtype, device=x.device)
-    args = _ext.RmsnormModulateArgs()
-    _fill_common(args, weight, [scale, shift], index, eps)
-    args.x, args.out = flat.data_ptr(), output.data_ptr()
-    args.scale, args.shift = scale.data_ptr(), shift.data_ptr()
-    args.scale_stride, args.shift_stride = scale.stride(0), shift.stride(0)
-    args.rows, args.cols = flat.shape[0], columns
-    args.x_stride, args.out_stride = flat.stride(0), output.stride(0)
-    lib = _ext.load_library()
-    with torch.cuda.device(x.device):
-        _raise(lib, lib.h3a_rmsnorm_modulate(ctypes.byref(args), _stream(x.device)))
+    output = flat.new_empty((flat.shape[0], columns))
+    _ext.rmsnorm_modulate.run(
+        x.device, _ext.ABI_VERSION, flat.data_ptr(), output.data_ptr(), weight.data_ptr(), _dtype(weight),
+        scale.data_ptr(), shift.data_ptr(), _dtype(scale), scale.stride(0), shift.stride(0),
+        min(scale.shape[0], shift.shape[0]), *_index_args(index), flat.shape[0], columns,
+        flat.stride(0), output.stride(0), float(eps),
+    )
     return output.view(x.shape)
 
 
@@ -135,20 +117,15 @@ def fused_residual_gate_rmsnorm_modulate(residual, branch, gate, weight, scale, 
     weight = _vector(weight, columns, residual.device, "weight")
     gate, scale, shift = _tables([gate, scale, shift], columns, residual.device)
     index = _index(index, residual.device)
-    hidden = torch.empty((residual_flat.shape[0], columns), dtype=residual.dtype, device=residual.device)
-    normed = torch.empty_like(hidden)
-    args = _ext.ResidualGateRmsnormModulateArgs()
-    _fill_common(args, weight, [gate, scale, shift], index, eps)
-    args.residual, args.branch = residual_flat.data_ptr(), branch_flat.data_ptr()
-    args.hidden_out, args.normed_out = hidden.data_ptr(), normed.data_ptr()
-    args.gate, args.scale, args.shift = gate.data_ptr(), scale.data_ptr(), shift.data_ptr()
-    args.gate_stride, args.scale_stride, args.shift_stride = gate.stride(0), scale.stride(0), shift.stride(0)
-    args.rows, args.cols = residual_flat.shape[0], columns
-    args.residual_stride, args.branch_stride = residual_flat.stride(0), branch_flat.stride(0)
-    args.hidden_stride, args.normed_stride = hidden.stride(0), normed.stride(0)
-    lib = _ext.load_library()
-    with torch.cuda.device(residual.device):
-        _raise(lib, lib.h3a_residual_gate_rmsnorm_modulate(ctypes.byref(args), _stream(residual.device)))
+    rows = residual_flat.shape[0]
+    hidden, normed = residual_flat.new_empty((rows, columns)), residual_flat.new_empty((rows, columns))
+    _ext.residual_gate_rmsnorm_modulate.run(
+        residual.device, _ext.ABI_VERSION, residual_flat.data_ptr(), branch_flat.data_ptr(), hidden.data_ptr(),
+        normed.data_ptr(), weight.data_ptr(), _dtype(weight), gate.data_ptr(), scale.data_ptr(), shift.data_ptr(),
+        _dtype(gate), gate.stride(0), scale.stride(0), shift.stride(0),
+        min(gate.shape[0], scale.shape[0], shift.shape[0]), *_index_args(index), residual_flat.shape[0], columns,
+        residual_flat.stride(0), branch_flat.stride(0), hidden.stride(0), normed.stride(0), float(eps),
+    )
     return hidden.view(residual.shape), normed.view(residual.shape)
 
 
@@ -159,13 +136,9 @@ def fused_swiglu(x):
         raise ValueError(f"swiglu needs an even last dimension, got {x.shape[-1]}")
     columns = x.shape[-1] // 2
     flat = _rows(x, "x", x.shape[-1])
-    output = torch.empty((flat.shape[0], columns), dtype=x.dtype, device=x.device)
-    args = _ext.SwigluArgs()
-    args.abi_version = _ext.ABI_VERSION
-    args.x, args.out = flat.data_ptr(), output.data_ptr()
-    args.rows, args.cols = flat.shape[0], columns
-    args.x_stride, args.out_stride = flat.stride(0), output.stride(0)
-    lib = _ext.load_library()
-    with torch.cuda.device(x.device):
-        _raise(lib, lib.h3a_swiglu(ctypes.byref(args), _stream(x.device)))
+    output = flat.new_empty((flat.shape[0], columns))
+    _ext.swiglu.run(
+        x.device, _ext.ABI_VERSION, flat.data_ptr(), output.data_ptr(), flat.shape[0], columns,
+        flat.stride(0), output.stride(0),
+    )
     return output.view(*x.shape[:-1], columns)

@@ -28,7 +28,6 @@ return ``None``, with the reason, so the caller keeps the unfused path.
 
 from __future__ import annotations
 
-import ctypes
 import weakref
 from typing import Any
 
@@ -79,38 +78,24 @@ def proj_gemm(
 
     if not 1 <= len(sections) <= _ext.H3A_PROJ_MAX_SECTIONS:
         raise ValueError(f"1 to {_ext.H3A_PROJ_MAX_SECTIONS} sections, got {len(sections)}")
-    args = _ext.ProjArgs()
-    args.abi_version = _ext.ABI_VERSION
-    args.x = x.data_ptr()
-    args.x_stride = x.stride(0)
-    args.m, args.k = x.shape
-    args.head_dim = HEAD_DIM
-    args.num_sections = len(sections)
-    for i, s in enumerate(sections):
-        d = args.sections[i]
-        d.weight = s.weight.data_ptr()
-        d.weight_stride = s.weight.stride(0)
-        d.n = s.weight.shape[0]
-        d.bias = s.bias.data_ptr() if s.bias is not None else None
-        d.y = s.y.data_ptr()
-        d.y_stride = s.y.stride(0)
-        d.mode = _ext.H3A_PROJ_QKNORM_ROPE if s.norm_weight is not None else _ext.H3A_PROJ_PLAIN
-        d.norm_weight = s.norm_weight.data_ptr() if s.norm_weight is not None else None
-        d.eps = s.eps
+    flat = []
+    for s in sections:
+        nw = s.norm_weight
+        flat += (
+            s.weight.data_ptr(), s.weight.stride(0), s.weight.shape[0], 0 if s.bias is None else s.bias.data_ptr(),
+            s.y.data_ptr(), s.y.stride(0), _ext.H3A_PROJ_PLAIN if nw is None else _ext.H3A_PROJ_QKNORM_ROPE,
+            0 if nw is None else nw.data_ptr(), s.eps,
+        )
+    for _ in range(_ext.H3A_PROJ_MAX_SECTIONS - len(sections)):
+        flat += (0, 0, 0, 0, 0, 0, 0, 0, 0.0)
+    tables = (0, 0, 0, 0, 0, 0)
     if cos is not None:
-        args.cos, args.sin = cos.data_ptr(), sin.data_ptr()
-        args.table_stride = cos.stride(0)
-        args.rotary_dim = cos.shape[-1]
-        args.seqlen = seqlen if seqlen is not None else cos.shape[0]
-        args.rotate_half_tables = 1 if rotate_half else 0
-    lib = _ext.load_library()
-    stream = torch.cuda.current_stream(x.device).cuda_stream
-    rc = lib.h3a_proj_gemm(ctypes.byref(args), ctypes.c_void_p(stream))
-    if rc != _ext.H3A_OK:
-        message = _ext.last_error(lib)
-        if rc == _ext.H3A_EINVAL:
-            raise ValueError(message)
-        raise RuntimeError(message)
+        tables = (cos.data_ptr(), sin.data_ptr(), cos.stride(0), cos.shape[-1],
+                  seqlen if seqlen is not None else cos.shape[0], 1 if rotate_half else 0)
+    m, k = x.shape
+    _ext.proj_gemm.run(
+        x.device, _ext.ABI_VERSION, x.data_ptr(), x.stride(0), m, k, HEAD_DIM, len(sections), *flat, *tables
+    )
 
 
 # Attribute under which a cos table object remembers its last check: (a weak
@@ -196,8 +181,8 @@ def qkv_projection(
             return no("to_qkv is not a bf16 linear with 16-byte aligned rows")
         w, b = parts
         n = w.shape[0] // 3
-        weights = (w[:n], w[n : 2 * n], w[2 * n :])
-        biases = (None, None, None) if b is None else (b[:n], b[n : 2 * n], b[2 * n :])
+        weights = w.split((n, n, w.shape[0] - 2 * n))
+        biases = (None, None, None) if b is None else b.split((n, n, b.shape[0] - 2 * n))
     else:
         ps = [_linear_parts(m) for m in (attn.to_q, attn.to_k, attn.to_v)]
         if any(q is None for q in ps):
@@ -219,21 +204,22 @@ def qkv_projection(
     # Checked on the caller's own table objects (the conversions below may
     # make fresh temporaries); a dtype or layout change keeps the form.
     half_form = rotate_half_tables(cos, sin) if R % 32 == 0 and R > 0 else False
-    cos = cos.to(device=x.device, dtype=torch.float32)
-    sin = sin.to(device=x.device, dtype=torch.float32)
+    if cos.dtype != torch.float32 or cos.device != x.device:
+        cos = cos.to(device=x.device, dtype=torch.float32)
+    if sin.dtype != torch.float32 or sin.device != x.device:
+        sin = sin.to(device=x.device, dtype=torch.float32)
     if not (cos.is_contiguous() and sin.is_contiguous()):
         cos, sin = cos.contiguous(), sin.contiguous()
-    wq_n, wk_n = (t.to(x.device) for t in (wq_n, wk_n))
-    out = torch.empty((B, S, 3 * n), dtype=torch.bfloat16, device=x.device)
-    y = out.view(B * S, 3 * n)
+    wq_n, wk_n = (t if t.device == x.device else t.to(x.device) for t in (wq_n, wk_n))
+    out = x.new_empty((B, S, 3 * n))
+    ys = out.view(B * S, 3 * n).split(n, 1)
     sections = [
-        Section(weights[0], y[:, :n], biases[0], wq_n, nq.eps),
-        Section(weights[1], y[:, n : 2 * n], biases[1], wk_n, nk.eps),
-        Section(weights[2], y[:, 2 * n :], biases[2]),
+        Section(weights[0], ys[0], biases[0], wq_n, nq.eps),
+        Section(weights[1], ys[1], biases[1], wk_n, nk.eps),
+        Section(weights[2], ys[2], biases[2]),
     ]
     proj_gemm(x.view(B * S, hidden), sections, cos, sin, S, rotate_half=half_form)
-    q, k, v = out.chunk(3, dim=-1)
-    return q.unflatten(-1, (H, HEAD_DIM)), k.unflatten(-1, (H, HEAD_DIM)), v.unflatten(-1, (H, HEAD_DIM))
+    return out.view(B, S, 3, H, HEAD_DIM).unbind(2)
 
 
 def out_projection(linear: Any, x: torch.Tensor) -> torch.Tensor | None:

@@ -10,8 +10,6 @@ calls it: the reference issues one launch per tensor
 
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from . import _ext
@@ -32,10 +30,10 @@ def _operand(x: torch.Tensor, name: str) -> torch.Tensor:
         raise ValueError(f"{name} must be 4-D (batch, seq, heads, head_dim), got {tuple(x.shape)}")
     if x.dtype != torch.bfloat16:
         raise TypeError(f"{name} must be bfloat16, got {x.dtype}")
-    if x.device.type != "cuda":
+    if not x.is_cuda:
         raise RuntimeError(f"{name} must be on a ROCm device, got {x.device}")
-    ok = x.stride(-1) == 1 and all(s % 8 == 0 for s in x.stride()[:3]) and x.data_ptr() % 16 == 0
-    return x if ok else x.contiguous()
+    b, s, h, d = x.stride()
+    return x if d == 1 and not (b | s | h) & 7 and not x.data_ptr() & 15 else x.contiguous()
 
 
 def _weight(w: torch.Tensor, head_dim: int, device: torch.device) -> torch.Tensor:
@@ -43,14 +41,16 @@ def _weight(w: torch.Tensor, head_dim: int, device: torch.device) -> torch.Tenso
         raise ValueError(f"norm weight must have shape ({head_dim},), got {tuple(w.shape)}")
     if w.dtype not in (torch.bfloat16, torch.float32):
         w = w.float()
-    w = w.to(device)
+    if w.device != device:
+        w = w.to(device)
     return w if (w.is_contiguous() and w.data_ptr() % 16 == 0) else w.contiguous().clone()
 
 
 def _table(t: torch.Tensor, seqlen: int, device: torch.device) -> torch.Tensor:
     if t.dim() != 2 or t.shape[0] != seqlen:
         raise ValueError(f"cos/sin tables must be (seq={seqlen}, rotary_dim), got {tuple(t.shape)}")
-    t = t.to(device=device, dtype=torch.float32)
+    if t.dtype != torch.float32 or t.device != device:
+        t = t.to(device=device, dtype=torch.float32)
     # broadcast rows (a row stride under the row, e.g. expand()) are written
     # out: the launch reads row s at s * table_stride with table_stride >= R
     return t if t.stride(-1) == 1 and t.stride(0) >= t.shape[-1] else t.contiguous()
@@ -67,29 +67,16 @@ def _tables(cos: torch.Tensor, sin: torch.Tensor, seqlen: int, device: torch.dev
 
 def _launch(q, k, wq, wk, cos, sin, eps_q, eps_k, out_q, out_k) -> None:
     B, S, H, D = q.shape
-    R = cos.shape[-1]
-    args = _ext.QkNormRopeArgs()
-    args.abi_version = _ext.ABI_VERSION
-    args.xq, args.yq, args.wq = q.data_ptr(), out_q.data_ptr(), wq.data_ptr()
-    if k is not None:
-        args.xk, args.yk, args.wk = k.data_ptr(), out_k.data_ptr(), wk.data_ptr()
-        args.xk_stride[:] = k.stride()[:3]
-        args.yk_stride[:] = out_k.stride()[:3]
-    args.w_dtype = _ext.H3A_DTYPE_F32 if wq.dtype == torch.float32 else _ext.H3A_DTYPE_BF16
-    args.cos, args.sin = cos.data_ptr(), sin.data_ptr()
-    args.table_stride = cos.stride(0)
-    args.batch, args.seqlen, args.heads, args.head_dim, args.rotary_dim = B, S, H, D, R
-    args.xq_stride[:] = q.stride()[:3]
-    args.yq_stride[:] = out_q.stride()[:3]
-    args.eps_q, args.eps_k = float(eps_q), float(eps_k)
-    lib = _ext.load_library()
-    stream = torch.cuda.current_stream(q.device).cuda_stream
-    rc = lib.h3a_qknorm_rope(ctypes.byref(args), ctypes.c_void_p(stream))
-    if rc != _ext.H3A_OK:
-        message = _ext.last_error(lib)
-        if rc == _ext.H3A_EINVAL:
-            raise ValueError(message)
-        raise RuntimeError(message)
+    second = (0, 0, 0) if k is None else (k.data_ptr(), out_k.data_ptr(), wk.data_ptr())
+    none = (0, 0, 0)
+    _ext.qknorm_rope.run(
+        q.device, _ext.ABI_VERSION, q.data_ptr(), second[0], out_q.data_ptr(), second[1], wq.data_ptr(), second[2],
+        _ext.H3A_DTYPE_F32 if wq.dtype == torch.float32 else _ext.H3A_DTYPE_BF16,
+        cos.data_ptr(), sin.data_ptr(), cos.stride(0), B, S, H, D, cos.shape[-1],
+        *q.stride()[:3], *(none if k is None else k.stride()[:3]),
+        *out_q.stride()[:3], *(none if k is None else out_k.stride()[:3]),
+        float(eps_q), float(eps_k),
+    )
 
 
 def fused_qknorm_rope(
@@ -138,7 +125,6 @@ def fused_qk_norm_rope(
     if wq.dtype != wk.dtype:
         wq, wk = wq.float(), wk.float()
     cos, sin = _tables(cos, sin, S, q.device)
-    out_q = torch.empty((B, S, H, D), dtype=q.dtype, device=q.device)
-    out_k = torch.empty((B, S, H, D), dtype=k.dtype, device=k.device)
+    out_q, out_k = q.new_empty((B, S, H, D)), k.new_empty((B, S, H, D))
     _launch(q, k, wq, wk, cos, sin, eps_q, eps_k, out_q, out_k)
     return out_q, out_k

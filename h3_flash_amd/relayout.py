@@ -25,8 +25,6 @@ The collectives themselves are not part of this single-GPU build.
 
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from . import _ext
@@ -40,18 +38,6 @@ __all__ = [
     "packed_qkv_attention",
     "qknorm_rope_pack_qkv",
 ]
-
-
-def _raise(lib: ctypes.CDLL, rc: int) -> None:
-    if rc != _ext.H3A_OK:
-        message = _ext.last_error(lib)
-        if rc == _ext.H3A_EINVAL:
-            raise ValueError(message)
-        raise RuntimeError(message)
-
-
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
 def can_pack_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
@@ -90,17 +76,10 @@ def pack_qkv_destination_major(
     out = torch.empty((world, rows, heads_local, 3 * head_dim), dtype=q.dtype, device=q.device)
     if out.numel() == 0:
         return out
-    args = _ext.PackQkvArgs()
-    args.abi_version = _ext.ABI_VERSION
-    args.q, args.k, args.v, args.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
-    args.elem_bytes = q.element_size()
-    args.rows, args.heads, args.head_dim, args.world = rows, heads, head_dim, world
-    args.q_stride[:] = q.stride()[:2]
-    args.k_stride[:] = k.stride()[:2]
-    args.v_stride[:] = v.stride()[:2]
-    lib = _ext.load_library()
-    with torch.cuda.device(q.device):
-        _raise(lib, lib.h3a_pack_qkv(ctypes.byref(args), _stream(q.device)))
+    _ext.pack_qkv.run(
+        q.device, _ext.ABI_VERSION, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), q.element_size(),
+        rows, heads, head_dim, world, *q.stride()[:2], *k.stride()[:2], *v.stride()[:2],
+    )
     return out
 
 
@@ -116,18 +95,12 @@ def merge_heads(x: torch.Tensor) -> torch.Tensor:
     inner = heads_local * head_dim
     if x.stride(3) != 1 or (heads_local > 1 and x.stride(2) != head_dim):
         x = x.contiguous()  # the (heads_local, head_dim) block must be contiguous
-    out = torch.empty((rows, world, heads_local, head_dim), dtype=x.dtype, device=x.device)
+    out = x.new_empty((rows, world, heads_local, head_dim))
     if out.numel() == 0:
         return out.reshape(rows, world * heads_local, head_dim)
-    args = _ext.MergeHeadsArgs()
-    args.abi_version = _ext.ABI_VERSION
-    args.x, args.out = x.data_ptr(), out.data_ptr()
-    args.elem_bytes = x.element_size()
-    args.world, args.rows, args.inner = world, rows, inner
-    args.x_stride[:] = (x.stride(0), x.stride(1))
-    lib = _ext.load_library()
-    with torch.cuda.device(x.device):
-        _raise(lib, lib.h3a_merge_heads(ctypes.byref(args), _stream(x.device)))
+    _ext.merge_heads.run(
+        x.device, _ext.ABI_VERSION, x.data_ptr(), out.data_ptr(), x.element_size(), world, rows, inner, *x.stride()[:2]
+    )
     return out.reshape(rows, world * heads_local, head_dim)
 
 
@@ -138,8 +111,8 @@ def _rows_operand(x: torch.Tensor, name: str) -> torch.Tensor:
         raise TypeError(f"{name} must be bfloat16, got {x.dtype}")
     if not x.is_cuda:
         raise RuntimeError(f"{name} must be on a ROCm device, got {x.device}")
-    ok = x.stride(-1) == 1 and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0 and x.data_ptr() % 16 == 0
-    return x if ok else x.contiguous()
+    r, h, d = x.stride()
+    return x if d == 1 and not (r | h) & 7 and not x.data_ptr() & 15 else x.contiguous()
 
 
 def qknorm_rope_pack_qkv(
@@ -179,23 +152,15 @@ def qknorm_rope_pack_qkv(
     if wq.dtype != wk.dtype:
         wq, wk = wq.float(), wk.float()
     cos, sin = _tables(cos, sin, rows, q.device)
-    out = torch.empty((world, rows, heads // world, 3 * head_dim), dtype=q.dtype, device=q.device)
+    out = q.new_empty((world, rows, heads // world, 3 * head_dim))
     if out.numel() == 0:
         return out
-    args = _ext.QkNormRopePackArgs()
-    args.abi_version = _ext.ABI_VERSION
-    args.q, args.k, args.v, args.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
-    args.wq, args.wk = wq.data_ptr(), wk.data_ptr()
-    args.w_dtype = _ext.H3A_DTYPE_F32 if wq.dtype == torch.float32 else _ext.H3A_DTYPE_BF16
-    args.cos, args.sin, args.table_stride = cos.data_ptr(), sin.data_ptr(), cos.stride(0)
-    args.rows, args.heads, args.head_dim, args.rotary_dim, args.world = rows, heads, head_dim, R, world
-    args.q_stride[:] = q.stride()[:2]
-    args.k_stride[:] = k.stride()[:2]
-    args.v_stride[:] = v.stride()[:2]
-    args.eps_q, args.eps_k = float(eps_q), float(eps_k)
-    lib = _ext.load_library()
-    with torch.cuda.device(q.device):
-        _raise(lib, lib.h3a_qknorm_rope_pack(ctypes.byref(args), _stream(q.device)))
+    _ext.qknorm_rope_pack.run(
+        q.device, _ext.ABI_VERSION, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), wq.data_ptr(), wk.data_ptr(),
+        _ext.H3A_DTYPE_F32 if wq.dtype == torch.float32 else _ext.H3A_DTYPE_BF16,
+        cos.data_ptr(), sin.data_ptr(), cos.stride(0), rows, heads, head_dim, R, world,
+        *q.stride()[:2], *k.stride()[:2], *v.stride()[:2], float(eps_q), float(eps_k),
+    )
     return out
 
 

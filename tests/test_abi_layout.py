@@ -60,3 +60,35 @@ def test_ctypes_structure_matches_the_header(c_layout, cname):
     assert ctypes.sizeof(cls) == want["size"], (cname, ctypes.sizeof(cls), want["size"])
     for field, _ in cls._fields_:
         assert getattr(cls, field).offset == want[field], (cname, field)
+
+
+# The packed form of every entry point's arguments: each member at its ctypes
+# offset, and values beyond a member's range as C would convert them.
+@pytest.mark.parametrize(
+    "launch, ctype",
+    [(_ext.attn_fwd, _ext.AttnArgs), (_ext.qknorm_rope, _ext.QkNormRopeArgs), (_ext.pack_qkv, _ext.PackQkvArgs),
+     (_ext.merge_heads, _ext.MergeHeadsArgs), (_ext.qknorm_rope_pack, _ext.QkNormRopePackArgs),
+     (_ext.rmsnorm_modulate, _ext.RmsnormModulateArgs),
+     (_ext.residual_gate_rmsnorm_modulate, _ext.ResidualGateRmsnormModulateArgs), (_ext.swiglu, _ext.SwigluArgs),
+     (_ext.attn_merge, _ext.AttnMergeArgs), (_ext.proj_gemm, _ext.ProjArgs)],
+)
+def test_packed_arguments_match_the_structure(launch, ctype):
+    def members(obj):
+        for name, t in obj._fields_:
+            v = getattr(obj, name)
+            if hasattr(t, "_fields_"):
+                yield from members(v)
+            elif hasattr(t, "_length_"):
+                for x in v:
+                    if hasattr(x, "_fields_"):
+                        yield from members(x)
+                    else:
+                        yield x or 0
+            else:
+                yield v or 0
+
+    raw = bytes((37 * i + 11) % 120 + 1 for i in range(ctypes.sizeof(ctype)))
+    args = ctype.from_buffer_copy(raw)
+    packed = launch._pack(*members(args))
+    assert len(packed) == ctypes.sizeof(ctype)
+    assert list(members(ctype.from_buffer_copy(packed))) == list(members(args))
