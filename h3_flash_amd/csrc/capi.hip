@@ -32,23 +32,38 @@ constexpr int64_t kVtMinKeys = 16384;
 // round) pays for its planning launch with segments of this many rows.
 constexpr int64_t kPlanMinSegment = 4096;
 
-// Shorter segments run on the persistent launch, unless their lengths vary
-// and there are few tiles per CU: its last tiles (up to max_seqlen_q / 64
-// key tiles each, claimed in segment order) then leave CUs idle, and each
-// tile past a shorter segment's rows costs a claim. The planned list (no
-// such tiles, longest segments first, the last round as key-range pieces)
-// balances them. Equal lengths and many rounds keep the persistent launch
-// (its next-tile loads). Timed on 47 mixes of H5 segments of 1 to 4,095
-// rows, this rule picked the faster launch for all but three, each within
-// 4% of it. The host knows only the packed rows, the segment count and the
-// longest segment, so "varied" is the longest against the mean.
-bool short_segments_planned(const h3a_attn_args* a, int cus) {
-    if (a->num_segments <= 0 || a->seqlen_q <= 0 || cus <= 0) return false;
+// Shorter segments run on the persistent launch (varied lengths claimed by
+// length, longest first), unless the planned list, whose last round is cut into
+// key-range pieces, balances the CUs better than it costs (its planning and
+// merge launches, about 15 us): with long segments and about one to four
+// rounds, where the last tiles are a large part of the time. Timed on 38 mixes
+// of 1 to 4,095 rows at 1 to 8 heads (us, persistent / planned): 48 segments up
+// to 2,048 rows, 3.8 rounds 214 / 207; 12 up to 2,598, 1.4 rounds 123 / 113; 12
+// up to 3,540, 2.9 rounds 278 / 258; but 48 up to 705, 2.6 rounds 80 / 96; 11 up
+// to 2,063, 1.6 rounds 117 / 123; 14 up to 3,233, 0.4 rounds 71 / 89; 47 up to
+// 2,500, 7.1 rounds 428 / 439. The host knows only the packed rows, the segment
+// count and the longest segment, so "varied" is the longest against the mean.
+struct ShortMix {
+    bool varied;
+    double rounds;
+};
+ShortMix short_mix(const h3a_attn_args* a, int cus) {
+    if (a->num_segments <= 0 || a->seqlen_q <= 0 || cus <= 0) return ShortMix{false, 0.0};
     const double mean = (double)a->seqlen_q / (double)a->num_segments;
     const double rounds =
         (double)a->heads * ((double)a->seqlen_q / h3a::attn_fwd_block_m() + a->num_segments / 2.0) / cus;
-    const bool varied = a->max_seqlen_q >= 1.6 * mean;
-    return varied && (rounds <= 3.2 || (a->max_seqlen_q >= 2900 && rounds <= 9.0));
+    return ShortMix{a->max_seqlen_q >= 1.6 * mean, rounds};
+}
+bool short_segments_planned(const h3a_attn_args* a, int cus) {
+    const ShortMix m = short_mix(a, cus);
+    return m.varied && a->max_seqlen_q >= 1900 && m.rounds >= 1.0 &&
+           (m.rounds <= 4.0 || (a->max_seqlen_q >= 2900 && m.rounds <= 9.0));
+}
+// Varied mixes of few rounds whose workspace has room for the planned list,
+// whichever launch they take.
+bool short_segments_plannable(const h3a_attn_args* a, int cus) {
+    const ShortMix m = short_mix(a, cus);
+    return m.varied && (m.rounds <= 3.2 || (a->max_seqlen_q >= 2900 && m.rounds <= 9.0));
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -231,7 +246,7 @@ struct AttnWorkspace {
 };
 
 AttnWorkspace attn_workspace(const h3a_attn_args* a, const h3a::AttnParams& p, bool allow_vt,
-                             int64_t max_workspace = INT64_MAX) {
+                             int64_t max_workspace = INT64_MAX, bool plannable = false) {
     if (p.n_units > 0) return AttnWorkspace{};
     AttnWorkspace w{attn_plan(a, p, max_workspace), 0, 0, 0, 0, 0, 0, false};
     w.total = w.plan.workspace_bytes;
@@ -244,7 +259,8 @@ AttnWorkspace attn_workspace(const h3a_attn_args* a, const h3a::AttnParams& p, b
         // the planning launch (max_seqlen_q bounds them).
         const int cus = device_cus();
         if (!allow_vt || cus <= 0) return w;
-        if (a->max_seqlen_q < kPlanMinSegment && !short_segments_planned(a, cus)) {
+        if (a->max_seqlen_q < kPlanMinSegment && !short_segments_planned(a, cus) &&
+            !(plannable && short_segments_plannable(a, cus))) {
             // Short segments: the persistent launch's tile counter.
             if (a->max_seqlen_q <= h3a::attn_fwd_persist_max_rows() && w.total + 256 <= max_workspace) {
                 w.persist = true;
@@ -283,6 +299,14 @@ AttnWorkspace attn_workspace(const h3a_attn_args* a, const h3a::AttnParams& p, b
     w.vt_rs = vt_rs;
     w.total = offset + bytes;
     return w;
+}
+
+// Points a packed launch of short segments at its tile counter.
+void apply_persist(const h3a_attn_args* a, h3a::AttnParams& p, void* counter, int cus) {
+    p.persist_queue = (int*)counter;
+    p.persist_blocks = cus;
+    p.persist_sort = a->num_segments <= h3a::attn_fwd_persist_max_segments() &&
+                     (double)a->max_seqlen_q * a->num_segments >= 1.2 * (double)a->seqlen_q;
 }
 
 // Points the launch at a workspace for the plan's split tiles.
@@ -378,10 +402,7 @@ int h3a_attn_fwd(const h3a_attn_args* a, void* stream) {
     if (ask && w.total > 0) return H3A_NEED_WORKSPACE;
     if (w.total > 0 && a->workspace != nullptr && a->workspace_bytes >= w.total && ((uintptr_t)a->workspace & 255u) == 0) {
         if (w.plan.split_n != 0) apply_plan(p, w.plan, a->workspace);
-        if (w.persist) {
-            p.persist_queue = (int*)a->workspace;
-            p.persist_blocks = w.cus;
-        }
+        if (w.persist) apply_persist(a, p, a->workspace, w.cus);
         if (w.ub_tiles > 0) {
             const int64_t pieces = (int64_t)h3a::attn_fwd_tail_pieces() * w.cus;
             p.ws_o = (uint16_t*)a->workspace;
@@ -438,10 +459,7 @@ int h3a_attn_fwd_noalloc(const h3a_attn_args* a, void* stream) {
     // results would not fit, so varied lengths take this launch too.
     if (plan.split_n == 0 && a->cu_seqlens_q != nullptr && a->max_seqlen_q <= h3a::attn_fwd_persist_max_rows()) {
         const int cus = device_cus();
-        if (cus > 0) {
-            p.persist_queue = (int*)scratch;
-            p.persist_blocks = cus;
-        }
+        if (cus > 0) apply_persist(a, p, scratch, cus);
     }
     e = h3a::launch_attn_fwd(p, (hipStream_t)stream);
     if (e != hipSuccess) return fail(H3A_ELAUNCH, "h3a_attn_fwd_noalloc: launch failed: %s", hipGetErrorString(e));
@@ -457,7 +475,7 @@ int64_t h3a_attn_fwd_workspace_size(const h3a_attn_args* a) {
     if (empty) return 0;
     // What all tiles would take (a launch that runs as units leaves it unused),
     // or the whole tiles alone beside their ragged rows' units.
-    const int64_t tiles = attn_workspace(a, p, true).total;
+    const int64_t tiles = attn_workspace(a, p, true, INT64_MAX, true).total;
     take_rag_units(a, p);
     const int64_t whole = attn_workspace(a, p, true).total;
     return tiles > whole ? tiles : whole;

@@ -76,6 +76,8 @@ struct AttnParams {
     // workgroup per tile.
     int* persist_queue;
     int32_t persist_blocks;
+    // 1: a persistent launch claims its tiles by segment length, longest first.
+    int32_t persist_sort;
     // Units of 32 query rows per (group, head) when the launch runs them in
     // place of tiles (short attention), else 0.
     int32_t n_units;
@@ -108,6 +110,7 @@ int attn_rag_blocks(int64_t tiles, int64_t units, int64_t keys, int cus);
 int attn_fwd_unit_rows();  // query rows of a unit of a short launch
 int attn_fwd_block_m();
 // Longest segment (max_seqlen_q) of a persistent packed launch.
+int attn_fwd_persist_max_segments();  // most segments a persistent launch orders by length
 int attn_fwd_persist_max_rows();
 // Most key-range pieces per tile of a tail, and the workspace bytes of one
 // piece's fp32 partial O and LSE.

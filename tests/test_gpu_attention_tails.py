@@ -94,3 +94,26 @@ def test_last_round_pieces_of_short_key_ranges(H, Sq, Sk):
     h = [0, H - 1]
     ref_out, ref_lse = sdpa_reference(q[:, :, h], k[:, :, h], v[:, :, h])
     assert_parity(out.cpu()[:, :, h], lse.cpu()[:, h], ref_out, ref_lse, f"{H}x{Sq}x{Sk}")
+
+
+# Persistent launches that order their segments by key length: more segments
+# than a wave has lanes, empty ones first, last and in between, equal lengths,
+# query and key lengths in different orders, and fewer tiles than CUs.
+@pytest.mark.parametrize(
+    "qlens, klens, H",
+    [([0, 300, 0, 257, 700, 1, 0], None, 40), ([700 - 7 * i if i % 3 else 0 for i in range(90)], None, 2),
+     ([256, 1000, 40, 600], [900, 64, 700, 1], 50), ([40] * 130 + [600] * 3, None, 3)],
+)
+def test_persistent_order_by_length(qlens, klens, H):
+    klens = qlens if klens is None else klens
+    q, k, v = _qkv(1, sum(qlens), sum(klens), H, sum(klens))
+    cq, ck = (torch.tensor([0, *torch.tensor(x).cumsum(0).tolist()], dtype=torch.int32, device=DEV) for x in (qlens, klens))
+    kw = dict(cu_seqlens_q=cq, cu_seqlens_k=ck, max_seqlen_q=max(qlens))
+    got = flash_attn_func(q.to(DEV), k.to(DEV), v.to(DEV), **kw)
+    whole = flash_attn_func(q.to(DEV), k.to(DEV), v.to(DEV), split_tail=False, **kw)
+    torch.cuda.synchronize()
+    assert_parity(got[0].cpu(), got[1].cpu(), whole[0].float().cpu(), whole[1].cpu(), "whole tiles")
+    a, b = qlens[0] + qlens[1], klens[0] + klens[1]
+    rows, keys = slice(qlens[0], a), slice(klens[0], b)
+    ref_out, ref_lse = sdpa_reference(q[:, rows, :2], k[:, keys, :2], v[:, keys, :2])
+    assert_parity(got[0][:, rows, :2].cpu(), got[1][:, :2, rows].cpu(), ref_out, ref_lse, "second segment")
