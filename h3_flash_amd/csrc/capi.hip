@@ -34,15 +34,16 @@ constexpr int64_t kPlanMinSegment = 4096;
 
 // Shorter segments run on the persistent launch (varied lengths claimed by
 // length, longest first), unless the planned list, whose last round is cut into
-// key-range pieces, balances the CUs better than it costs (its planning and
-// merge launches, about 15 us): with long segments and about one to four
-// rounds, where the last tiles are a large part of the time. Timed on 38 mixes
-// of 1 to 4,095 rows at 1 to 8 heads (us, persistent / planned): 48 segments up
-// to 2,048 rows, 3.8 rounds 214 / 207; 12 up to 2,598, 1.4 rounds 123 / 113; 12
-// up to 3,540, 2.9 rounds 278 / 258; but 48 up to 705, 2.6 rounds 80 / 96; 11 up
-// to 2,063, 1.6 rounds 117 / 123; 14 up to 3,233, 0.4 rounds 71 / 89; 47 up to
-// 2,500, 7.1 rounds 428 / 439. The host knows only the packed rows, the segment
-// count and the longest segment, so "varied" is the longest against the mean.
+// key-range pieces, balances the CUs better than its planning and merge
+// launches cost (about 12 us): with varied lengths from about one round on.
+// Timed on 50 mixes of 1 to 4,095 rows at 1 to 8 heads (us, persistent /
+// planned): 48 segments up to 2,048 rows, 3.8 rounds 205 / 190; 16 up to 1,916,
+// 1.2 rounds 87 / 73; 24 up to 567, 1.05 rounds 44 / 37; 42 up to 1,056, 3.3
+// rounds 122 / 110; 39 up to 2,130, 4.9 rounds 262 / 250; but 14 up to 3,233,
+// 0.4 rounds 69 / 84; 12 up to 984, 0.85 rounds 37 / 45; equal lengths, 48 of
+// 1,024 145 / 158; past five rounds the two are level. The host knows only the
+// packed rows, the segment count and the longest segment, so "varied" is the
+// longest against the mean.
 struct ShortMix {
     bool varied;
     double rounds;
@@ -56,8 +57,7 @@ ShortMix short_mix(const h3a_attn_args* a, int cus) {
 }
 bool short_segments_planned(const h3a_attn_args* a, int cus) {
     const ShortMix m = short_mix(a, cus);
-    return m.varied && a->max_seqlen_q >= 1900 && m.rounds >= 1.0 &&
-           (m.rounds <= 4.0 || (a->max_seqlen_q >= 2900 && m.rounds <= 9.0));
+    return m.varied && m.rounds >= 1.0 && (m.rounds <= 5.0 || (a->max_seqlen_q >= 2900 && m.rounds <= 9.0));
 }
 // Varied mixes of few rounds whose workspace has room for the planned list,
 // whichever launch they take.

@@ -131,11 +131,10 @@ extern "C" {
  *     the counter is zeroed by a small kernel first). Results are
  *     bit-identical to one workgroup per tile, whatever the order. When the
  *     segment lengths vary (max_seqlen_q at least 1.6 times seqlen_q /
- *     num_segments) and the last tiles are a large part of the time
- *     (max_seqlen_q of 1,900 or more, and heads x (seqlen_q / 256 +
- *     num_segments / 2) one to four per CU, or up to 9 with max_seqlen_q of
- *     2,900 or more), such calls take the planned work list above instead; the
- *     size has room for it wherever lengths vary and tiles per CU are few.
+ *     num_segments) over one to five rounds of tiles (heads x (seqlen_q / 256
+ *     + num_segments / 2) per CU; up to nine with max_seqlen_q of 2,900 or
+ *     more), such calls take the planned work list above instead; the size has
+ *     room for it also where lengths vary over less than a round.
  * With a workspace given, short attention (up to about 256 units of 32 query
  * rows of one head and 2,048 keys, or more units over fewer keys) runs without
  * using it, as one workgroup per unit with the keys split over its waves; so
