@@ -49,6 +49,10 @@ __all__ = [
 HEAD_DIM = 128
 
 
+def _strides3(t: torch.Tensor) -> tuple[int, int, int]:
+    return t.stride()[:3]
+
+
 def _as_kernel_operand(t: torch.Tensor, name: str) -> torch.Tensor:
     if t.dtype != torch.bfloat16:
         raise TypeError(f"{name} must be bfloat16, got {t.dtype}")
@@ -153,7 +157,7 @@ def flash_attn_func(
             return out, lse
     args = (
         _ext.ABI_VERSION, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), B, H, Sq, Sk, D,
-        *q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3], *lse.stride()[:2],
+        *_strides3(q), *_strides3(k), *_strides3(v), *_strides3(out), *lse.stride()[:2],
         scale, 0, cu_q_ptr, cu_k_ptr, segments, longest,
     )
     rc = _ext.attn_fwd(device, *args, 0, _ext.H3A_WORKSPACE_ASK if split_tail else 0)
