@@ -159,13 +159,15 @@ struct Tile {
 // multiple of 16 another lane's 8 columns, read from the row in LDS;
 // otherwise any_r_partners. cos / sin of the next token are loaded before the
 // current one is computed, once for the heads of the tile.
-// Bound by VALU issue (one wave per SIMD, the matrix cores idle): row-wise it
-// needs about 90 instructions per four rows, roughly 5 us of a 256 x 256 tile
-// at R = 128 where a head's columns in the accumulator layout (4 lanes x 32
-// columns) took 13, and R = 126 costs little more (element-wise partner and
-// table reads there: 332 us for the q/k/v launch of 1,296 tokens x 40 heads,
-// now 200 with the tile shape of that launch). The longest launches hardly
-// gain (6,240 tokens: 741 -> 742 us): there the clock follows the power drawn.
+// Bound by VALU issue (one wave per SIMD, the matrix cores idle), and on long
+// launches by the power it draws: the weights are multiplied into the token's
+// tables once for the tile's heads, so that a rotated value takes three
+// instructions (with the norm and the rotation applied one after the other,
+// and both selected per column, 49,920 tokens x 40 heads took 5,905 us, now
+// 5,745; the epilogue in the accumulator layout, 4 lanes x 32 columns of a
+// head, 5,710). At R = 126, where that layout read partners and tables element
+// by element, the q/k/v launch of 1,296 tokens went from 332 to 205 us with the
+// tile shape of that launch; 6,240 tokens at R = 128 from 748 to 730.
 template <typename T>
 __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoord& tc, const f32x4 (&acc)[T::NA][T::NB],
                                          int wn, int wm, int tid, char* smem) {
@@ -227,26 +229,34 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
     unpack8(*(const i32x4*)((const uint16_t*)sec.norm_w + col0), wv);
 
     // Norm and RoPE of the tile's rows: kForm 0: no rotary columns, 1: R a
-    // multiple of 16 and tables with 16-byte rows, 2: any even R.
+    // multiple of 16 and tables with 16-byte rows (3: R = 128, every lane
+    // rotary), 2: any even R.
     auto rows = [&](auto form_c) __attribute__((always_inline)) {
         constexpr int kForm = decltype(form_c)::value;
-        const bool rot = kForm == 1 && col0 < R;
+        constexpr bool kLanes = kForm == 1 || kForm == 3;
+        const bool rot = kForm == 3 || (kForm == 1 && col0 < R);
         const bool first = col0 < half;
-        const int pj = rot ? (first ? j + (half >> 3) : j - (half >> 3)) : j;  // partner lane (kForm 1)
+        const int pj = rot ? (first ? j + (half >> 3) : j - (half >> 3)) : j;  // partner lane (kLanes)
         uint32_t pmask[4];
-        if constexpr (kForm == 1) unpack8(*(const i32x4*)((const uint16_t*)sec.norm_w + 8 * pj), wp);
+        // Partner weights with the rotation's sign, zero past R.
+        if constexpr (kLanes) {
+            unpack8(*(const i32x4*)((const uint16_t*)sec.norm_w + 8 * pj), wp);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) wp[e] = !rot ? 0.f : first ? -wp[e] : wp[e];
+        }
         if constexpr (kForm == 2) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const int c = min(col0 + e, R - 1);
-                wp[e] = bf16_to_f32(((const uint16_t*)sec.norm_w)[c < half ? c + half : c - half]);
+                const float w = bf16_to_f32(((const uint16_t*)sec.norm_w)[c < half ? c + half : c - half]);
+                wp[e] = col0 + e >= R ? 0.f : c < half ? -w : w;
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) pmask[i] = col0 + 2 * i < R ? 0xffffffffu : 0u;
         }
         // Tables of a rotate-half pair are equal in both halves: reading the
         // first alone halves their cache traffic.
-        const int tcol = kForm != 1 ? 0 : !rot ? 0 : (p.rope_full_tables == 0 && !first) ? col0 - half : col0;
+        const int tcol = !kLanes ? 0 : !rot ? 0 : (p.rope_full_tables == 0 && !first) ? col0 - half : col0;
         const bool pairs = (((uintptr_t)p.cos | (uintptr_t)p.sin) & 7) == 0 && (p.table_stride & 1) == 0;  // uniform
         struct Tabs {
             f32x4 c[2], s[2];  // cos and sin of the lane's 8 columns
@@ -260,7 +270,7 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
                 const float* const sr = p.sin + (int64_t)s * p.table_stride;
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    if constexpr (kForm == 1) {
+                    if constexpr (kLanes) {
                         w.c[i] = *(const f32x4*)(cr + tcol + 4 * i);
                         w.s[i] = *(const f32x4*)(sr + tcol + 4 * i);
                     } else {
@@ -283,6 +293,15 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
         // the wave's, so every lane joins the row sums and partner reads.
         const int t_end = (tokens - 4 * (g >> 2) + 15) / 16;  // iterations of this wave
         auto token = [&](int t, const Tabs& tab) __attribute__((always_inline)) {
+            // y = r (x w cos + x' w' sin): the weights times the tables are the
+            // token's, shared by its heads.
+            float tc_[8], ts_[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const bool in = kLanes ? rot : kForm == 2 && col0 + e < R;
+                tc_[e] = in ? wv[e] * tab.c[e >> 2][e & 3] : wv[e];
+                ts_[e] = in ? wp[e] * tab.s[e >> 2][e & 3] : 0.f;
+            }
 #pragma unroll
             for (int h = 0; h < kHeads; ++h) {
                 if (h >= heads) break;
@@ -298,7 +317,7 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
                     for (int e = 0; e < 8; ++e) o[e] = (xv[e] * r) * wv[e];
                 } else {
                     i32x4 px;
-                    if constexpr (kForm == 1) {
+                    if constexpr (kLanes) {
                         px = load_row(t, h, pj);
                     } else {
                         px = any_r_partners(out + T::kOutBytes + g * T::kPartner, x, j, R);
@@ -308,18 +327,7 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
                     float xp[8];
                     unpack8(px, xp);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const float n = (xv[e] * r) * wv[e];
-                        const float pn = (xp[e] * r) * wp[e];
-                        if constexpr (kForm == 1) {
-                            o[e] = rot ? n * tab.c[e >> 2][e & 3] + (first ? -pn : pn) * tab.s[e >> 2][e & 3] : n;
-                        } else {
-                            const bool in = col0 + e < R;
-                            const float c = in ? tab.c[e >> 2][e & 3] : 1.f, sn = tab.s[e >> 2][e & 3];
-                            const float s = !in ? -0.f : col0 + e < half ? -sn : sn;
-                            o[e] = n * c + pn * s;
-                        }
-                    }
+                    for (int e = 0; e < 8; ++e) o[e] = (xv[e] * tc_[e] + xp[e] * ts_[e]) * r;
                 }
                 i32x4 w;
 #pragma unroll
@@ -340,6 +348,8 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
     const bool tab16 = (((uintptr_t)p.cos | (uintptr_t)p.sin) & 15) == 0 && (p.table_stride & 3) == 0;
     if (R == 0)
         rows(std::integral_constant<int, 0>{});
+    else if (R == 128 && tab16)
+        rows(std::integral_constant<int, 3>{});
     else if ((R & 15) == 0 && tab16)
         rows(std::integral_constant<int, 1>{});
     else
@@ -560,10 +570,13 @@ hipError_t launch_tile(ProjGemmParams& p, hipStream_t stream) {
     p.n_tiles = 0;
     for (int i = 0; i < p.n_sections; ++i) p.n_tiles += p.sec[i].tiles = (p.sec[i].n + TF - 1) / TF;
     // Token tiles of a group: all of a short launch (every W row is then read
-    // from HBM once), else about 1,024 tokens. 1,296 x 5,120 x 5,120 at 128
-    // tokens a tile: 69.9 us with groups of 2, 63.6 with 8, 61.5 with all 11;
-    // 6,240 x 15,360 x 5,120 at 256: 742 (1), 698 (2), 697 (4), 703 (8), 739 (16).
-    p.group_m = p.m_tiles <= 12 ? p.m_tiles : 1024 / T::kTokens;
+    // from HBM once), else about 1,024 tokens, a little less in a long one.
+    // 1,296 x 5,120 x 5,120 at 128 tokens a tile: 69.9 us with groups of 2, 63.6
+    // with 8, 61.5 with all 11; at 256 tokens and 15,360 x 5,120, 3,000 tokens:
+    // 382 (2), 371 (4), 386 (12); 6,240: 742 (1), 698 (2), 697 (4), 739 (16);
+    // 49,920: 5,767 (2), 5,751 (3), 5,826 (4), 6,041 (8).
+    const int group_tokens = p.m <= 2048 ? 2048 : p.m <= 16384 ? 1024 : 768;
+    p.group_m = group_tokens / T::kTokens < p.m_tiles ? group_tokens / T::kTokens : p.m_tiles;
     hipLaunchKernelGGL((proj_gemm_kernel<TF, NT, SW, SX>), dim3((unsigned)(p.m_tiles * p.n_tiles)), dim3(kPThreads), 0, stream, p);
     return hipGetLastError();
 }
