@@ -1045,7 +1045,9 @@ __device__ __forceinline__ void attn_unit(Params& p, const UnitView& u) {
         const f32x2 hm = halves(mx);
         const float m_new = fmaxf(mc, fmaxf(hm.x, hm.y) * c);
         if (__builtin_amdgcn_ballot_w64(m_new > mc)) {
-            const float alpha = fast_exp2(mc - m_new);
+            // (A row without a finite score so far has nothing to rescale:
+            // -inf less -inf would make NaN of it.)
+            const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(mc - m_new);
             mc = m_new;
             l_run *= alpha;
 #pragma unroll

@@ -85,6 +85,41 @@ def test_short_packed_segments(qlens, klens):
         assert_parity(out[:, a:b].cpu(), lse[:, :, a:b].cpu(), ref_out, ref_lse, f"rows {a}:{b}")
 
 
+def _overflowed_block(Sq, Sk, H, row, block, seed):
+    """q, k, v in which the scores of query row `row` against the 32 keys of
+    `block` overflow fp32 to -inf, all other scores being ordinary: the row
+    lives in dims 0..63 (where the other keys are tiny), the others in 64..127."""
+    q, k, v = _qkv(1, Sq, Sk, H, seed)
+    q[..., :64], k[..., :64] = 0, k[..., :64] * 1e-18
+    q[:, row, :, :64], q[:, row, :, 64:] = 1e18, 0
+    k[:, 32 * block : 32 * block + 32, :, :64] = -1e20
+    return q, k, v
+
+
+# Each wave of a unit starts on its own block of keys: one row whose scores
+# there are all -inf, while the wave's other rows have finite ones, keeps the
+# weights of the finite blocks that follow. Units of a dense call and of a
+# packed one (48 keys leave the later waves without keys), and the ragged rows
+# beside whole tiles.
+@pytest.mark.parametrize(
+    "Sq, Sk, H, row, block, packed",
+    [(64, 600, 2, 5, 0, False), (64, 600, 2, 40, 3, False), (40, 48, 3, 39, 0, False), (1296, 300, 40, 1290, 1, False),
+     (64, 600, 2, 5, 0, True), (64, 600, 2, 40, 3, True), (40, 48, 3, 39, 0, True)],
+)
+def test_units_keep_rows_with_a_block_of_overflowed_scores(Sq, Sk, H, row, block, packed):
+    q, k, v = _overflowed_block(Sq, Sk, H, row, block, Sq + Sk + block)
+    kw = {}
+    if packed:
+        kw = dict(cu_seqlens_q=torch.tensor([0, Sq], dtype=torch.int32, device=DEV),
+                  cu_seqlens_k=torch.tensor([0, Sk], dtype=torch.int32, device=DEV), max_seqlen_q=Sq)
+    out, lse = flash_attn_func(q.to(DEV), k.to(DEV), v.to(DEV), **kw)
+    torch.cuda.synchronize()
+    rows = list(range(row // 32 * 32, min(Sq, row // 32 * 32 + 32)))
+    ref_out, ref_lse = sdpa_reference(q[:, rows], k, v)
+    assert torch.isfinite(ref_lse).all()
+    assert_parity(out.cpu()[:, rows], lse.cpu()[:, :, rows], ref_out, ref_lse, f"{Sq}x{Sk} block {block}")
+
+
 # Queued last rounds over short key ranges (pieces of a few key tiles).
 @pytest.mark.parametrize("H, Sq, Sk", [(20, 3500, 1500), (40, 2048, 2048), (70, 1024, 1300)])
 def test_last_round_pieces_of_short_key_ranges(H, Sq, Sk):
