@@ -161,7 +161,7 @@ struct Tile {
 // current one is computed, once for the heads of the tile.
 // Bound by VALU issue (one wave per SIMD, the matrix cores idle), and on long
 // launches by the power it draws: the weights are multiplied into the token's
-// tables once for the tile's heads, so that a rotated value takes three
+// tables once for the tile's heads, so that a rotated value takes four
 // instructions (with the norm and the rotation applied one after the other,
 // and both selected per column, 49,920 tokens x 40 heads took 5,905 us, now
 // 5,745; the epilogue in the accumulator layout, 4 lanes x 32 columns of a
@@ -293,8 +293,10 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
         // the wave's, so every lane joins the row sums and partner reads.
         const int t_end = (tokens - 4 * (g >> 2) + 15) / 16;  // iterations of this wave
         auto token = [&](int t, const Tabs& tab) __attribute__((always_inline)) {
-            // y = r (x w cos + x' w' sin): the weights times the tables are the
-            // token's, shared by its heads.
+            // y = (x r) (w cos) + (x' r) (w' sin): the weights times the tables
+            // are the token's, shared by its heads. r comes first, as in the
+            // separate steps: a row whose squares overflow fp32 (r = 0) gives
+            // zeros, and small rows lose no bits to a subnormal product.
             float tc_[8], ts_[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -327,7 +329,7 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
                     float xp[8];
                     unpack8(px, xp);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) o[e] = (xv[e] * tc_[e] + xp[e] * ts_[e]) * r;
+                    for (int e = 0; e < 8; ++e) o[e] = (xv[e] * r) * tc_[e] + (xp[e] * r) * ts_[e];
                 }
                 i32x4 w;
 #pragma unroll

@@ -102,6 +102,33 @@ def check_qkv(x, w, b, nwq, nwk, cos, sin, seqlen, y, rows=None, eps=1e-6):
     assert_matches(ys[:, 2 * n :], projection_reference(xs, w[2 * n :], bb(2)), "v")
 
 
+@pytest.mark.parametrize("M", [40, 3000])
+@pytest.mark.parametrize("R", [128, 96, 42, 0])
+def test_edge_magnitudes(M, R):
+    # the projection by the identity leaves rows of zeros (r = rsqrt(eps)), of
+    # tiny values (squares underflow), of large ones whose squares still sum
+    # finitely and of ones whose squares overflow fp32 (r = 0, so zeros, also
+    # where a rotated pair's products would pass fp32): small and large tiles
+    # against the oracle's projection followed by the norm and RoPE
+    g = torch.Generator().manual_seed(R + M)
+    x = torch.randn((M, 128), generator=g).to(torch.bfloat16)
+    x[0], x[1], x[2], x[3] = 0.0, x[1] * 1e-30, x[2] * 1e17, x[3] * 1e30
+    x[4], x[5] = 3.0e38, -3.0e38
+    x[6] = x[6] * 1e-38
+    w = torch.eye(128).to(torch.bfloat16).repeat(3, 1)
+    nw = (1 + 0.1 * torch.randn(128, generator=g)).to(torch.bfloat16)
+    cos, sin = tables(M, R) if R else (None, None)
+    if R:
+        cos[4:6], sin[4:6] = 0.5**0.5, 0.5**0.5
+    y = run_qkv(x, w, None, nw, nw, cos, sin, M, rotate_half=R % 32 == 0)
+    ref = projection_reference(x, w[:128], None, nw, 1e-6, cos, sin, M)
+    assert torch.isfinite(ref.float()).all()
+    assert torch.isfinite(y.float()).all()
+    assert torch.equal(y[:, 256:], x)
+    assert_matches(y[:, :128], ref, "q")
+    assert_matches(y[:, 128:256], ref, "k")
+
+
 @pytest.mark.parametrize(
     "M, K, heads, R, bias, seqlen",
     [
