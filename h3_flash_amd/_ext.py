@@ -388,6 +388,8 @@ class Launch:
         self._bound = (None, None)  # library, function
 
     def __call__(self, device: torch.device, *members) -> int:
+        if device.type != "cuda":  # the kernel would read host memory
+            raise ValueError(f"{self.name} needs tensors on a ROCm device, got {device}")
         lib = load_library()
         bound, fn = self._bound
         if bound is not lib:

@@ -12,6 +12,7 @@ import subprocess
 from pathlib import Path
 
 import pytest
+import torch
 
 from h3_flash_amd import _ext
 
@@ -92,3 +93,20 @@ def test_packed_arguments_match_the_structure(launch, ctype):
     packed = launch._pack(*members(args))
     assert len(packed) == ctypes.sizeof(ctype)
     assert list(members(ctype.from_buffer_copy(packed))) == list(members(args))
+
+
+def test_host_tensors_never_reach_a_launch(monkeypatch):
+    """An entry point called with tensors that are not on a GPU raises before
+    the library is called (the kernel would read host addresses)."""
+    from h3_flash_amd.projection import Section, proj_gemm
+
+    called = []
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0, raising=False)
+    monkeypatch.setattr(_ext.proj_gemm, "_proto", lambda bound: lambda *args: called.append(args) or 0)
+    monkeypatch.setattr(_ext.proj_gemm, "_bound", (None, None))
+    monkeypatch.setattr(_ext, "load_library", lambda path=None: called)
+    x, w = torch.zeros(4, 128, dtype=torch.bfloat16), torch.zeros(128, 128, dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="ROCm device"):
+        proj_gemm(x, [Section(w, torch.empty(4, 128, dtype=torch.bfloat16))])
+    assert called == []
