@@ -300,25 +300,30 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
     bf16x8 qf_own[8];
     bf16x8(&qf)[8] = *(kPersist ? (bf16x8(*)[8])qcarry : &qf_own);
     const bool issue = !kPersist || !prefetched;  // false: the previous tile issued Q and the first K / V
-    if (kPersist && issue) {
-        // Q is carried across the loop of a persistent launch, where the
-        // compiler may copy its registers: compiler-tracked loads, which it
-        // waits for before any copy or use.
-        const __amdgpu_buffer_rsrc_t rqb = make_rsrc(qb, span_bytes(sq, p.q_rs));
+    // (Called only on the path that goes on to use Q: the loads are not tracked
+    // by the compiler, which hands registers that no path ahead reads out again
+    // while they are in flight.)
+    auto load_q = [&]() __attribute__((always_inline)) {
+        if constexpr (kPersist) {
+            // Q is carried across the loop of a persistent launch, where the
+            // compiler may copy its registers: compiler-tracked loads, which it
+            // waits for before any copy or use.
+            const __amdgpu_buffer_rsrc_t rqb = make_rsrc(qb, span_bytes(sq, p.q_rs));
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
-            qf[ks] = __builtin_bit_cast(bf16x8, buf_load16(rqb, (uint32_t)(mq * p.q_rs + ks * 32 + hi * 16)));
-    } else if (issue) {
+            for (int ks = 0; ks < 8; ++ks)
+                qf[ks] = __builtin_bit_cast(bf16x8, buf_load16(rqb, (uint32_t)(mq * p.q_rs + ks * 32 + hi * 16)));
+        } else {
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            i32x4 raw;
-            asm volatile("buffer_load_dwordx4 %0, %1, %2, 0 offen"
-                         : "=v"(raw)
-                         : "v"((uint32_t)((mq - q_first) * p.q_rs + ks * 32 + hi * 16)), "s"(rq)
-                         : "memory");
-            qf[ks] = __builtin_bit_cast(bf16x8, raw);
+            for (int ks = 0; ks < 8; ++ks) {
+                i32x4 raw;
+                asm volatile("buffer_load_dwordx4 %0, %1, %2, 0 offen"
+                             : "=v"(raw)
+                             : "v"((uint32_t)((mq - q_first) * p.q_rs + ks * 32 + hi * 16)), "s"(rq)
+                             : "memory");
+                qf[ks] = __builtin_bit_cast(bf16x8, raw);
+            }
         }
-    }
+    };
 
     // DMA map: wave w fills rows 8w .. 8w+7 of a tile with two 4-row loads;
     // lane L writes LDS chunk (L & 15) of row r0 + (L >> 4), which holds the
@@ -696,15 +701,13 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
     // power it would take go to the other waves.
     if (kEven && m0 + wave * 32 >= sq && ntiles > 0) {
         auto stage = [&](int t) { return (t + off) & 3; };
-        if (issue) {
-            dma_k(0, stage(0));
-            dma_k(1, stage(1));
-            dma_v(0, stage(0));
-            dma_k(2, stage(2));
-            dma_v(1, stage(1));
-            dma_k(3, stage(3));
-            dma_v(2, stage(2));
-        }
+        dma_k(0, stage(0));
+        dma_k(1, stage(1));
+        dma_v(0, stage(0));
+        dma_k(2, stage(2));
+        dma_v(1, stage(1));
+        dma_k(3, stage(3));
+        dma_v(2, stage(2));
         wait_vmcnt<6 * kDmaPerTile>();
         barrier();
         barrier();
@@ -726,6 +729,7 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
     }
     if (ntiles > 0) {
         if (issue) {
+            load_q();
             dma_k(0, off);
             dma_k(1, 1 + off);
             dma_v(0, off);

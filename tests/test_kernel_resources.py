@@ -13,13 +13,20 @@ change elsewhere in the kernel easily tips them into spilling. So:
   SIMD (at most 256 VGPRs + AGPRs per wave) and at most the CU's 160 KiB of
   LDS.
 
+* the Q loads of the attention forms, which the compiler does not track, are
+  used on every path that follows them.
+
 Reads the built library only (skipped where it has not been built); the
 parse needs no GPU.
 """
 
 from __future__ import annotations
 
+import os
+import re
+import shutil
 import struct
+import subprocess
 
 import pytest
 
@@ -118,3 +125,78 @@ def test_attention_forms_fit_one_workgroup_per_cu(kernels):
         assert k[".vgpr_count"] + k.get(".agpr_count", 0) <= 256, (name, k[".vgpr_count"], k.get(".agpr_count"))
         assert k[".group_segment_fixed_size"] <= 160 * 1024, name
         assert k[".max_flat_workgroup_size"] == 512, name
+
+
+def _objdump() -> str | None:
+    llvm = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
+    return llvm if os.path.isfile(llvm) else shutil.which("llvm-objdump")
+
+
+def _vgprs(operand: str) -> set[int]:
+    m = re.fullmatch(r"v\[(\d+):(\d+)\]|v(\d+)", operand)
+    if m is None:
+        return set()
+    lo = int(m[1] or m[3])
+    return set(range(lo, int(m[2] or m[3]) + 1))
+
+
+def _unused_loads(asm: str) -> list[str]:
+    """Plain buffer loads into VGPRs (not the LDS DMA) from which some path
+    reaches the end of the kernel, or another write of the registers, without
+    having read them: the compiler may hand such registers out again while the
+    load is in flight."""
+
+    code, at = [], {}  # (opcode, operands, branch target), index by address
+    for line in asm.splitlines():
+        m = re.match(r"\s+(\S+)(.*?)//\s*([0-9A-F]+):[^<]*(?:<\S+\+0x([0-9a-f]+)>)?", line)
+        if m is None:
+            continue
+        at[int(m[3], 16)] = len(code)
+        operands = [o.strip() for o in m[2].split(",")]
+        operands[-1] = operands[-1].split(" ")[0]
+        code.append((m[1], operands, m[4], m[2]))
+    start = min(at)
+    bad = []
+    for i, (op, operands, _, text) in enumerate(code):
+        if not op.startswith("buffer_load") or text.rstrip().endswith("lds"):
+            continue
+        dst, todo, seen = _vgprs(operands[0]), [i + 1], set()
+        while todo:
+            j = todo.pop()
+            if j in seen:
+                continue
+            seen.add(j)
+            o, args, target, _ = code[j]
+            store = "store" in o or o.startswith("ds_write")
+            reads = set().union(*(_vgprs(a) for a in (args if store else args[1:])))
+            if dst & reads:
+                continue
+            if o == "s_endpgm" or (not store and dst & _vgprs(args[0])):
+                bad.append(f"{op} {text.strip()} -> {o} {','.join(args)}")
+                break
+            if o.startswith(("s_cbranch", "s_branch")):
+                todo.append(at[start + int(target, 16)])
+            if o != "s_branch":
+                todo.append(j + 1)
+    return bad
+
+
+def test_loads_the_compiler_does_not_track_are_always_used(tmp_path):
+    if not LIB_PATH.is_file():
+        pytest.skip("library not built")
+    if _objdump() is None:
+        pytest.skip("no llvm-objdump")
+    forms = 0
+    for i, co in enumerate(gfx950_code_objects(LIB_PATH.read_bytes())):
+        names = [k[".name"] for k in kernel_metadata(co) if "attn_fwd_kernel" in k[".name"]]
+        if not names:
+            continue
+        path = tmp_path / f"{i}.co"
+        path.write_bytes(co)
+        for name in names:
+            asm = subprocess.run([_objdump(), "-d", f"--disassemble-symbols={name}", str(path)], check=True,
+                                 capture_output=True, text=True).stdout
+            assert "buffer_load_dwordx4" in asm
+            assert _unused_loads(asm) == [], name
+            forms += 1
+    assert forms >= 4
