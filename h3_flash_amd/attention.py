@@ -96,8 +96,8 @@ def flash_attn_func(
     more tiles than CUs; statically assigned when a single round would
     leave most CUs idle), merged by a second kernel; the workspace comes
     from torch's stream-ordered caching allocator. Short attention, and at
-    most 32 rows past the whole tiles, run as units of 32 rows with the keys
-    split over a workgroup's waves (no workspace). ``False`` runs every tile
+    most 32 rows past whole tiles that are not cut, run as units of 32 rows
+    with the keys split over a workgroup's waves (no workspace). ``False`` runs every tile
     whole (results differ by rounding).
 
     Raises RuntimeError for semantics the dense path does not serve (causal,

@@ -82,7 +82,7 @@ constexpr int kQueueMinKeyTiles = 48;
 // Key tiles from which a 4-way queued split is graded (its small pieces keep
 // 32 key tiles or more).
 constexpr int kGradedMinKeyTiles = 256;
-// Times in a launch's last round (plan_attn_split), in us: the fixed part of a
+// Times in a launch's last round (plan_attn_last_round), in us: the fixed part of a
 // tile or piece, and the launches that pieces add. At most kMaxPieces pieces.
 constexpr double kTileUs = 9.7, kPiecesUs = 14.0;
 constexpr int kMaxPieces = 8;
@@ -1742,6 +1742,32 @@ int attn_fwd_block_n() { return kBN; }
 int attn_fwd_window_rows() { return kWindowRows > kBM ? kWindowRows : kBM; }
 int attn_fwd_row_margin() { return kBM + kBN * (2 * kStages + 2); }
 
+// Expected time of the jobs (tiles or pieces of kt key tiles) of the last rounds
+// of a launch: their fixed part and their key tiles, slower the more CUs are
+// busy (power).
+static double round_us(int64_t jobs, double kt, int cus) {
+    const double busy = jobs < cus ? (double)jobs / (double)cus : 1.0;
+    return (double)((jobs + cus - 1) / cus) * (kTileUs + kt * (1.0 + 0.6 * busy));
+}
+
+// Expected time of whole tiles, the last round cut where that is shorter.
+static double tiles_us(int64_t tiles, int64_t key_tiles, int cus) {
+    const int64_t full = (tiles - 1) / cus * cus, rest = tiles - full;
+    const int n = plan_attn_last_round(tiles, key_tiles, cus, INT64_MAX).split_n;
+    return (double)(full / cus) * round_us(cus, (double)key_tiles, cus) +
+           (n > 0 ? round_us(rest * n, (double)key_tiles / n, cus) + kPiecesUs : round_us(rest, (double)key_tiles, cus));
+}
+
+bool attn_rag_pays(int64_t whole, int64_t units, int64_t keys, int cus) {
+    if (cus <= 0) return false;
+    if (whole + units <= cus) return true;  // all at once, as the tiles would be
+    // The units read every head's K and V again, which the ragged tiles have
+    // from the L2 beside their neighbours (512 bytes a key at about 3.4 TB/s
+    // while the tiles run).
+    const int64_t kt = (keys + kBN - 1) / kBN;
+    return tiles_us(whole + units, kt, cus) - tiles_us(whole, kt, cus) > 1.5e-4 * (double)units * (double)keys;
+}
+
 int attn_rag_blocks(int64_t tiles, int64_t units, int64_t keys, int cus) {
     // The units run one after another on the CUs that the last round of tiles
     // leaves idle where they have the time for it, else one per workgroup. (As
@@ -1769,27 +1795,6 @@ SplitPlan plan_attn_split(int64_t tiles, int64_t key_tiles, int cus, int64_t max
         auto bytes = [&](int n) { return ((int64_t)n * rest * piece_bytes + 255) / 256 * 256 + 256; };
         int n = kQueuePieces;
         while (n > 1 && (key_tiles / n < kQueueMinKeyTiles || bytes(n) > max_workspace)) --n;
-        if (n < 2) {
-            // Shorter key ranges: pieces pay where they fill a last round that
-            // would leave CUs idle, by the expected time: a tile's or piece's
-            // fixed part, its key tiles (slower the more CUs are busy: power),
-            // and what pieces cost besides (the counter's reset, the merge).
-            // Measured (us, whole -> pieces): 24 heads of 4,096 x 4,096 200 ->
-            // 185, 40 of 2,048 x 2,048 100 -> 92, 20 of 3,500 x 3,500 162 ->
-            // 125; 8 of 10,240 x 1,024 58 -> 60, which the rule leaves whole.
-            auto last_round = [&](int64_t jobs, double kt) {
-                const double busy = jobs < cus ? (double)jobs / (double)cus : 1.0;
-                return (double)((jobs + cus - 1) / cus) * (kTileUs + kt * (1.0 + 0.6 * busy));
-            };
-            double best = last_round(rest, (double)key_tiles) - 2.0;
-            for (int c = 2; c <= kMaxPieces && key_tiles / c >= 2 && bytes(c) <= max_workspace; ++c) {
-                const double us = last_round(rest * c, (double)key_tiles / c) + kPiecesUs;
-                if (us < best) {
-                    best = us;
-                    n = c;
-                }
-            }
-        }
         if (n < 2) return plan;
         plan.n_full = (int32_t)full;
         plan.split_n = n;
@@ -1821,6 +1826,36 @@ SplitPlan plan_attn_split(int64_t tiles, int64_t key_tiles, int cus, int64_t max
     plan.split_n = best_n;
     plan.split_tiles = (int32_t)tiles;
     plan.workspace_bytes = (int64_t)best_n * tiles * piece_bytes;
+    return plan;
+}
+
+SplitPlan plan_attn_last_round(int64_t tiles, int64_t key_tiles, int cus, int64_t max_workspace) {
+    SplitPlan plan{(int32_t)tiles, 0, 0, 0, 0, 0};
+    if (cus < 8 || cus % 8 != 0 || tiles <= cus) return plan;
+    const int64_t piece_bytes = attn_fwd_piece_bytes();
+    const int64_t full = (tiles - 1) / cus * cus, rest = tiles - full;
+    auto bytes = [&](int n) { return ((int64_t)n * rest * piece_bytes + 255) / 256 * 256 + 256; };
+    // Pieces pay where they fill a last round that would leave CUs idle, by the
+    // expected time, with what they cost besides (the counter's reset, the
+    // merge). Measured (us, whole -> pieces): 24 heads of 4,096 x 4,096 200 ->
+    // 185, 40 of 2,048 x 2,048 100 -> 92, 20 of 3,500 x 3,500 162 -> 125; 8 of
+    // 10,240 x 1,024 58 -> 60, which the rule leaves whole.
+    int n = 0;
+    double best = round_us(rest, (double)key_tiles, cus) - 2.0;
+    for (int c = 2; c <= kMaxPieces && key_tiles / c >= 2 && bytes(c) <= max_workspace; ++c) {
+        const double us = round_us(rest * c, (double)key_tiles / c, cus) + kPiecesUs;
+        if (us < best) {
+            best = us;
+            n = c;
+        }
+    }
+    if (n == 0) return plan;
+    plan.n_full = (int32_t)full;
+    plan.split_n = n;
+    plan.split_tiles = (int32_t)rest;
+    plan.queue_blocks = (int32_t)(rest * n < cus ? rest * n : cus);
+    plan.queue_offset = ((int64_t)n * rest * piece_bytes + 255) / 256 * 256;
+    plan.workspace_bytes = bytes(n);
     return plan;
 }
 

@@ -179,16 +179,6 @@ int device_cus() {
     return n;
 }
 
-// Dense launches with at most 32 rows past their whole tiles run those rows as
-// units beside the tiles.
-void take_rag_units(const h3a_attn_args* a, h3a::AttnParams& p) {
-    const int64_t rag = a->seqlen_q % h3a::attn_fwd_block_m();
-    if (p.cu_q != nullptr || p.wide != 0 || p.n_qtiles < 2 || rag == 0 || rag > h3a::attn_fwd_unit_rows()) return;
-    p.n_qtiles -= 1;
-    const int64_t units = (int64_t)p.heads * p.n_groups;
-    p.rag_blocks = h3a::attn_rag_blocks(units * p.n_qtiles, units, a->seqlen_k, device_cus());
-}
-
 // Units per (group, head) of a launch that runs as units of 32 rows (short
 // attention), or 0 where the 256-row tiles are faster.
 int32_t attn_units(const h3a_attn_args* a, const h3a::AttnParams& p) {
@@ -221,13 +211,34 @@ int32_t attn_units(const h3a_attn_args* a, const h3a::AttnParams& p) {
 }
 
 // Split plan of a validated launch: dense inputs only (varlen tiles are not
-// uniform work).
+// uniform work). The whole tiles beside ragged units stay whole but for a last
+// round of short key ranges.
 h3a::SplitPlan attn_plan(const h3a_attn_args* a, const h3a::AttnParams& p, int64_t max_workspace = INT64_MAX) {
     const int64_t tiles = (int64_t)p.n_qtiles * p.heads * p.n_groups;
-    h3a::SplitPlan none{(int32_t)tiles, 0, 0, 0, 0, 0};
+    const h3a::SplitPlan none{(int32_t)tiles, 0, 0, 0, 0, 0};
     if (a->cu_seqlens_q != nullptr) return none;
-    const int bn = h3a::attn_fwd_block_n();
-    return h3a::plan_attn_split(tiles, (a->seqlen_k + bn - 1) / bn, device_cus(), max_workspace);
+    const int bn = h3a::attn_fwd_block_n(), cus = device_cus();
+    const int64_t key_tiles = (a->seqlen_k + bn - 1) / bn;
+    const h3a::SplitPlan split = p.rag_blocks > 0 ? none : h3a::plan_attn_split(tiles, key_tiles, cus, max_workspace);
+    return split.split_n != 0 ? split : h3a::plan_attn_last_round(tiles, key_tiles, cus, max_workspace);
+}
+
+// Dense launches of whole tiles with at most 32 rows past them run those rows
+// as units beside the tiles. Where plan_attn_split cuts the tiles, the ragged
+// ones are cut with them: a unit passes all keys alone, and without the ragged
+// tiles the plan would be another (us, with units / as planned: 8 heads of
+// 2,064 x 2,064, 72 tiles in 7 pieces each 46 / 35, 20 of 1,296 x 1,296 53 / 35,
+// 1 of 528 x 49,920 236 / 154, 16 of 2,832 x 2,832, where 176 tiles would be
+// cut and 192 are not, 90 / 73).
+void take_rag_units(const h3a_attn_args* a, h3a::AttnParams& p, int64_t max_workspace = INT64_MAX) {
+    const int64_t rag = a->seqlen_q % h3a::attn_fwd_block_m();
+    if (p.cu_q != nullptr || p.wide != 0 || p.n_qtiles < 2 || rag == 0 || rag > h3a::attn_fwd_unit_rows()) return;
+    const int bn = h3a::attn_fwd_block_n(), cus = device_cus();
+    const int64_t units = (int64_t)p.heads * p.n_groups;
+    if (h3a::plan_attn_split(units * p.n_qtiles, (a->seqlen_k + bn - 1) / bn, cus, max_workspace).split_n != 0) return;
+    if (!h3a::attn_rag_pays(units * (p.n_qtiles - 1), units, a->seqlen_k, cus)) return;
+    p.n_qtiles -= 1;
+    p.rag_blocks = h3a::attn_rag_blocks(units * p.n_qtiles, units, a->seqlen_k, cus);
 }
 
 // The workspace of a launch: the split plan's partial results and counter,
@@ -440,7 +451,7 @@ int h3a_attn_fwd_noalloc(const h3a_attn_args* a, void* stream) {
         if (e != hipSuccess) return fail(H3A_ELAUNCH, "h3a_attn_fwd_noalloc: launch failed: %s", hipGetErrorString(e));
         return H3A_OK;
     }
-    take_rag_units(a, p);
+    take_rag_units(a, p, h3a::kStaticScratchBytes);
     void* scratch = nullptr;
     hipError_t e = h3a::attn_static_scratch(&scratch);
     if (e != hipSuccess)

@@ -98,6 +98,8 @@ struct SplitPlan {
 };
 // max_workspace bounds the plan's workspace_bytes (fewer pieces, or none).
 SplitPlan plan_attn_split(int64_t tiles, int64_t key_tiles, int cus, int64_t max_workspace);
+// Pieces of the last round where plan_attn_split cuts none (short key ranges).
+SplitPlan plan_attn_last_round(int64_t tiles, int64_t key_tiles, int cus, int64_t max_workspace);
 
 // Bytes of the file-scope device array that serves as the workspace of the
 // allocation-free attention entry point, and the lookup of the current
@@ -105,6 +107,8 @@ SplitPlan plan_attn_split(int64_t tiles, int64_t key_tiles, int cus, int64_t max
 constexpr int64_t kStaticScratchBytes = H3A_NOALLOC_SCRATCH_BYTES;
 hipError_t attn_static_scratch(void** ptr);
 
+// Whether `units` ragged units beside `whole` whole tiles beat as many more tiles.
+bool attn_rag_pays(int64_t whole, int64_t units, int64_t keys, int cus);
 // Workgroups for `units` ragged units beside `tiles` whole tiles.
 int attn_rag_blocks(int64_t tiles, int64_t units, int64_t keys, int cus);
 int attn_fwd_unit_rows();  // query rows of a unit of a short launch

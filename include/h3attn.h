@@ -138,8 +138,8 @@ extern "C" {
  * With a workspace given, short attention (up to about 256 units of 32 query
  * rows of one head and 2,048 keys, or more units over fewer keys) runs without
  * using it, as one workgroup per unit with the keys split over its waves; so
- * do, beside the tiles, the rows past a dense call's whole tiles when they are
- * at most 32.
+ * may, beside the tiles, the rows past a dense call's whole tiles when they are
+ * at most 32 and the tiles are not cut into pieces.
  * With a NULL workspace every tile runs whole on V as given (a smaller one
  * keeps the units). The results differ only by rounding. A caller that would
  * allocate the workspace only where the launch takes one passes NULL with

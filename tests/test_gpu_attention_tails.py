@@ -52,6 +52,26 @@ def test_rows_past_the_whole_tiles(B, H, Sq, Sk, split):
     assert_parity(out.cpu()[:, rows], lse.cpu()[:, :, rows], ref_out, ref_lse, f"{B}x{H}x{Sq}x{Sk}")
 
 
+# The ragged rows become units only in launches whose tiles all run whole:
+# where the tiles are cut into key-range pieces the ragged ones are cut with
+# them (the rows equal those of a call with 40 rows more, which has as many
+# tiles and no units), and whole tiles stay whole without them.
+@pytest.mark.parametrize("H, Sq, Sk", [(8, 2064, 2064), (20, 1296, 1296), (2, 2064, 17000), (16, 1040, 300)])
+def test_ragged_rows_of_a_split_launch(H, Sq, Sk):
+    q, k, v = (x.to(DEV) for x in _qkv(1, Sq + 40, Sk, H, Sq + Sk))
+    got = flash_attn_func(q[:, :Sq], k, v)
+    more = flash_attn_func(q, k, v)
+    assert torch.equal(got[0], more[0][:, :Sq]) and torch.equal(got[1], more[1][..., :Sq])
+
+
+@pytest.mark.parametrize("H, Sq, Sk", [(16, 2832, 2832), (8, 5904, 300)])
+def test_whole_tiles_beside_ragged_rows_stay_whole(H, Sq, Sk):
+    q, k, v = (x.to(DEV) for x in _qkv(1, Sq, Sk, H, Sq + Sk))
+    got, whole = flash_attn_func(q, k, v), flash_attn_func(q, k, v, split_tail=False)
+    n = Sq // 256 * 256
+    assert torch.equal(got[0][:, :n], whole[0][:, :n]) and torch.equal(got[1][..., :n], whole[1][..., :n])
+
+
 # Units alone: one key, fewer blocks than waves, a last block of one key, no
 # keys, many blocks; packed segments with empty ones and unequal key lengths.
 @pytest.mark.parametrize("B, H, Sq, Sk", [(1, 1, 1, 1), (2, 3, 33, 0), (1, 4, 31, 257), (1, 5, 640, 640), (3, 2, 70, 225), (1, 2, 32, 2048)])
