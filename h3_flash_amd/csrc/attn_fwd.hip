@@ -39,7 +39,7 @@
 #include "common.h"
 #include "kernels.h"
 
-// Workspace of h3a_attn_fwd_noalloc: the partial results (bf16 O, fp32 LSE) of the tail's
+// Workspace of h3a_attn_fwd_noalloc: the partial results (O, fp32 LSE) of the tail's
 // key-range pieces and the tail's counter, for callers that cannot allocate.
 // Every GPU the library runs on holds its own copy until the process ends.
 // Host code never passes `scratch` itself (on the host it names a shadow
@@ -84,7 +84,7 @@ constexpr int kQueueMinKeyTiles = 48;
 constexpr int kGradedMinKeyTiles = 256;
 // Times in a launch's last round (plan_attn_last_round), in us: the fixed part of a
 // tile or piece, and the launches that pieces add. At most kMaxPieces pieces.
-constexpr double kTileUs = 9.7, kPiecesUs = 14.0;
+constexpr double kTileUs = 9.7, kPiecesUs = 17.0;
 constexpr int kMaxPieces = 8;
 
 static_assert(kDmaPerTile == 2, "vmcnt accounting below assumes 2 K + 2 V loads per iteration");
@@ -178,12 +178,12 @@ __device__ __forceinline__ char* attn_lds() {
 // iterations. cu_cur and cu_next hold cu_q[s], cu_q[s + 1], cu_k[s],
 // cu_k[s + 1] of this tile's and the next tile's segment, loaded by the
 // caller one tile ahead. Returns whether it issued the next tile's loads.
-template <bool kWide, bool kVT, bool kPersist = false, typename Params>
+template <bool kWide, bool kVT, bool kPersist = false, bool kPartF32 = false, typename Params>
 __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int chunks, int slot,
                                           bool graded = false, bf16x8* qcarry = nullptr, bool prefetched = false,
                                           int next_tile = -1, const int* cu_cur = nullptr,
                                           const int* cu_next = nullptr, int wave_first = 0) {
-    static_assert(!kPersist || (!kWide && !kVT), "persistent launches use the narrow token-major form");
+    static_assert((!kPersist && !kPartF32) || (!kWide && !kVT), "persistent launches and fp32 pieces use the narrow token-major form");
     char* const smem = attn_lds();
     // V stages 0..3 first, then K stages 0..3: with a per-lane base in a VGPR
     // every fragment read offset then fits the 16-bit ds_read immediate.
@@ -938,9 +938,33 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
         }
     };
     if (slot >= 0) {
-        // Partial result of a key-range piece: normalised O in bf16 (as the
-        // output itself is rounded) and the LSE in fp32, every row.
-        staged_store((char*)(p.ws_o + ((int64_t)slot * kBM + wave * 32) * kD), kD * 2, 32);
+        // Partial result of a key-range piece: normalised O and the LSE in
+        // fp32, every row of the wave. O in bf16 (as the output itself is
+        // rounded), or in fp32 (kPartF32).
+        if constexpr (kPartF32) {
+            // As staged_store, 4 KB a wave over V stages 2 and 3 (both read for
+            // the last time by this call): rows of 128 bytes per 32 dims, the
+            // 16-byte chunks swizzled by row.
+            typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+            lds_char* const staged = (lds_char*)(vst + 2 * kTile) + wave * 32 * 128;
+            char* const base = (char*)p.ws_o + ((int64_t)slot * kBM + wave * 32) * (kD * 4);
+#pragma unroll
+            for (int db = 0; db < 4; ++db) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    *(lds_f32x4*)(staged + l32 * 128 + (((2 * i + hi) ^ (l32 & 7)) << 4)) =
+                        f32x4{oacc[db][i * 4 + 0] * inv, oacc[db][i * 4 + 1] * inv, oacc[db][i * 4 + 2] * inv,
+                              oacc[db][i * 4 + 3] * inv};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int row = (lane >> 3) + 8 * k, c = lane & 7;
+                    const f32x4 v = *(const lds_f32x4*)(staged + row * 128 + ((c ^ (row & 7)) << 4));
+                    *(f32x4*)(base + (int64_t)row * (kD * 4) + db * 128 + c * 16) = v;
+                }
+            }
+        } else {
+            staged_store((char*)p.ws_o + ((int64_t)slot * kBM + wave * 32) * (kD * 2), kD * 2, 32);
+        }
         if (hi == 0) p.ws_lse[(int64_t)slot * kBM + wave * 32 + l32] = lse;
         return false;
     }
@@ -1205,7 +1229,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_short_kernel(AttnParams p) {
 // that the workgroups after the whole tiles take from a counter in the
 // workspace as they free up, so CUs that ran their whole tiles faster (XCD
 // clocks differ) take more of the tail.
-template <bool kWide, bool kVT>
+template <bool kWide, bool kVT, bool kPartF32 = false>
 __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
     __shared__ int queue_head;
     // Workgroups are dispatched round-robin over the 8 XCDs, workgroup i to
@@ -1272,7 +1296,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
     // code (a single call inside the loop below changed its register
     // allocation and made it 1-2% slower).
     if (!queued) {
-        attn_tile<kWide, kVT>(p, tile, chunk, chunks, slot, false, nullptr, false, -1, nullptr, nullptr, wave_first);
+        attn_tile<kWide, kVT, false, kPartF32>(p, tile, chunk, chunks, slot, false, nullptr, false, -1, nullptr, nullptr, wave_first);
         return;
     }
     int* const counter = planned ? (int*)p.vplan + kPlanQueue : p.queue;
@@ -1310,7 +1334,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_fwd_kernel(AttnParams p) {
         int zero;
         asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
         KernArgs* pk = (KernArgs*)((const __attribute__((address_space(4))) char*)&p + zero);
-        attn_tile<kWide, kVT>(*pk, tile, chunk, chunks, slot, !planned, nullptr, false, -1, nullptr, nullptr, wave_first);
+        attn_tile<kWide, kVT, false, kPartF32>(*pk, tile, chunk, chunks, slot, !planned, nullptr, false, -1, nullptr, nullptr, wave_first);
     }
 }
 
@@ -1650,7 +1674,7 @@ __global__ void attn_queue_reset(int* queue) {
 // sequence, ending on a wave-uniform branch at split_n, before any is used.
 constexpr int kMergeRows = 32;
 
-template <int kMaxP>
+template <int kMaxP, bool kPartF32 = false>
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
     const int split_tile = blockIdx.x / (kBM / kMergeRows);
     const int row = (blockIdx.x % (kBM / kMergeRows)) * kMergeRows + threadIdx.x / 8;
@@ -1680,15 +1704,16 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
     const int mq = qt * kBM + row;
     if (mq >= sq) return;
     float lq[kMaxP];
-    i32x4 part[kMaxP][2];  // 16 bf16 head dims of the row per piece
+    constexpr int kLoads = kPartF32 ? 4 : 2;
+    i32x4 part[kMaxP][kLoads];  // 16 head dims of the row per piece
 #pragma unroll
     for (int c = 0; c < kMaxP; ++c) {
         if (c >= n) break;
         const int64_t pc = slot0 + c * slot_step;
         lq[c] = p.ws_lse[pc * kBM + row];
-        const i32x4* src = (const i32x4*)(p.ws_o + (pc * kBM + row) * kD + d0);
-        part[c][0] = src[0];
-        part[c][1] = src[1];
+        const i32x4* src = (const i32x4*)((const char*)p.ws_o + ((pc * kBM + row) * kD + d0) * (kPartF32 ? 4 : 2));
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) part[c][i] = src[i];
     }
     float lse_max = -INFINITY;
 #pragma unroll
@@ -1707,9 +1732,14 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
         wsum += w;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const uint32_t lo = (uint32_t)part[c][i >> 1][2 * (i & 1)], up = (uint32_t)part[c][i >> 1][2 * (i & 1) + 1];
-            const f32x4 x{__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(up << 16),
+            f32x4 x;
+            if constexpr (kPartF32) {
+                x = __builtin_bit_cast(f32x4, part[c][i]);
+            } else {
+                const uint32_t lo = (uint32_t)part[c][i >> 1][2 * (i & 1)], up = (uint32_t)part[c][i >> 1][2 * (i & 1) + 1];
+                x = f32x4{__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(up << 16),
                           __uint_as_float(up & 0xffff0000u)};
+            }
             acc[i] += w * x;
         }
     }
@@ -1737,7 +1767,7 @@ int attn_fwd_block_m() { return kBM; }
 int attn_fwd_persist_max_segments() { return kPersistSegs; }
 int attn_fwd_persist_max_rows() { return kPersistMaxQTiles * kBM; }
 int attn_fwd_tail_pieces() { return kQueuePieces; }
-int64_t attn_fwd_piece_bytes() { return (int64_t)kBM * (kD * 2 + 4); }
+int64_t attn_fwd_piece_bytes(bool f32) { return (int64_t)kBM * (kD * (f32 ? 4 : 2) + 4); }
 int attn_fwd_block_n() { return kBN; }
 int attn_fwd_window_rows() { return kWindowRows > kBM ? kWindowRows : kBM; }
 int attn_fwd_row_margin() { return kBM + kBN * (2 * kStages + 2); }
@@ -1781,9 +1811,9 @@ int attn_rag_blocks(int64_t tiles, int64_t units, int64_t keys, int cus) {
 }
 
 SplitPlan plan_attn_split(int64_t tiles, int64_t key_tiles, int cus, int64_t max_workspace) {
-    SplitPlan plan{(int32_t)tiles, 0, 0, 0, 0, 0};
+    SplitPlan plan{(int32_t)tiles, 0, 0, 0, 0, 0, 0};
     if (cus < 8 || cus % 8 != 0 || tiles <= 0) return plan;
-    const int64_t piece_bytes = attn_fwd_piece_bytes();  // bf16 partial O and fp32 LSE of a piece's rows
+    const int64_t piece_bytes = attn_fwd_piece_bytes(false);  // bf16 partial O and fp32 LSE of a piece's rows
     if (tiles > cus) {
         // Dynamic tail: the whole rounds but the last run as they are; the
         // last round's tiles become kQueuePieces key-range pieces each, taken
@@ -1830,16 +1860,17 @@ SplitPlan plan_attn_split(int64_t tiles, int64_t key_tiles, int cus, int64_t max
 }
 
 SplitPlan plan_attn_last_round(int64_t tiles, int64_t key_tiles, int cus, int64_t max_workspace) {
-    SplitPlan plan{(int32_t)tiles, 0, 0, 0, 0, 0};
+    SplitPlan plan{(int32_t)tiles, 0, 0, 0, 0, 0, 0};
     if (cus < 8 || cus % 8 != 0 || tiles <= cus) return plan;
-    const int64_t piece_bytes = attn_fwd_piece_bytes();
+    const int64_t piece_bytes = attn_fwd_piece_bytes(true);
     const int64_t full = (tiles - 1) / cus * cus, rest = tiles - full;
     auto bytes = [&](int n) { return ((int64_t)n * rest * piece_bytes + 255) / 256 * 256 + 256; };
     // Pieces pay where they fill a last round that would leave CUs idle, by the
     // expected time, with what they cost besides (the counter's reset, the
-    // merge). Measured (us, whole -> pieces): 24 heads of 4,096 x 4,096 200 ->
-    // 185, 40 of 2,048 x 2,048 100 -> 92, 20 of 3,500 x 3,500 162 -> 125; 8 of
-    // 10,240 x 1,024 58 -> 60, which the rule leaves whole.
+    // merge; 3-4 us of it for partial results in fp32 against bf16). Measured
+    // (us, whole -> pieces): 24 heads of 4,096 x 4,096 218 -> 210, 40 of 2,048 x
+    // 2,048 105 -> 101, 20 of 3,500 x 3,500 166 -> 136, 9 of 7,424 x 6,000 271
+    // -> 195; 8 of 10,240 x 1,024 58 -> 60 (bf16), which the rule leaves whole.
     int n = 0;
     double best = round_us(rest, (double)key_tiles, cus) - 2.0;
     for (int c = 2; c <= kMaxPieces && key_tiles / c >= 2 && bytes(c) <= max_workspace; ++c) {
@@ -1856,6 +1887,7 @@ SplitPlan plan_attn_last_round(int64_t tiles, int64_t key_tiles, int cus, int64_
     plan.queue_blocks = (int32_t)(rest * n < cus ? rest * n : cus);
     plan.queue_offset = ((int64_t)n * rest * piece_bytes + 255) / 256 * 256;
     plan.workspace_bytes = bytes(n);
+    plan.part_f32 = 1;
     return plan;
 }
 
@@ -1926,6 +1958,8 @@ hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t stream) {
         hipLaunchKernelGGL((attn_fwd_kernel<true, false>), grid, block, 0, stream, p);
     else if (p.vt != nullptr)
         hipLaunchKernelGGL((attn_fwd_kernel<false, true>), grid, block, 0, stream, p);
+    else if (p.part_f32 != 0)
+        hipLaunchKernelGGL((attn_fwd_kernel<false, false, true>), grid, block, 0, stream, p);
     else
         hipLaunchKernelGGL((attn_fwd_kernel<false, false>), grid, block, 0, stream, p);
     hipError_t e = hipGetLastError();
@@ -1939,7 +1973,9 @@ hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t stream) {
     }
     if (p.split_n == 0) return e;
     const dim3 merge_grid((unsigned)(p.split_tiles * (kBM / kMergeRows)));
-    if (p.split_n <= 4)
+    if (p.part_f32 != 0)
+        hipLaunchKernelGGL((attn_merge_kernel<8, true>), merge_grid, dim3(256), 0, stream, p);
+    else if (p.split_n <= 4)
         hipLaunchKernelGGL(attn_merge_kernel<4>, merge_grid, dim3(256), 0, stream, p);
     else
         hipLaunchKernelGGL(attn_merge_kernel<8>, merge_grid, dim3(256), 0, stream, p);

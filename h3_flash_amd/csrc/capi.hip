@@ -215,12 +215,13 @@ int32_t attn_units(const h3a_attn_args* a, const h3a::AttnParams& p) {
 // round of short key ranges.
 h3a::SplitPlan attn_plan(const h3a_attn_args* a, const h3a::AttnParams& p, int64_t max_workspace = INT64_MAX) {
     const int64_t tiles = (int64_t)p.n_qtiles * p.heads * p.n_groups;
-    const h3a::SplitPlan none{(int32_t)tiles, 0, 0, 0, 0, 0};
+    const h3a::SplitPlan none{(int32_t)tiles, 0, 0, 0, 0, 0, 0};
     if (a->cu_seqlens_q != nullptr) return none;
     const int bn = h3a::attn_fwd_block_n(), cus = device_cus();
     const int64_t key_tiles = (a->seqlen_k + bn - 1) / bn;
     const h3a::SplitPlan split = p.rag_blocks > 0 ? none : h3a::plan_attn_split(tiles, key_tiles, cus, max_workspace);
-    return split.split_n != 0 ? split : h3a::plan_attn_last_round(tiles, key_tiles, cus, max_workspace);
+    if (split.split_n != 0 || p.wide != 0) return split;
+    return h3a::plan_attn_last_round(tiles, key_tiles, cus, max_workspace);
 }
 
 // Dense launches of whole tiles with at most 32 rows past them run those rows
@@ -286,7 +287,7 @@ AttnWorkspace attn_workspace(const h3a_attn_args* a, const h3a::AttnParams& p, b
         ub = ub < grid ? ub : grid;
         const int64_t pieces = (int64_t)h3a::attn_fwd_tail_pieces() * cus;
         const int64_t words = h3a::kPlanWords + ub + 2 * pieces + 2 * cus + 4 * nseg;
-        w.plan_offset = pieces * h3a::attn_fwd_piece_bytes();
+        w.plan_offset = pieces * h3a::attn_fwd_piece_bytes(false);
         w.total = w.plan_offset + (4 * words + 255) / 256 * 256;
         if (w.total > max_workspace) return AttnWorkspace{w.plan, 0, 0, 0, 0, 0, 0, false};
         w.ub_tiles = (int32_t)ub;
@@ -325,8 +326,10 @@ void apply_plan(h3a::AttnParams& p, const h3a::SplitPlan& plan, void* workspace)
     p.n_full = plan.n_full;
     p.split_n = plan.split_n;
     p.split_tiles = plan.split_tiles;
-    p.ws_o = (uint16_t*)workspace;
-    p.ws_lse = (float*)(p.ws_o + (int64_t)plan.split_n * plan.split_tiles * h3a::attn_fwd_block_m() * 128);
+    const int64_t rows = (int64_t)plan.split_n * plan.split_tiles * h3a::attn_fwd_block_m();
+    p.part_f32 = plan.part_f32;
+    p.ws_o = workspace;
+    p.ws_lse = (float*)((char*)workspace + rows * 128 * (plan.part_f32 ? 4 : 2));
     if (plan.queue_blocks > 0) {
         p.queue = (int*)((char*)workspace + plan.queue_offset);
         p.queue_blocks = plan.queue_blocks;
@@ -416,8 +419,8 @@ int h3a_attn_fwd(const h3a_attn_args* a, void* stream) {
         if (w.persist) apply_persist(a, p, a->workspace, w.cus);
         if (w.ub_tiles > 0) {
             const int64_t pieces = (int64_t)h3a::attn_fwd_tail_pieces() * w.cus;
-            p.ws_o = (uint16_t*)a->workspace;
-            p.ws_lse = (float*)(p.ws_o + pieces * h3a::attn_fwd_block_m() * 128);
+            p.ws_o = a->workspace;
+            p.ws_lse = (float*)((char*)a->workspace + pieces * h3a::attn_fwd_block_m() * 128 * 2);
             int32_t* words = (int32_t*)((char*)a->workspace + w.plan_offset);
             p.vplan = p.vplan_w = words;
             p.vlist = p.vlist_w = words + h3a::kPlanWords;

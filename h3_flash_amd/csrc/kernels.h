@@ -31,13 +31,14 @@ struct AttnParams {
     const int32_t* cu_k;
     // Key-range split of the last tiles (dense only; split_n == 0: none).
     // Tiles [0, n_full) run whole; tiles [n_full, n_full + split_tiles) run as
-    // split_n pieces each, which write normalised bf16 partial O and fp32
+    // split_n pieces each, which write normalised partial O and fp32
     // LSE to ws_o / ws_lse for attn_merge to combine.
     int32_t n_full;
     int32_t split_n;
     int32_t split_tiles;
-    uint16_t* ws_o;  // bf16 [split_n * split_tiles][kBM][128], normalised
+    void* ws_o;      // bf16 or (part_f32) fp32 [split_n * split_tiles][kBM][128], normalised
     float* ws_lse;   // [split_n * split_tiles][kBM]
+    int32_t part_f32;  // (dense, narrow, V as given)
     // Dynamic tail (queue != NULL): workgroups [0, n_full) run whole tiles;
     // the queue_blocks workgroups after them take piece indices
     // [0, split_n * split_tiles) from *queue, which the launch zeroes, until
@@ -95,10 +96,12 @@ struct SplitPlan {
     int32_t queue_blocks;   // > 0: dynamic tail with this many workgroups
     int64_t queue_offset;   // byte offset of the tail counter in the workspace
     int64_t workspace_bytes;
+    int32_t part_f32;       // pieces keep fp32 O (else bf16)
 };
 // max_workspace bounds the plan's workspace_bytes (fewer pieces, or none).
 SplitPlan plan_attn_split(int64_t tiles, int64_t key_tiles, int cus, int64_t max_workspace);
-// Pieces of the last round where plan_attn_split cuts none (short key ranges).
+// Pieces of the last round where plan_attn_split cuts none (short key ranges);
+// fp32, as these tiles would otherwise hold their sums in fp32 to the end.
 SplitPlan plan_attn_last_round(int64_t tiles, int64_t key_tiles, int cus, int64_t max_workspace);
 
 // Bytes of the file-scope device array that serves as the workspace of the
@@ -119,7 +122,7 @@ int attn_fwd_persist_max_rows();
 // Most key-range pieces per tile of a tail, and the workspace bytes of one
 // piece's fp32 partial O and LSE.
 int attn_fwd_tail_pieces();
-int64_t attn_fwd_piece_bytes();
+int64_t attn_fwd_piece_bytes(bool f32);
 int attn_fwd_block_n();
 // Rows one buffer resource of the kernel spans from its base (a query tile, or
 // a window of key tiles in the wide form); their bytes must stay below 2^31.
