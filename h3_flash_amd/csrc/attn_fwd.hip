@@ -84,7 +84,7 @@ constexpr int kQueueMinKeyTiles = 48;
 constexpr int kGradedMinKeyTiles = 256;
 // Times in a launch's last round (plan_attn_last_round), in us: the fixed part of a
 // tile or piece, and the launches that pieces add. At most kMaxPieces pieces.
-constexpr double kTileUs = 9.7, kPiecesUs = 17.0;
+constexpr double kTileUs = 9.7, kPiecesUs = 14.0;
 constexpr int kMaxPieces = 8;
 
 static_assert(kDmaPerTile == 2, "vmcnt accounting below assumes 2 K + 2 V loads per iteration");
@@ -380,6 +380,71 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
         for (int i = 0; i < kDmaPerTile; ++i) dma_v1(tile, stage, i);
     };
 
+    // The loop's steps come in groups of four with fixed stages (step U of a
+    // group: key tile jj with jj + off = U mod 4). Key tiles are padded to an
+    // even count: off = 2 shifts every tile by two stages, so that the steps
+    // start in the middle of a group and the last one still has U = 3. (The
+    // wide forms, whose V window moves with the groups, and persistent
+    // launches, whose next-tile loads go to fixed stages, pad to a multiple of
+    // four. 40 heads of 1,296 x 1,296, 21 key tiles: 22 steps against 24.)
+    constexpr bool kEven = !kWide && !kPersist, kEarly = kEven && !kVT;
+    const int ntiles = (sk + kBN - 1) / kBN;
+    const int nsteps = kEven ? (ntiles + 1) & ~1 : (ntiles + 3) & ~3;
+    const int off = kEven ? nsteps & 2 : 0;
+    if (kEarly && ntiles == 0) {
+        // No keys: O = 0, LSE = -inf (never a piece: those hold keys).
+        const int wrow = m0 + wave * 32, rows = min(sq - wrow, 32);
+        char* const ob = (char*)p.o + 2 * (b * p.o_sb + h * p.o_sh) + (int64_t)(q0 + wrow) * p.o_rs;
+        for (int row = lane >> 4; row < rows; row += 4) *(i32x4*)(ob + (int64_t)row * p.o_rs + (lane & 15) * 16) = i32x4{};
+        if (lane < rows && p.lse != nullptr) p.lse[b * p.lse_sb + h * p.lse_sh + q0 + wrow + lane] = -INFINITY;
+        return false;
+    }
+    // Whether this wave's 32 rows lie past the last query row: it only keeps
+    // its share of the DMA and the barriers going, so that the SIMDs and the
+    // power it would take go to the other waves.
+    if (kEven && ntiles > 0 && m0 + wave * 32 >= sq) {
+        auto stage = [&](int t) { return (t + off) & 3; };
+        dma_k(0, stage(0));
+        dma_k(1, stage(1));
+        dma_v(0, stage(0));
+        dma_k(2, stage(2));
+        dma_v(1, stage(1));
+        dma_k(3, stage(3));
+        dma_v(2, stage(2));
+        wait_vmcnt<6 * kDmaPerTile>();
+        barrier();
+        barrier();
+        dma_k(4, stage(4));
+        wait_vmcnt<6 * kDmaPerTile>();
+        barrier();
+        wait_vmcnt<2 * kDmaPerTile>();
+        barrier();
+        for (int jj = 0; jj < nsteps; ++jj) {
+            if (jj < nsteps - 2) {
+                dma_k(jj + 5, stage(jj + 1));
+                dma_v(jj + 3, stage(jj + 3));
+            }
+            wait_vmcnt<2 * kDmaPerTile>();
+            barrier();
+        }
+        wait_vmcnt<0>();
+        return false;
+    }
+    // kEarly: the first loads go out before the accumulators and fragment
+    // addresses are set up (about 0.2 us a tile: 36 heads of 2,048 x 1,024, two
+    // rounds, 57.8 -> 57.5 us); the other forms would spill.
+    auto first_loads = [&]() __attribute__((always_inline)) {
+        load_q();
+        dma_k(0, off);
+        dma_k(1, 1 + off);
+        dma_v(0, off);
+        dma_k(2, 2 ^ off);
+        dma_v(1, 1 + off);
+        dma_k(3, 3 ^ off);
+        dma_v(2, 2 ^ off);
+    };
+    if constexpr (kEarly) first_loads();
+
     // K fragment of QK^T MFMA t (key block t & 1, head-dim step t >> 1): row
     // 32*(t & 1) + l32, logical chunk 2*(t >> 1) + hi.
     // The swizzle only moves bits 4-7 of an in-row byte offset, so every
@@ -400,7 +465,6 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
     }
 
     const float c = p.scale_log2;
-    const int ntiles = (sk + kBN - 1) / kBN;
 
     f32x16 oacc[4];
 #pragma unroll
@@ -686,58 +750,8 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
     constexpr std::integral_constant<int, 0> kNoSoftmax{};
     constexpr std::integral_constant<int, 1> kSoftmax{};
     constexpr std::integral_constant<int, 2> kFirstSoftmax{};
-    // The loop's steps come in groups of four with fixed stages (step U of a
-    // group: key tile jj with jj + off = U mod 4). Key tiles are padded to an
-    // even count: off = 2 shifts every tile by two stages, so that the steps
-    // start in the middle of a group and the last one still has U = 3. (The
-    // wide forms, whose V window moves with the groups, and persistent
-    // launches, whose next-tile loads go to fixed stages, pad to a multiple of
-    // four. 40 heads of 1,296 x 1,296, 21 key tiles: 22 steps against 24.)
-    constexpr bool kEven = !kWide && !kPersist;
-    const int nsteps = kEven ? (ntiles + 1) & ~1 : (ntiles + 3) & ~3;
-    const int off = kEven ? nsteps & 2 : 0;
-    // Whether this wave's 32 rows lie past the last query row: it only keeps
-    // its share of the DMA and the barriers going, so that the SIMDs and the
-    // power it would take go to the other waves.
-    if (kEven && m0 + wave * 32 >= sq && ntiles > 0) {
-        auto stage = [&](int t) { return (t + off) & 3; };
-        dma_k(0, stage(0));
-        dma_k(1, stage(1));
-        dma_v(0, stage(0));
-        dma_k(2, stage(2));
-        dma_v(1, stage(1));
-        dma_k(3, stage(3));
-        dma_v(2, stage(2));
-        wait_vmcnt<6 * kDmaPerTile>();
-        barrier();
-        barrier();
-        dma_k(4, stage(4));
-        wait_vmcnt<6 * kDmaPerTile>();
-        barrier();
-        wait_vmcnt<2 * kDmaPerTile>();
-        barrier();
-        for (int jj = 0; jj < nsteps; ++jj) {
-            if (jj < nsteps - 2) {
-                dma_k(jj + 5, stage(jj + 1));
-                dma_v(jj + 3, stage(jj + 3));
-            }
-            wait_vmcnt<2 * kDmaPerTile>();
-            barrier();
-        }
-        wait_vmcnt<0>();
-        return false;
-    }
-    if (ntiles > 0) {
-        if (issue) {
-            load_q();
-            dma_k(0, off);
-            dma_k(1, 1 + off);
-            dma_v(0, off);
-            dma_k(2, 2 ^ off);
-            dma_v(1, 1 + off);
-            dma_k(3, 3 ^ off);
-            dma_v(2, 2 ^ off);
-        }
+    if (kEarly || ntiles > 0) {
+        if (!kEarly && issue) first_loads();
         // Prefetched by the previous tile, in this order, before that
         // tile's O stores: the stores are younger, so each wait below only
         // gets stronger.
@@ -879,7 +893,7 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
         hi = lane >> 5;
         l32 = lane & 31;
     }
-    if (nsteps > 0) {
+    if (kEarly || nsteps > 0) {
         if (!kEven || nsteps > 2) {
             step(std::integral_constant<int, 0>{}, j, std::false_type{});
             step(std::integral_constant<int, 1>{}, j + 1, std::false_type{});
