@@ -59,12 +59,6 @@ bool short_segments_planned(const h3a_attn_args* a, int cus) {
     const ShortMix m = short_mix(a, cus);
     return m.varied && m.rounds >= 1.0 && (m.rounds <= 5.0 || (a->max_seqlen_q >= 2900 && m.rounds <= 9.0));
 }
-// Varied mixes of few rounds whose workspace has room for the planned list,
-// whichever launch they take.
-bool short_segments_plannable(const h3a_attn_args* a, int cus) {
-    const ShortMix m = short_mix(a, cus);
-    return m.varied && (m.rounds <= 3.2 || (a->max_seqlen_q >= 2900 && m.rounds <= 9.0));
-}
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 bool aligned4(const void* p) { return ((uintptr_t)p & 3u) == 0; }
@@ -258,7 +252,7 @@ struct AttnWorkspace {
 };
 
 AttnWorkspace attn_workspace(const h3a_attn_args* a, const h3a::AttnParams& p, bool allow_vt,
-                             int64_t max_workspace = INT64_MAX, bool plannable = false) {
+                             int64_t max_workspace = INT64_MAX) {
     if (p.n_units > 0) return AttnWorkspace{};
     AttnWorkspace w{attn_plan(a, p, max_workspace), 0, 0, 0, 0, 0, 0, false};
     w.total = w.plan.workspace_bytes;
@@ -271,8 +265,7 @@ AttnWorkspace attn_workspace(const h3a_attn_args* a, const h3a::AttnParams& p, b
         // the planning launch (max_seqlen_q bounds them).
         const int cus = device_cus();
         if (!allow_vt || cus <= 0) return w;
-        if (a->max_seqlen_q < kPlanMinSegment && !short_segments_planned(a, cus) &&
-            !(plannable && short_segments_plannable(a, cus))) {
+        if (a->max_seqlen_q < kPlanMinSegment && !short_segments_planned(a, cus)) {
             // Short segments: the persistent launch's tile counter.
             if (a->max_seqlen_q <= h3a::attn_fwd_persist_max_rows() && w.total + 256 <= max_workspace) {
                 w.persist = true;
@@ -489,7 +482,7 @@ int64_t h3a_attn_fwd_workspace_size(const h3a_attn_args* a) {
     if (empty) return 0;
     // What all tiles would take (a launch that runs as units leaves it unused),
     // or the whole tiles alone beside their ragged rows' units.
-    const int64_t tiles = attn_workspace(a, p, true, INT64_MAX, true).total;
+    const int64_t tiles = attn_workspace(a, p, true).total;
     take_rag_units(a, p);
     const int64_t whole = attn_workspace(a, p, true).total;
     return tiles > whole ? tiles : whole;

@@ -134,8 +134,7 @@ extern "C" {
  *     segment lengths vary (max_seqlen_q at least 1.6 times seqlen_q /
  *     num_segments) over one to five rounds of tiles (heads x (seqlen_q / 256
  *     + num_segments / 2) per CU; up to nine with max_seqlen_q of 2,900 or
- *     more), such calls take the planned work list above instead; the size has
- *     room for it also where lengths vary over less than a round.
+ *     more), such calls take the planned work list above instead.
  * With a workspace given, short attention (up to about 256 units of 32 query
  * rows of one head and 2,048 keys, or more units over fewer keys) runs without
  * using it, as one workgroup per unit with the keys split over its waves; so

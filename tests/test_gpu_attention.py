@@ -437,7 +437,7 @@ def test_workspace_plan_on_this_device():
     assert need(1, 64, 1) == 0  # one key tile: nothing to split, no d-major V
 
 
-def _varlen_workspace(lens, H):
+def _varlen_workspace(lens, H, keys=None):
     import ctypes
 
     from h3_flash_amd import _ext
@@ -446,12 +446,14 @@ def _varlen_workspace(lens, H):
     a = _ext.AttnArgs()
     a.abi_version = _ext.ABI_VERSION
     a.q = a.k = a.v = a.o = 1 << 20
-    a.batch, a.heads, a.seqlen_q, a.seqlen_k, a.head_dim = 1, H, S, S, 128
+    a.batch, a.heads, a.seqlen_q, a.seqlen_k, a.head_dim = 1, H, S, S if keys is None else int(sum(keys)), 128
     for name in ("q_stride", "k_stride", "v_stride", "o_stride"):
         getattr(a, name)[:] = (S * H * 128, H * 128, 128)
     a.lse_stride[:] = (H * S, S)
     a.softmax_scale = 0.088
     a.cu_seqlens_q = a.cu_seqlens_k = 1 << 20
+    if keys is not None:
+        a.cu_seqlens_k = 1 << 21
     a.num_segments, a.max_seqlen_q = len(lens), int(max(lens))
     return _ext.load_library().h3a_attn_fwd_workspace_size(ctypes.byref(a))
 
@@ -459,12 +461,11 @@ def _varlen_workspace(lens, H):
 def test_short_segments_route_by_length_spread():
     """Packed calls whose longest segment has fewer than 4,096 rows run on
     the persistent launch (its 256-byte tile counter) unless their lengths
-    vary (the longest at least 1.6 times the mean) and there are few tiles
-    per CU (at most 3.2 rounds, or 9 with segments of 2,900 rows or more):
-    then the planned list (no tiles past a segment's rows, longest segments
-    first, the last round as key-range pieces) balances the CUs. The
-    workspace each asks for tells the two apart. The planned route then
-    matches the oracle on sampled rows of its segments."""
+    vary (the longest at least 1.6 times the mean) over one to five rounds of
+    tiles per CU (nine with segments of 2,900 rows or more): then the planned
+    list (longest key ranges first) balances the CUs. The workspace each asks for
+    tells the two apart. The planned route then matches the oracle on sampled
+    rows of its segments."""
 
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the rule's rounds are stated for a 256-CU part")
@@ -475,10 +476,12 @@ def test_short_segments_route_by_length_spread():
     assert _varlen_workspace([2048] * 8, 5) == 256  # equal lengths, 1.3 rounds: persistent
     assert _varlen_workspace(ragged_short, 5) == 256  # varied, 5.3 rounds of short tiles: persistent
     assert _varlen_workspace(ragged_long, 5) > 256  # varied, 6.6 rounds, tiles up to 64 key tiles: planned
-    tiny = [3000] + [40] * 30
-    assert _varlen_workspace(tiny, 5) > 256  # varied, 0.6 rounds: planned
+    tiny, mixed = [3000] + [40] * 30, [3900, 40, 2500, 7, 1200, 3100, 64, 900]
+    assert _varlen_workspace(tiny, 5) == 256  # varied, 0.6 rounds: persistent
+    assert _varlen_workspace(mixed, 2) == 256  # varied, 0.4 rounds: persistent
 
-    for lens, H, seed in ((tiny, 5, 31), ([3900, 40, 2500, 7, 1200, 3100, 64, 900], 2, 32)):
+    # 1.25 and 1.6 rounds, and 4.3 over 48 segments
+    for lens, H, seed in ((tiny, 10, 31), (mixed, 8, 32), (torch.randint(1, 2049, (48,), generator=g).tolist(), 5, 33)):
         assert _varlen_workspace(lens, H) > 256
         cu = torch.tensor([0, *torch.cumsum(torch.tensor(lens), 0).tolist()], dtype=torch.int32)
         S = int(cu[-1])
