@@ -33,17 +33,20 @@ constexpr int64_t kVtMinKeys = 16384;
 constexpr int64_t kPlanMinSegment = 4096;
 
 // Shorter segments run on the persistent launch (varied lengths claimed by
-// length, longest first), unless the planned list, whose last round is cut into
-// key-range pieces, balances the CUs better than its planning and merge
-// launches cost (about 12 us): with varied lengths from about one round on.
+// length, longest first), unless the planned list balances the CUs better than
+// its planning and merge launches cost (about 12 us): with varied lengths from
+// about one round on (its workgroups are dispatched one tile each as CUs free
+// up, with no claim between tiles, and every tile follows from the list).
 // Timed on 50 mixes of 1 to 4,095 rows at 1 to 8 heads (us, persistent /
 // planned): 48 segments up to 2,048 rows, 3.8 rounds 205 / 190; 16 up to 1,916,
 // 1.2 rounds 87 / 73; 24 up to 567, 1.05 rounds 44 / 37; 42 up to 1,056, 3.3
 // rounds 122 / 110; 39 up to 2,130, 4.9 rounds 262 / 250; but 14 up to 3,233,
 // 0.4 rounds 69 / 84; 12 up to 984, 0.85 rounds 37 / 45; equal lengths, 48 of
-// 1,024 145 / 158; past five rounds the two are level. The host knows only the
-// packed rows, the segment count and the longest segment, so "varied" is the
-// longest against the mean.
+// 1,024 145 / 158; past five rounds the two are level. (None of these mixes
+// has a key range of 96 key tiles, so the list cut no pieces there.) The host
+// knows only the packed rows, the segment count and the longest segment, so
+// "varied" is the longest against the mean.
+constexpr int64_t kLongKeys = 6144;  // key ranges from here on are cut into pieces (96 key tiles)
 struct ShortMix {
     bool varied;
     double rounds;
@@ -57,7 +60,14 @@ ShortMix short_mix(const h3a_attn_args* a, int cus) {
 }
 bool short_segments_planned(const h3a_attn_args* a, int cus) {
     const ShortMix m = short_mix(a, cus);
-    return m.varied && m.rounds >= 1.0 && (m.rounds <= 5.0 || (a->max_seqlen_q >= 2900 && m.rounds <= 9.0));
+    if (!m.varied) return false;
+    if (a->max_seqlen_q >= 2900 && m.rounds >= 1.0 && m.rounds <= 9.0) return true;
+    // Key offsets of their own: a key range may be long, which the list starts
+    // early and cuts into pieces from 96 key tiles on (us, persistent / planned:
+    // 8 segments of 1 to 2,000 rows against 7,000 keys each, 5 heads, 0.45 rounds
+    // 141 / 116), unless all keys together are fewer than that.
+    if (a->cu_seqlens_k != a->cu_seqlens_q && a->seqlen_k >= kLongKeys) return m.rounds <= 3.2;
+    return m.rounds >= 1.0 && m.rounds <= 5.0;
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }

@@ -134,7 +134,9 @@ extern "C" {
  *     segment lengths vary (max_seqlen_q at least 1.6 times seqlen_q /
  *     num_segments) over one to five rounds of tiles (heads x (seqlen_q / 256
  *     + num_segments / 2) per CU; up to nine with max_seqlen_q of 2,900 or
- *     more), such calls take the planned work list above instead.
+ *     more; any number up to 3.2 when cu_seqlens_k is not cu_seqlens_q and
+ *     seqlen_k is 6,144 or more), such calls take the planned work list above
+ *     instead.
  * With a workspace given, short attention (up to about 256 units of 32 query
  * rows of one head and 2,048 keys, or more units over fewer keys) runs without
  * using it, as one workgroup per unit with the keys split over its waves; so

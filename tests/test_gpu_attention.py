@@ -462,10 +462,11 @@ def test_short_segments_route_by_length_spread():
     """Packed calls whose longest segment has fewer than 4,096 rows run on
     the persistent launch (its 256-byte tile counter) unless their lengths
     vary (the longest at least 1.6 times the mean) over one to five rounds of
-    tiles per CU (nine with segments of 2,900 rows or more): then the planned
-    list (longest key ranges first) balances the CUs. The workspace each asks for
-    tells the two apart. The planned route then matches the oracle on sampled
-    rows of its segments."""
+    tiles per CU (nine with segments of 2,900 rows or more) or, with key
+    offsets of their own and 6,144 keys or more, up to 3.2: then the planned
+    list (longest key ranges first, long ones in pieces) balances the CUs. The
+    workspace each asks for tells the two apart. The planned route then
+    matches the oracle on sampled rows of its segments."""
 
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the rule's rounds are stated for a 256-CU part")
@@ -479,6 +480,10 @@ def test_short_segments_route_by_length_spread():
     tiny, mixed = [3000] + [40] * 30, [3900, 40, 2500, 7, 1200, 3100, 64, 900]
     assert _varlen_workspace(tiny, 5) == 256  # varied, 0.6 rounds: persistent
     assert _varlen_workspace(mixed, 2) == 256  # varied, 0.4 rounds: persistent
+    assert _varlen_workspace(mixed, 2, mixed) > 256  # key offsets of its own: planned
+    assert _varlen_workspace(mixed, 2, [700] * 8) == 256  # unless its keys are few
+    assert _varlen_workspace([500, 20, 300, 100] * 2, 5, [7000] * 8) > 256  # long key ranges: planned
+    assert _varlen_workspace(ragged_short[:50], 5, ragged_short[:50]) == 256  # 4.5 rounds: persistent
 
     # 1.25 and 1.6 rounds, and 4.3 over 48 segments
     for lens, H, seed in ((tiny, 10, 31), (mixed, 8, 32), (torch.randint(1, 2049, (48,), generator=g).tolist(), 5, 33)):
