@@ -184,8 +184,9 @@ int device_cus() {
 }
 
 // Units per (group, head) of a launch that runs as units of 32 rows (short
-// attention), or 0 where the 256-row tiles are faster.
-int32_t attn_units(const h3a_attn_args* a, const h3a::AttnParams& p) {
+// attention), or 0 where the 256-row tiles are faster. list: a packed launch
+// may take the planned list.
+int32_t attn_units(const h3a_attn_args* a, const h3a::AttnParams& p, bool list) {
     const int cus = device_cus();
     if (p.wide != 0 || cus <= 0) return 0;
     const int64_t rows = a->cu_seqlens_q != nullptr ? a->max_seqlen_q : a->seqlen_q;
@@ -195,9 +196,12 @@ int32_t attn_units(const h3a_attn_args* a, const h3a::AttnParams& p) {
     // -> units): 5 x 640 x 640 14.5 -> 9.0, 10 x 640 x 640 18.5 -> 9.4, 4 x
     // 2,048 x 2,048 25.3 -> 18.5, 10 x 1,024 x 1,024 24.5 -> 22.1; 4 x 640 x
     // 4,096 24.6 -> 25.1, 5 x 2,048 x 2,048 28.6 -> 32.7, 40 x 640 x 640 26.5
-    // -> 34.7.
+    // -> 34.7. Few units over long key ranges lose to tiles in pieces: 1 x 64 x
+    // 2,500 19.8 -> 19.4, x 4,000 24.2 -> 25.1, x 8,000 36 -> 44, x 50,000 153
+    // -> 238; 40 x 1 x 2,500 27.8 -> 24.8, x 4,000 32 -> 35.
     if (a->cu_seqlens_q == nullptr) {
         const int64_t units = n * p.heads * p.n_groups;
+        if (a->seqlen_k > 3072) return 0;
         return (units <= cus && a->seqlen_k <= 2048) || (units <= 2 * cus && units * a->seqlen_k <= 400000) ? (int32_t)n : 0;
     }
     // Packed: by the expected time of either, from the units there can be (the
@@ -207,10 +211,21 @@ int32_t attn_units(const h3a_attn_args* a, const h3a::AttnParams& p) {
     // 0.9 per 64 keys + 0.018 per unit (planning launch, the longest tile, the
     // work), rounds of units 4.3 us + 1.5 per 256 keys, a tenth more with
     // ragged ends; this picked the faster one for all but one (0.84 of it).
+    // The planned list runs a long key range in up to four pieces (by the mean
+    // range, the longest taken for twice that), for some 30 us of launches: 3
+    // segments of up to 2,000 rows against up to 30,000 keys, 5 heads, 93 us in
+    // tiles, 151 in units; 6 of up to 600 against up to 12,000, 5 heads, 90 / 66.
     const int64_t units = p.heads * (a->seqlen_q / h3a::attn_fwd_unit_rows() + (int64_t)a->num_segments);
-    const int64_t keys = a->cu_seqlens_k == a->cu_seqlens_q ? a->max_seqlen_q : a->seqlen_k;
-    const double tiles_us = 13.0 + 0.9 / 64.0 * (double)keys + 0.018 * (double)units;
-    const double units_us = 1.1 * (double)((units + cus - 1) / cus) * (4.3 + 1.5 * (double)((keys + 255) / 256));
+    const double mean = (double)a->seqlen_k / a->num_segments;
+    double keys = a->cu_seqlens_k == a->cu_seqlens_q ? (double)a->max_seqlen_q : (double)a->seqlen_k;
+    double base_us = 13.0, pieces = 1.0;
+    if (list && mean > kLongKeys / 2 && (a->max_seqlen_q >= kPlanMinSegment || short_segments_planned(a, cus))) {
+        base_us = 30.0;
+        pieces = fmin(mean / (kLongKeys / 2), (double)h3a::attn_fwd_tail_pieces());
+        keys = fmin(keys, 2.0 * mean);
+    }
+    const double tiles_us = base_us + 0.9 / 64.0 * keys / pieces + 0.018 * (double)units;
+    const double units_us = 1.1 * (double)((units + cus - 1) / cus) * (4.3 + 1.5 * ceil(keys / 256.0));
     return units_us < tiles_us ? (int32_t)n : 0;
 }
 
@@ -412,7 +427,7 @@ int h3a_attn_fwd(const h3a_attn_args* a, void* stream) {
     // told where the launch takes one.
     const bool ask = a->workspace == nullptr && a->workspace_bytes == H3A_WORKSPACE_ASK;
     if (ask || a->workspace != nullptr) {
-        p.n_units = attn_units(a, p);
+        p.n_units = attn_units(a, p, true);
         if (p.n_units == 0) take_rag_units(a, p);
     }
     const AttnWorkspace w = attn_workspace(a, p, true);
@@ -451,7 +466,7 @@ int h3a_attn_fwd_noalloc(const h3a_attn_args* a, void* stream) {
     bool empty = false;
     const int rc = prepare_attn(a, p, &empty);
     if (rc != H3A_OK || empty) return rc;
-    p.n_units = attn_units(a, p);
+    p.n_units = attn_units(a, p, false);
     if (p.n_units > 0) {
         const hipError_t e = h3a::launch_attn_fwd(p, (hipStream_t)stream);
         if (e != hipSuccess) return fail(H3A_ELAUNCH, "h3a_attn_fwd_noalloc: launch failed: %s", hipGetErrorString(e));

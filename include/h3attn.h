@@ -138,7 +138,8 @@ extern "C" {
  *     seqlen_k is 6,144 or more), such calls take the planned work list above
  *     instead.
  * With a workspace given, short attention (up to about 256 units of 32 query
- * rows of one head and 2,048 keys, or more units over fewer keys) runs without
+ * rows of one head and 2,048 keys, more units over fewer keys, fewer ones over
+ * up to 3,072; packed calls by an expected time) runs without
  * using it, as one workgroup per unit with the keys split over its waves; so
  * may, beside the tiles, the rows past a dense call's whole tiles when they are
  * at most 32 and the tiles are not cut into pieces.

@@ -8,7 +8,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from h3_flash_amd import flash_attn_func
+from h3_flash_amd import _ext, flash_attn_func
 from oracle.attention import sdpa_reference
 from tests.test_gpu_attention import _varlen_workspace, assert_parity
 
@@ -84,6 +84,46 @@ def test_short_attention(B, H, Sq, Sk):
         return
     ref_out, ref_lse = sdpa_reference(q, k, v)
     assert_parity(out.cpu(), lse.cpu(), ref_out, ref_lse, f"{B}x{H}x{Sq}x{Sk}")
+
+
+def _runs_as_units(Sq, Sk, H, offsets=None):
+    """Whether the call launches without a workspace (asked for, one would be
+    named where tiles are cut into pieces)."""
+    q, k, v = (torch.zeros((1, S, H, 128), dtype=torch.bfloat16, device=DEV) for S in (Sq, Sk, Sk))
+    out, s = torch.empty_like(q), H * 128
+    cq, ck, longest = (None, None, 0) if offsets is None else offsets
+    rc = _ext.attn_fwd(
+        DEV, _ext.ABI_VERSION, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), 0, 1, H, Sq, Sk, 128,
+        *(Sq * s, s, 128), *(Sk * s, s, 128), *(Sk * s, s, 128), *(Sq * s, s, 128), 0, 0, 0.1, 0,
+        *((0, 0, 0, 0) if cq is None else (cq.data_ptr(), ck.data_ptr(), cq.numel() - 1, longest)),
+        0, _ext.H3A_WORKSPACE_ASK,
+    )
+    assert rc in (_ext.H3A_OK, _ext.H3A_NEED_WORKSPACE)
+    torch.cuda.synchronize()
+    return rc == _ext.H3A_OK
+
+
+# Units pass all keys of their head: over long key ranges tiles in key-range
+# pieces are shorter, few units or many.
+@pytest.mark.parametrize(
+    "H, Sq, Sk, units",
+    [(1, 64, 2500, True), (5, 640, 640, True), (1, 64, 8000, False), (1, 1, 50000, False), (4, 256, 4000, False), (16, 1, 20000, False)],
+)
+def test_units_by_key_range(H, Sq, Sk, units):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the rule was timed on a 256-CU part")
+    assert _runs_as_units(Sq, Sk, H) == units
+
+
+@pytest.mark.parametrize(
+    "H, qlens, klens, units",
+    [(5, [1900, 30, 400], [30000, 26000, 24000], False), (1, [60, 3], [60000, 40000], False), (2, [500, 20, 300], [900, 800, 700], True)],
+)
+def test_packed_units_by_key_range(H, qlens, klens, units):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the rule was timed on a 256-CU part")
+    cq, ck = (torch.tensor([0, *torch.tensor(x).cumsum(0).tolist()], dtype=torch.int32, device=DEV) for x in (qlens, klens))
+    assert _runs_as_units(sum(qlens), sum(klens), H, (cq, ck, max(qlens))) == units
 
 
 @pytest.mark.parametrize("qlens, klens", [([5, 0, 64, 33], [70, 9, 0, 300]), ([1], [1]), ([200, 31, 32], [200, 31, 32])])
