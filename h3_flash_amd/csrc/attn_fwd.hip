@@ -430,12 +430,15 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
         wait_vmcnt<0>();
         return false;
     }
-    // kEarly: the first loads go out before the accumulators and fragment
-    // addresses are set up (about 0.2 us a tile: 36 heads of 2,048 x 1,024, two
-    // rounds, 57.8 -> 57.5 us); the other forms would spill.
+    // kEarly: Q and K_0, which the first QK^T waits for, go out before the
+    // accumulators and fragment addresses are set up, the other loads after
+    // that (all at once, the last wave's Q would queue behind the first wave's
+    // V_2); the other forms would spill.
     auto first_loads = [&]() __attribute__((always_inline)) {
         load_q();
         dma_k(0, off);
+    };
+    auto more_loads = [&]() __attribute__((always_inline)) {
         dma_k(1, 1 + off);
         dma_v(0, off);
         dma_k(2, 2 ^ off);
@@ -751,7 +754,10 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
     constexpr std::integral_constant<int, 1> kSoftmax{};
     constexpr std::integral_constant<int, 2> kFirstSoftmax{};
     if (kEarly || ntiles > 0) {
-        if (!kEarly && issue) first_loads();
+        if (issue) {
+            if constexpr (!kEarly) first_loads();
+            more_loads();
+        }
         // Prefetched by the previous tile, in this order, before that
         // tile's O stores: the stores are younger, so each wait below only
         // gets stronger.
