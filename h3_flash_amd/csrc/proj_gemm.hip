@@ -119,6 +119,13 @@ __device__ __forceinline__ void unpack8(const i32x4& raw, float* f) {
     }
 }
 
+// Eight norm weights, of which only 8-byte alignment is known.
+__device__ __forceinline__ void load_w8(const void* w, int col0, float* f) {
+    const i32x2* const a = (const i32x2*)((const uint16_t*)w + col0);
+    const i32x2 lo = a[0], up = a[1];
+    unpack8(i32x4{lo.x, lo.y, up.x, up.y}, f);
+}
+
 // A tile shape: TF features x 16*NT tokens; SW stages of W rows, SX of X rows.
 template <int TF, int NT, int SW, int SX>
 struct Tile {
@@ -226,7 +233,7 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
     const int half = R >> 1, col0 = 8 * j;
     const float eps = sec.eps;
     float wv[8], wp[8];
-    unpack8(*(const i32x4*)((const uint16_t*)sec.norm_w + col0), wv);
+    load_w8(sec.norm_w, col0, wv);
 
     // Norm and RoPE of the tile's rows: kForm 0: no rotary columns, 1: R a
     // multiple of 16 and tables with 16-byte rows (3: R = 128, every lane
@@ -240,7 +247,7 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
         uint32_t pmask[4];
         // Partner weights with the rotation's sign, zero past R.
         if constexpr (kLanes) {
-            unpack8(*(const i32x4*)((const uint16_t*)sec.norm_w + 8 * pj), wp);
+            load_w8(sec.norm_w, 8 * pj, wp);
 #pragma unroll
             for (int e = 0; e < 8; ++e) wp[e] = !rot ? 0.f : first ? -wp[e] : wp[e];
         }

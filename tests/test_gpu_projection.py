@@ -102,6 +102,20 @@ def check_qkv(x, w, b, nwq, nwk, cos, sin, seqlen, y, rows=None, eps=1e-6):
     assert_matches(ys[:, 2 * n :], projection_reference(xs, w[2 * n :], bb(2)), "v")
 
 
+def test_norm_weights_at_eight_byte_alignment():
+    # the least alignment the entry point takes: a view eight bytes past an
+    # aligned allocation gives the bits of an aligned copy
+    x, w, b, nwq, nwk = make(200, 256, 1, 128, True, seed=3)
+    cos, sin = tables(200, 128)
+    buf = torch.empty(2 * 136, dtype=torch.bfloat16, device=DEV)
+    views = buf[4:132], buf[136:][4:132]
+    for view, nw in zip(views, (nwq, nwk)):
+        view.copy_(nw)
+        assert view.data_ptr() % 16 == 8
+    got = run_qkv(x, w, b, *views, cos, sin, 200)
+    assert torch.equal(got, run_qkv(x, w, b, nwq, nwk, cos, sin, 200))
+
+
 @pytest.mark.parametrize("M", [40, 3000])
 @pytest.mark.parametrize("R", [128, 96, 42, 0])
 def test_edge_magnitudes(M, R):
