@@ -895,7 +895,7 @@ int h3a_proj_gemm(const h3a_proj_args* a, void* stream) {
             return fail(H3A_EINVAL, "%s: section %d: strides must be multiples of 8 elements covering the row", fn, i);
         if (!spans(tile - 1, s.weight_stride, a->k * 2))
             return fail(H3A_EUNSUPPORTED, "%s: section %d: weight_stride too large", fn, i);
-        // A wave's output resource spans half a tile of token rows.
+        // (Rows of y are addressed in 64 bits; the bound keeps what was refused.)
         if (!spans(tile / 2 - 1, s.y_stride, 256))
             return fail(H3A_EUNSUPPORTED, "%s: section %d: y_stride too large", fn, i);
         if (s.bias && ((uintptr_t)s.bias & 7u) != 0)
@@ -929,13 +929,12 @@ int h3a_proj_gemm(const h3a_proj_args* a, void* stream) {
         p.table_stride = a->table_stride;
         p.rotary_dim = (int32_t)R;
         p.seqlen = (int32_t)a->seqlen;
-        // The in-lane epilogue (partners in the same lane, only the first
-        // half of the tables read) needs R a multiple of 32, the caller's
-        // word that the tables are in the rotate-half form, and 16-byte
-        // table rows; anything else reads the tables at every column.
-        const bool in_lane = R % 32 == 0 && a->rotate_half_tables == 1 && aligned16(a->cos) && aligned16(a->sin) &&
+        // Half of the tables is read where the caller's word is that they are
+        // in the rotate-half form (the form is checked for R a multiple of 32)
+        // and their rows are 16-byte aligned; else every column.
+        const bool half_tables = R % 32 == 0 && a->rotate_half_tables == 1 && aligned16(a->cos) && aligned16(a->sin) &&
                              a->table_stride % 4 == 0;
-        p.rope_full_tables = in_lane ? 0 : 1;
+        p.rope_full_tables = half_tables ? 0 : 1;
     } else {
         p.rotary_dim = 0;
         p.seqlen = 1;

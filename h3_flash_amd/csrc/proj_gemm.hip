@@ -155,26 +155,26 @@ struct Tile {
 // accumulators, rounds to bf16 (as the module's linear outputs it) and writes
 // the values into the tile's output rows in LDS: token t, head h of the tile
 // (128 features) at byte t * 2 TF + 256 h, its 16-byte chunk c at c ^ (t & 15)
-// (both passes bank-conflict free). Then 16 lanes take one (token, head) row
-// at a time, 16 bytes each: plain rows go out as they are; norm rows are
-// RMS-normalised in fp32 (sum of squares over the 16 lanes by DPP), scaled by
-// the norm weight, rotated and rounded once more, as the reference's separate
-// steps do (dense_fa4.py:123-140, transformer.py:146-173; normalising the
-// unrounded accumulator moves the LSE of the attention that follows by up to
-// about 2e-3 against that order). Rows go out as whole 256-byte pieces,
-// non-temporal (no later tile reads them). RoPE partners c +- R/2: with R a
-// multiple of 16 another lane's 8 columns, read from the row in LDS;
-// otherwise any_r_partners. cos / sin of the next token are loaded before the
-// current one is computed, once for the heads of the tile.
+// (both passes bank-conflict free). Then rows go out: plain ones as they are,
+// 16 lanes each; norm rows are RMS-normalised in fp32 (sum of squares over the
+// row's lanes by DPP), scaled by the norm weight, rotated and rounded once more,
+// as the reference's separate steps do (dense_fa4.py:123-140,
+// transformer.py:146-173; normalising the unrounded accumulator moves the LSE of
+// the attention that follows by up to about 2e-3 against that order). With R a
+// multiple of 16, 8 lanes take a row and each holds both columns of its pairs;
+// otherwise 16 lanes, the partners c +- R/2 through any_r_partners. Stores are
+// non-temporal (no later tile reads the rows), whole 128-byte lines. cos / sin
+// of the next token are loaded before the current one is computed, once for the
+// heads of the tile.
 // Bound by VALU issue (one wave per SIMD, the matrix cores idle), and on long
-// launches by the power it draws: the weights are multiplied into the token's
-// tables once for the tile's heads, so that a rotated value takes four
-// instructions (with the norm and the rotation applied one after the other,
-// and both selected per column, 49,920 tokens x 40 heads took 5,905 us, now
-// 5,745; the epilogue in the accumulator layout, 4 lanes x 32 columns of a
-// head, 5,710). At R = 126, where that layout read partners and tables element
-// by element, the q/k/v launch of 1,296 tokens went from 332 to 205 us with the
-// tile shape of that launch; 6,240 tokens at R = 128 from 748 to 730.
+// launches by the power it draws. So the weights are multiplied into the token's
+// tables once for the tile's heads, and a pair's two values are unpacked and
+// scaled once: with 16 lanes a row, each unpacking its partners again, 49,920
+// tokens x 40 heads took 5,730 us, 6,240 x 40 725, 6,240 x 5 26.6; now 5,600,
+// 712 and 23.5 (the epilogue in the accumulator layout, 4 lanes x 32 columns of
+// a head, 5,624, 722 and 25.9). At R = 126, where that layout read partners and
+// tables element by element, 1,296 x 40 went from 322 to 226 us, in part by the
+// tile shape.
 template <typename T>
 __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoord& tc, const f32x4 (&acc)[T::NA][T::NB],
                                          int wn, int wm, int tid, char* smem) {
@@ -230,67 +230,156 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
                 if (h < heads) store_row(t, h, load_row(t, h, j));
         return;
     }
-    const int half = R >> 1, col0 = 8 * j;
     const float eps = sec.eps;
+    const bool tab16 = (((uintptr_t)p.cos | (uintptr_t)p.sin) & 15) == 0 && (p.table_stride & 3) == 0;
+    auto table_row = [&](int t) {
+        int s = tc.m0 + min(t, tokens - 1);
+        s = s < p.seqlen ? s : s % p.seqlen;
+        return (int64_t)s * p.table_stride;
+    };
+
+    // R a multiple of 16 and tables with 16-byte rows: eight lanes take a row,
+    // each one two 16-byte chunks that rotate with each other (columns 8 j and
+    // R/2 on), or two of those past R. kAll: R = 128, every lane rotary. kFull:
+    // the tables are read at both chunks' columns, else at the first's, the
+    // halves being equal. A wave's eight rows of one access are two tokens' t
+    // and t + 8 over, so that each 16 lanes read 16 different bank groups.
+    auto pair_rows = [&](auto all_c, auto full_c) __attribute__((always_inline)) {
+        constexpr bool kAll = decltype(all_c)::value, kFull = decltype(full_c)::value;
+        const int j8 = lane & 7, g8 = lane >> 3, wave = tid >> 6;
+        const int row0 = 16 * (wave >> 1) + 4 * (wave & 1) + (g8 >> 1) + 8 * (g8 & 1);  // of every 32 tokens
+        const int np = kAll ? 8 : R >> 4;
+        const bool rot = kAll || j8 < np;
+        const int ca = rot ? j8 : 2 * j8, cb = rot ? j8 + np : 2 * j8 + 1;
+        float wa[8], wb[8];
+        load_w8(sec.norm_w, 8 * ca, wa);
+        load_w8(sec.norm_w, 8 * cb, wb);
+        constexpr int kTabs = kFull ? 4 : 2;
+        struct Tabs {
+            f32x4 c[kTabs], s[kTabs];
+        };
+        const int ta_col = rot ? 8 * ca : 0, tb_col = rot ? 8 * cb : 0;
+        auto load_tables = [&](int t) __attribute__((always_inline)) {
+            Tabs w;
+            const float* const cr = p.cos + table_row(t);
+            const float* const sr = p.sin + table_row(t);
+#pragma unroll
+            for (int i = 0; i < kTabs; ++i) {
+                const int c = (i < 2 ? ta_col : tb_col) + 4 * (i & 1);
+                w.c[i] = *(const f32x4*)(cr + c);
+                w.s[i] = *(const f32x4*)(sr + c);
+            }
+            return w;
+        };
+        auto token = [&](int t, const Tabs& tab) __attribute__((always_inline)) {
+            // y = (x r) (w cos) + (x' r) (w' sin): the weights times the tables
+            // are the token's, shared by its heads. r comes first, as in the
+            // separate steps: a row whose squares overflow fp32 (r = 0) gives
+            // zeros, and small rows lose no bits to a subnormal product.
+            float ta[8], tb[8], sa[8], sb[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float c0 = tab.c[e >> 2][e & 3], s0 = tab.s[e >> 2][e & 3];
+                const float c1 = tab.c[(kFull ? 2 : 0) + (e >> 2)][e & 3], s1 = tab.s[(kFull ? 2 : 0) + (e >> 2)][e & 3];
+                ta[e] = rot ? wa[e] * c0 : wa[e];
+                tb[e] = rot ? wb[e] * c1 : wb[e];
+                sa[e] = rot ? -(wb[e] * s0) : -0.f;
+                sb[e] = rot ? wa[e] * s1 : -0.f;
+            }
+            char* const yr = (char*)sec.y + (int64_t)(tc.m0 + t) * sec.y_rs + (int64_t)tc.f0 * 2;
+#pragma unroll
+            for (int h = 0; h < kHeads; ++h) {
+                if (h >= heads) break;
+                float xa[8], xb[8];
+                unpack8(load_row(t, h, ca), xa);
+                unpack8(load_row(t, h, cb), xb);
+                float ss = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) ss += xa[e] * xa[e];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) ss += xb[e] * xb[e];
+                const float r = rsqrtf(group_sum<8>(ss) * (1.0f / 128.0f) + eps);
+                float oa[8], ob[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float na = xa[e] * r, nb = xb[e] * r;
+                    oa[e] = na * ta[e] + (rot ? nb : 0.f) * sa[e];
+                    ob[e] = nb * tb[e] + (rot ? na : 0.f) * sb[e];
+                }
+                i32x4 va, vb;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    va[e] = (int)pack_bf16x2(oa[2 * e], oa[2 * e + 1]);
+                    vb[e] = (int)pack_bf16x2(ob[2 * e], ob[2 * e + 1]);
+                }
+                if (t < tokens) {
+                    __builtin_nontemporal_store(va, (i32x4*)(yr + h * 256 + 16 * ca));
+                    __builtin_nontemporal_store(vb, (i32x4*)(yr + h * 256 + 16 * cb));
+                }
+            }
+        };
+        const int n = (tokens + 31) / 32;
+        Tabs t0 = load_tables(row0);
+        int it = 0, t = row0;
+        for (; it + 2 <= n; it += 2, t += 64) {
+            const Tabs t1 = load_tables(t + 32);
+            token(t, t0);
+            t0 = load_tables(t + 64);
+            token(t + 32, t1);
+        }
+        if (it < n) token(t, t0);
+    };
+    if (R > 0 && (R & 15) == 0 && tab16) {
+        if (R == 128 && p.rope_full_tables == 0)
+            pair_rows(std::true_type{}, std::false_type{});
+        else if (R == 128)
+            pair_rows(std::true_type{}, std::true_type{});
+        else if (p.rope_full_tables == 0)
+            pair_rows(std::false_type{}, std::false_type{});
+        else
+            pair_rows(std::false_type{}, std::true_type{});
+        return;
+    }
+
+    // No rotary columns, or (kRope) any even R and tables at any alignment:
+    // sixteen lanes a row.
+    const int half = R >> 1, col0 = 8 * j;
     float wv[8], wp[8];
     load_w8(sec.norm_w, col0, wv);
-
-    // Norm and RoPE of the tile's rows: kForm 0: no rotary columns, 1: R a
-    // multiple of 16 and tables with 16-byte rows (3: R = 128, every lane
-    // rotary), 2: any even R.
-    auto rows = [&](auto form_c) __attribute__((always_inline)) {
-        constexpr int kForm = decltype(form_c)::value;
-        constexpr bool kLanes = kForm == 1 || kForm == 3;
-        const bool rot = kForm == 3 || (kForm == 1 && col0 < R);
-        const bool first = col0 < half;
-        const int pj = rot ? (first ? j + (half >> 3) : j - (half >> 3)) : j;  // partner lane (kLanes)
+    auto rows = [&](auto rope_c) __attribute__((always_inline)) {
+        constexpr bool kRope = decltype(rope_c)::value;
         uint32_t pmask[4];
-        // Partner weights with the rotation's sign, zero past R.
-        if constexpr (kLanes) {
-            load_w8(sec.norm_w, 8 * pj, wp);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) wp[e] = !rot ? 0.f : first ? -wp[e] : wp[e];
-        }
-        if constexpr (kForm == 2) {
+        if constexpr (kRope) {
+            // Partner weights with the rotation's sign, zero past R.
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const int c = min(col0 + e, R - 1);
                 const float w = bf16_to_f32(((const uint16_t*)sec.norm_w)[c < half ? c + half : c - half]);
-                wp[e] = col0 + e >= R ? 0.f : c < half ? -w : w;
+                wp[e] = c < half ? -w : w;
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) pmask[i] = col0 + 2 * i < R ? 0xffffffffu : 0u;
         }
-        // Tables of a rotate-half pair are equal in both halves: reading the
-        // first alone halves their cache traffic.
-        const int tcol = !kLanes ? 0 : !rot ? 0 : (p.rope_full_tables == 0 && !first) ? col0 - half : col0;
         const bool pairs = (((uintptr_t)p.cos | (uintptr_t)p.sin) & 7) == 0 && (p.table_stride & 1) == 0;  // uniform
         struct Tabs {
             f32x4 c[2], s[2];  // cos and sin of the lane's 8 columns
         };
         auto load_tables = [&](int t) __attribute__((always_inline)) {
             Tabs w{};
-            if constexpr (kForm != 0) {
-                int s = tc.m0 + min(t, tokens - 1);
-                s = s < p.seqlen ? s : s % p.seqlen;
-                const float* const cr = p.cos + (int64_t)s * p.table_stride;
-                const float* const sr = p.sin + (int64_t)s * p.table_stride;
+            if constexpr (kRope) {
+                const float* const cr = p.cos + table_row(t);
+                const float* const sr = p.sin + table_row(t);
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    if constexpr (kLanes) {
-                        w.c[i] = *(const f32x4*)(cr + tcol + 4 * i);
-                        w.s[i] = *(const f32x4*)(sr + tcol + 4 * i);
+                    const int c0 = min(col0 + 4 * i, R - 2), c1 = min(col0 + 4 * i + 2, R - 2);
+                    if (pairs) {
+                        const f32x2 a = *(const f32x2*)(cr + c0), b = *(const f32x2*)(cr + c1);
+                        const f32x2 c = *(const f32x2*)(sr + c0), d = *(const f32x2*)(sr + c1);
+                        w.c[i] = f32x4{a.x, a.y, b.x, b.y};
+                        w.s[i] = f32x4{c.x, c.y, d.x, d.y};
                     } else {
-                        const int c0 = min(col0 + 4 * i, R - 2), c1 = min(col0 + 4 * i + 2, R - 2);
-                        if (pairs) {
-                            const f32x2 a = *(const f32x2*)(cr + c0), b = *(const f32x2*)(cr + c1);
-                            const f32x2 c = *(const f32x2*)(sr + c0), d = *(const f32x2*)(sr + c1);
-                            w.c[i] = f32x4{a.x, a.y, b.x, b.y};
-                            w.s[i] = f32x4{c.x, c.y, d.x, d.y};
-                        } else {
-                            w.c[i] = f32x4{cr[c0], cr[c0 + 1], cr[c1], cr[c1 + 1]};
-                            w.s[i] = f32x4{sr[c0], sr[c0 + 1], sr[c1], sr[c1 + 1]};
-                        }
+                        w.c[i] = f32x4{cr[c0], cr[c0 + 1], cr[c1], cr[c1 + 1]};
+                        w.s[i] = f32x4{sr[c0], sr[c0 + 1], sr[c1], sr[c1 + 1]};
                     }
                 }
             }
@@ -300,16 +389,14 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
         // the wave's, so every lane joins the row sums and partner reads.
         const int t_end = (tokens - 4 * (g >> 2) + 15) / 16;  // iterations of this wave
         auto token = [&](int t, const Tabs& tab) __attribute__((always_inline)) {
-            // y = (x r) (w cos) + (x' r) (w' sin): the weights times the tables
-            // are the token's, shared by its heads. r comes first, as in the
-            // separate steps: a row whose squares overflow fp32 (r = 0) gives
-            // zeros, and small rows lose no bits to a subnormal product.
-            float tc_[8], ts_[8];
+            float tc_[8], ts_[8];  // as above
+            if constexpr (kRope) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const bool in = kLanes ? rot : kForm == 2 && col0 + e < R;
-                tc_[e] = in ? wv[e] * tab.c[e >> 2][e & 3] : wv[e];
-                ts_[e] = in ? wp[e] * tab.s[e >> 2][e & 3] : 0.f;
+                for (int e = 0; e < 8; ++e) {
+                    const bool in = col0 + e < R;
+                    tc_[e] = in ? wv[e] * tab.c[e >> 2][e & 3] : wv[e];
+                    ts_[e] = in ? wp[e] * tab.s[e >> 2][e & 3] : -0.f;
+                }
             }
 #pragma unroll
             for (int h = 0; h < kHeads; ++h) {
@@ -321,18 +408,13 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
 #pragma unroll
                 for (int e = 0; e < 8; ++e) ss += xv[e] * xv[e];
                 const float r = rsqrtf(group_sum<16>(ss) * (1.0f / 128.0f) + eps);
-                if constexpr (kForm == 0) {
+                if constexpr (!kRope) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) o[e] = (xv[e] * r) * wv[e];
                 } else {
-                    i32x4 px;
-                    if constexpr (kLanes) {
-                        px = load_row(t, h, pj);
-                    } else {
-                        px = any_r_partners(out + T::kOutBytes + g * T::kPartner, x, j, R);
+                    i32x4 px = any_r_partners(out + T::kOutBytes + g * T::kPartner, x, j, R);
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) px[i] &= (int)pmask[i];
-                    }
+                    for (int i = 0; i < 4; ++i) px[i] &= (int)pmask[i];
                     float xp[8];
                     unpack8(px, xp);
 #pragma unroll
@@ -354,15 +436,10 @@ __device__ __forceinline__ void epilogue(const ProjGemmParams& p, const TileCoor
         }
         if (it < t_end) token(t, t0);
     };
-    const bool tab16 = (((uintptr_t)p.cos | (uintptr_t)p.sin) & 15) == 0 && (p.table_stride & 3) == 0;
     if (R == 0)
-        rows(std::integral_constant<int, 0>{});
-    else if (R == 128 && tab16)
-        rows(std::integral_constant<int, 3>{});
-    else if ((R & 15) == 0 && tab16)
-        rows(std::integral_constant<int, 1>{});
+        rows(std::false_type{});
     else
-        rows(std::integral_constant<int, 2>{});
+        rows(std::true_type{});
 }
 
 template <int TF, int NT, int SW, int SX>

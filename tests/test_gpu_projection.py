@@ -102,6 +102,22 @@ def check_qkv(x, w, b, nwq, nwk, cos, sin, seqlen, y, rows=None, eps=1e-6):
     assert_matches(ys[:, 2 * n :], projection_reference(xs, w[2 * n :], bb(2)), "v")
 
 
+@pytest.mark.parametrize("R", [16, 48, 64, 112, 128])
+@pytest.mark.parametrize("M, full", [(31, False), (33, True), (300, False), (300, True)])
+def test_rotary_pairs_of_whole_chunks(M, R, full):
+    # rotary widths of an odd and an even number of 16-column pairs, with the
+    # columns past them, on token counts around the 32 that a pass takes; tables
+    # in the rotate-half form or different in every column
+    heads = 3  # a last feature tile of one head
+    x, w, b, nwq, nwk = make(M, 256, heads, R, True, seed=R + M)
+    cos, sin = tables(M, R)
+    if full:
+        g = torch.Generator().manual_seed(R)
+        cos, sin = torch.rand((M, R), generator=g) - 0.5, torch.rand((M, R), generator=g) - 0.5
+    y = run_qkv(x, w, b, nwq, nwk, cos, sin, M, rotate_half=not full and R % 32 == 0)
+    check_qkv(x, w, b, nwq, nwk, cos, sin, M, y)
+
+
 def test_norm_weights_at_eight_byte_alignment():
     # the least alignment the entry point takes: a view eight bytes past an
     # aligned allocation gives the bits of an aligned copy
