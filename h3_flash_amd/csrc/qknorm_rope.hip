@@ -90,10 +90,12 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
     const int tid = threadIdx.x;
     const int j = tid % L;
     const int s = (int)blockIdx.x * kGroups + tid / L;  // token
-    const int64_t b = blockIdx.z;
+    const bool apart = kAnyR && !kCopy && p.tensors_apart != 0;
+    const int64_t b = apart ? blockIdx.z >> 1 : blockIdx.z;
     const int D = p.head_dim, R = p.rotary_dim, half = R >> 1;
-    const int hb = p.head_first + (int)blockIdx.y * kChunk;  // this block's heads: [hb, H)
-    const int H = min(p.heads, hb + kChunk);
+    const int chunk = kAnyR ? p.head_chunk : kChunk;
+    const int hb = p.head_first + (int)blockIdx.y * chunk;  // this block's heads: [hb, H)
+    const int H = min(p.heads, hb + chunk);
     const int col0 = j * 8;
     const bool on = s < p.seqlen && col0 < D;
     const bool rot = col0 < R;
@@ -257,7 +259,8 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
         }
     } else {
         // Tensor by tensor, each tensor's loads issued first.
-        for (int which = 0; which < p.n_tensors; ++which) {
+        const int from = apart ? (int)blockIdx.z & 1 : 0, to = apart ? from + 1 : p.n_tensors;
+        for (int which = from; which < to; ++which) {
             const bool second = which != 0;
             const void* w = second ? p.w[1] : p.w[0];
             const float eps = second ? p.eps[1] : p.eps[0];
@@ -288,13 +291,33 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
 template <int L, bool kAnyR>
 hipError_t launch_l(QkNormRopeParams p, hipStream_t stream) {
     const int64_t batch = p.rows / ((int64_t)p.seqlen * p.n_tensors * p.heads);
-    const int chunk = p.xc != nullptr ? kHeadChunkCopy : kHeadChunk;
+    const int64_t token_blocks = (p.seqlen + kThreads / L - 1) / (kThreads / L);
+    int chunk = p.xc != nullptr ? kHeadChunkCopy : kHeadChunk;
+    p.tensors_apart = 0;
+    if (kAnyR) {
+        // Few workgroups: q and k apart and fewer heads each, so that no row
+        // waits for others. Where all heads of both tensors, eight a workgroup,
+        // give up to about 1,024 workgroups, two are faster than one: 5 heads of
+        // 6,240 tokens (780) 12.5 us against 14.0, of 12,480 (1,560) level, of
+        // 49,920 66 against 63. Heads: as few as stay within 1,024 workgroups:
+        // 5 heads of 640 tokens 5.3 us with one (800), 6.2 with eight; of 1,300
+        // 6.2 with two (978), 7.1 with one, 7.2 with eight; the pack of 640 rows
+        // x 8 heads 7.0 with one (640), 9.7 with four; x 40 heads 11.7 with four
+        // (800), 17.0 with one. (One row per lane group: 6.5, 13.6, 7.9, 45.6.)
+        const int64_t blocks = token_blocks * batch, few = 1024;
+        p.tensors_apart = p.xc == nullptr && p.n_tensors == 2 && 2 * batch <= 65535 &&
+                          blocks * ((p.heads + chunk - 1) / chunk) <= few;
+        const int64_t per_head = blocks * (p.tensors_apart != 0 ? 2 : 1);
+        const int most = chunk;
+        for (chunk = 1; chunk < most && per_head * ((p.heads + chunk - 1) / chunk) > few;) chunk *= 2;
+    }
+    p.head_chunk = chunk;
     const int chunks = (p.heads + chunk - 1) / chunk;
     // (Head chunks past the grid's 65,535 in y go into further launches.)
     for (int first = 0; first < chunks; first += 65535) {
         p.head_first = first * chunk;
-        const dim3 grid((unsigned)((p.seqlen + kThreads / L - 1) / (kThreads / L)), (unsigned)min(chunks - first, 65535),
-                        (unsigned)batch);
+        const dim3 grid((unsigned)token_blocks, (unsigned)min(chunks - first, 65535),
+                        (unsigned)(p.tensors_apart != 0 ? 2 * batch : batch));
         if (p.xc != nullptr)
             hipLaunchKernelGGL((qknorm_rope_kernel<L, true, kAnyR>), grid, dim3(kThreads), 0, stream, p);
         else

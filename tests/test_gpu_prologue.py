@@ -191,3 +191,20 @@ def test_partners_across_lanes(D, R, tables):
         cos, sin = (t[:, at : at + R] for t in wide)
     y = fused_qknorm_rope(x.to(DEV), w.to(DEV), cos, sin, 1e-5)
     assert_rounding_parity(y, qknorm_rope_reference(x, w, cos.cpu(), sin.cpu(), 1e-5), (D, R, tables))
+
+
+# Launches of few and of many workgroups: q and k in workgroups of their own or
+# one, heads by one, two, four and eight to a workgroup, the last one partial.
+@pytest.mark.parametrize("B, S, H", [(1, 1, 1), (2, 21, 13), (1, 100, 40), (1, 640, 13), (3, 700, 7), (1, 3000, 11), (1, 9000, 9)])
+def test_q_and_k_across_launch_sizes(B, S, H):
+    D, R = 128, 126
+    q, k = _rand((B, S, H, D), S + H), _rand((B, S, H, D), S + H + 1)
+    wq, wk = (torch.randn(D, generator=torch.Generator().manual_seed(s)).to(torch.bfloat16) for s in (3, 4))
+    ang = torch.randn((S, R), generator=torch.Generator().manual_seed(5))
+    cos, sin = ang.cos(), ang.sin()
+    dev = [t.to(DEV) for t in (q, k, wq, wk, cos, sin)]
+    oq, ok = fused_qk_norm_rope(*dev, 1e-5, 1e-6)
+    assert torch.equal(oq, fused_qknorm_rope(dev[0], dev[2], dev[4], dev[5], 1e-5))
+    rows = sorted({0, S // 2, S - 1})
+    assert_rounding_parity(oq[:, rows], qknorm_rope_reference(q[:, rows], wq, cos[rows], sin[rows], 1e-5), ("q", B, S, H))
+    assert_rounding_parity(ok[:, rows], qknorm_rope_reference(k[:, rows], wk, cos[rows], sin[rows], 1e-6), ("k", B, S, H))
