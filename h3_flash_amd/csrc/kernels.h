@@ -151,9 +151,9 @@ struct QkNormRopeParams {
     const float* sin;
     int64_t table_stride;
     int64_t rows;  // batch * seqlen * n_tensors * heads, < 2^31
-    // Set by the launcher: first head of the launch's grid, heads per workgroup,
-    // and 1 where q and k go to workgroups of their own.
-    int32_t head_first, head_chunk, tensors_apart;
+    // Set by the launcher (any rotary width): heads per workgroup, and 1 where q
+    // and k go to workgroups of their own.
+    int32_t head_chunk, tensors_apart;
     int32_t seqlen;
     int32_t heads;
     int32_t n_tensors;  // 1 (q only) or 2 (q and k)

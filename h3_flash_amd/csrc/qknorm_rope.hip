@@ -90,11 +90,17 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
     const int tid = threadIdx.x;
     const int j = tid % L;
     const int s = (int)blockIdx.x * kGroups + tid / L;  // token
-    const bool apart = kAnyR && !kCopy && p.tensors_apart != 0;
-    const int64_t b = apart ? blockIdx.z >> 1 : blockIdx.z;
+    // (The form without kAnyR takes nothing from the launch that it need not:
+    // its code stays as it was tuned.)
+    bool apart = false;
+    int64_t b = blockIdx.z;
+    if constexpr (kAnyR && !kCopy) {
+        apart = p.tensors_apart != 0;
+        if (apart) b = blockIdx.z >> 1;
+    }
     const int D = p.head_dim, R = p.rotary_dim, half = R >> 1;
     const int chunk = kAnyR ? p.head_chunk : kChunk;
-    const int hb = p.head_first + (int)blockIdx.y * chunk;  // this block's heads: [hb, H)
+    const int hb = (int)blockIdx.y * chunk;  // this block's heads: [hb, H)
     const int H = min(p.heads, hb + chunk);
     const int col0 = j * 8;
     const bool on = s < p.seqlen && col0 < D;
@@ -143,16 +149,12 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
         sv[0] = s0.x; sv[1] = s0.y; sv[2] = s0.z; sv[3] = s0.w; sv[4] = s1.x; sv[5] = s1.y; sv[6] = s1.z; sv[7] = s1.w;
     }
 
-    // Norm weights of the lane's partner columns.
+    // Norm weights of the lane's partner columns (kAnyR).
     auto load_wp = [&](const void* w, float* wp) __attribute__((always_inline)) {
-        if constexpr (kAnyR) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int c = min(col0 + e, R - 1);
-                wp[e] = load_w(w, c < half ? c + half : c - half, wf);
-            }
-        } else if (on && rot) {
-            load_w8(w, src * 8, wf, wp);
+        for (int e = 0; e < 8; ++e) {
+            const int c = min(col0 + e, R - 1);
+            wp[e] = load_w(w, c < half ? c + half : c - half, wf);
         }
     };
     // Normalise, rotate and store one row chunk (all L lanes of the group join
@@ -244,7 +246,8 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
         for (int which = 0; which < 2; ++which) {
             float wv[8], wp[8];
             if (on) load_w8(p.w[which], col0, wf, wv);
-            load_wp(p.w[which], wp);
+            if constexpr (kAnyR) load_wp(p.w[which], wp);
+            else if (on && rot) load_w8(p.w[which], src * 8, wf, wp);
 #pragma unroll
             for (int i = 0; i < kChunk; ++i) {
                 if (i >= nh) break;  // uniform
@@ -260,7 +263,7 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
     } else {
         // Tensor by tensor, each tensor's loads issued first.
         const int from = apart ? (int)blockIdx.z & 1 : 0, to = apart ? from + 1 : p.n_tensors;
-        for (int which = from; which < to; ++which) {
+        for (int which = kAnyR ? from : 0; which < (kAnyR ? to : p.n_tensors); ++which) {
             const bool second = which != 0;
             const void* w = second ? p.w[1] : p.w[0];
             const float eps = second ? p.eps[1] : p.eps[0];
@@ -272,7 +275,8 @@ __global__ __launch_bounds__(kThreads, kCopy ? 3 : 4) void qknorm_rope_kernel(Qk
                            (int64_t)s * (second ? p.y_ss[1] : p.y_ss[0]) + col0;
             float wv[8], wp[8];
             if (on) load_w8(w, col0, wf, wv);
-            load_wp(w, wp);
+            if constexpr (kAnyR) load_wp(w, wp);
+            else if (on && rot) load_w8(w, src * 8, wf, wp);
             i32x4 raw[kChunk];
 #pragma unroll
             for (int i = 0; i < kChunk; ++i) {
@@ -308,15 +312,30 @@ hipError_t launch_l(QkNormRopeParams p, hipStream_t stream) {
         p.tensors_apart = p.xc == nullptr && p.n_tensors == 2 && 2 * batch <= 65535 &&
                           blocks * ((p.heads + chunk - 1) / chunk) <= few;
         const int64_t per_head = blocks * (p.tensors_apart != 0 ? 2 : 1);
-        const int most = chunk;
-        for (chunk = 1; chunk < most && per_head * ((p.heads + chunk - 1) / chunk) > few;) chunk *= 2;
+        const int widest = chunk;
+        for (chunk = 1; chunk < widest && per_head * ((p.heads + chunk - 1) / chunk) > few;) chunk *= 2;
     }
     p.head_chunk = chunk;
-    const int chunks = (p.heads + chunk - 1) / chunk;
-    // (Head chunks past the grid's 65,535 in y go into further launches.)
-    for (int first = 0; first < chunks; first += 65535) {
-        p.head_first = first * chunk;
-        const dim3 grid((unsigned)token_blocks, (unsigned)min(chunks - first, 65535),
+    // Head chunks past the grid's 65,535 in y go into further launches, each
+    // from the views of its first head (whole groups of the output's heads).
+    const int64_t heads = p.heads, hpg = p.div_hpg.d, most = (int64_t)65535 * chunk;
+    const int64_t step = hpg >= heads ? most : most / hpg * hpg;
+    if (step == 0) return hipErrorInvalidValue;
+    const QkNormRopeParams all = p;
+    for (int64_t first = 0; first < heads; first += step) {
+        p.heads = (int32_t)(heads - first < step ? heads - first : step);
+        if (first > 0) {
+            const int64_t group = hpg >= heads ? 0 : first / hpg, in = first - group * hpg;
+            for (int i = 0; i < p.n_tensors; ++i) {
+                p.x[i] = (const uint16_t*)all.x[i] + first * all.x_sh[i];
+                p.y[i] = (uint16_t*)all.y[i] + group * all.y_sg[i] + in * all.y_sh[i];
+            }
+            if (p.xc != nullptr) {
+                p.xc = (const uint16_t*)all.xc + first * all.xc_sh;
+                p.yc = (uint16_t*)all.yc + group * all.yc_sg + in * all.yc_sh;
+            }
+        }
+        const dim3 grid((unsigned)token_blocks, (unsigned)((p.heads + chunk - 1) / chunk),
                         (unsigned)(p.tensors_apart != 0 ? 2 * batch : batch));
         if (p.xc != nullptr)
             hipLaunchKernelGGL((qknorm_rope_kernel<L, true, kAnyR>), grid, dim3(kThreads), 0, stream, p);

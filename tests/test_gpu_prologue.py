@@ -208,3 +208,16 @@ def test_q_and_k_across_launch_sizes(B, S, H):
     rows = sorted({0, S // 2, S - 1})
     assert_rounding_parity(oq[:, rows], qknorm_rope_reference(q[:, rows], wq, cos[rows], sin[rows], 1e-5), ("q", B, S, H))
     assert_rounding_parity(ok[:, rows], qknorm_rope_reference(k[:, rows], wk, cos[rows], sin[rows], 1e-6), ("k", B, S, H))
+
+
+# More head chunks than a grid has in y (eight heads each: 524,280 heads).
+@pytest.mark.parametrize("R", [16, 14, 0])
+def test_more_heads_than_one_launch_takes(R):
+    H, D = 524_300, 16
+    x = _rand((1, 1, H, D), R)
+    w = torch.randn(D, generator=torch.Generator().manual_seed(6)).to(torch.bfloat16)
+    ang = torch.randn((1, R), generator=torch.Generator().manual_seed(7))
+    y = fused_qknorm_rope(x.to(DEV), w.to(DEV), ang.cos().to(DEV), ang.sin().to(DEV), 1e-5)
+    heads = [0, 7, 524_279, 524_280, H - 1]
+    assert_rounding_parity(y[:, :, heads], qknorm_rope_reference(x[:, :, heads], w, ang.cos(), ang.sin(), 1e-5), R)
+    assert torch.isfinite(y.float()).all()

@@ -222,3 +222,15 @@ def test_single_gpu_ulysses_equality_gate(world, heads, base_rows):
     torch.cuda.synchronize()
     for s in range(world):
         assert torch.equal(merged[s].view(torch.int16), full_out[offs[s] : offs[s + 1]].view(torch.int16)), s
+
+
+@pytest.mark.parametrize("R", [16, 14])
+def test_fused_pack_of_more_heads_than_one_launch_takes(R):
+    # four heads a workgroup in y: 262,140 heads a launch, cut at a destination
+    heads, world, D = 262_160, 8, 16
+    q, k, v = (t.to(DEV) for t in torch.randn((3, 1, heads, D), generator=torch.Generator().manual_seed(R)).to(torch.bfloat16))
+    w = torch.ones(D, dtype=torch.bfloat16, device=DEV)
+    ang = torch.randn((1, R), generator=torch.Generator().manual_seed(3)).to(DEV)
+    packed = qknorm_rope_pack_qkv(q, k, v, w, w, ang.cos(), ang.sin(), 1e-5, 1e-6, world)
+    qn, kn = fused_qk_norm_rope(q.unsqueeze(0), k.unsqueeze(0), w, w, ang.cos(), ang.sin(), 1e-5, 1e-6)
+    assert torch.equal(packed, pack_qkv_destination_major(qn.squeeze(0), kn.squeeze(0), v, world))
