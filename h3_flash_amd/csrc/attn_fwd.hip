@@ -743,10 +743,10 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
     // last PV steps already read the first K fragments of tile j+3. At its
     // end vmcnt(4) leaves only its own loads in flight, so after the barrier
     // every wave sees K_{j+4} and V_{j+2} (issued at iteration j-1), the
-    // tiles iteration j+1 reads ahead. The loop runs a multiple of 4 iterations,
-    // unrolled so that every stage offset is a compile-time constant and S
-    // and P ping-pong between two register sets each; tiles past the end read
-    // as zeros and are fully masked.
+    // tiles iteration j+1 reads ahead. The loop is unrolled over groups of four
+    // iterations (nsteps is even, or a multiple of four), so that every stage
+    // offset is a compile-time constant and S and P ping-pong between two
+    // register sets each; tiles past the end read as zeros and are fully masked.
     f32x16 sa[2], sb[2];
     bf16x8 pfa[4], pfb[4];
     auto no_hook = [](int) {};
@@ -923,10 +923,10 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
     // This wave's 32 rows of O, normalised to bf16, written through its
     // 2 KB of V stage 3. The stage is free here: its last reader, the final
     // step's PV, finished before that step's barrier; a persistent launch's
-    // prefetch fills the other stages; a later call writes it only in its
-    // first main-loop step, and there each wave's DMA fills exactly its own
-    // 2 KB (eight 256-byte key rows, or sixteen 128-byte dim rows of a
-    // d-major tile) after its own reads here. A lane holds four dims of
+    // prefetch fills the other stages; a later call writes it no sooner than
+    // with its first loads, where each wave's DMA fills exactly its own 2 KB
+    // (eight 256-byte key rows, or sixteen 128-byte dim rows of a d-major
+    // tile) after its own reads here. A lane holds four dims of
     // every 8-dim block of one row; in four passes of 32 dims the lanes
     // write their pieces, then each reads back 16 bytes, four lanes one
     // row's 64 contiguous bytes, and stores them: 128 L2 requests per wave
@@ -959,11 +959,12 @@ __device__ __forceinline__ bool attn_tile(Params& p, int tile, int chunk, int ch
     };
     if (slot >= 0) {
         // Partial result of a key-range piece: normalised O and the LSE in
-        // fp32, every row of the wave. O in bf16 (as the output itself is
+        // fp32, all 32 rows of the wave. O in bf16 (as the output itself is
         // rounded), or in fp32 (kPartF32).
         if constexpr (kPartF32) {
             // As staged_store, 4 KB a wave over V stages 2 and 3 (both read for
-            // the last time by this call): rows of 128 bytes per 32 dims, the
+            // the last time by this call; before a next piece's loads come the
+            // queue's barriers): rows of 128 bytes per 32 dims, the
             // 16-byte chunks swizzled by row.
             typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
             lds_char* const staged = (lds_char*)(vst + 2 * kTile) + wave * 32 * 128;
@@ -1093,8 +1094,8 @@ __device__ __forceinline__ void attn_unit(Params& p, const UnitView& u) {
         const f32x2 hm = halves(mx);
         const float m_new = fmaxf(mc, fmaxf(hm.x, hm.y) * c);
         if (__builtin_amdgcn_ballot_w64(m_new > mc)) {
-            // (A row without a finite score so far has nothing to rescale:
-            // -inf less -inf would make NaN of it.)
+            // (A row all of whose scores so far overflowed to -inf has nothing
+            // to rescale: -inf less -inf would make NaN of it.)
             const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(mc - m_new);
             mc = m_new;
             l_run *= alpha;
@@ -1746,7 +1747,8 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
 #pragma unroll
     for (int c = 0; c < kMaxP; ++c) {
         if (c >= n) break;
-        // Every piece holds keys and writes all its rows; a -inf LSE would
+        // Every piece holds keys and writes its rows up to the last query row
+        // (waves past it write none, and none is read here); a -inf LSE would
         // still weigh nothing.
         const float w = lq[c] == -INFINITY ? 0.f : __expf(lq[c] - lse_max);
         wsum += w;

@@ -201,7 +201,8 @@ H3A_API int64_t h3a_attn_fwd_workspace_size(const h3a_attn_args *args);
  * or none), so any problem size runs; a plan that could not be fitted would
  * be rejected with H3A_EINVAL. Packed calls with max_seqlen_q below 4,096
  * run the persistent launch, its tile counter in the same array (also those
- * of varied lengths, whose planned list would not fit). The call allocates
+ * of varied lengths, whose planned list would not fit); short attention and
+ * ragged rows run as units, as with a workspace. The call allocates
  * nothing, issues no memset and does not synchronise.
  *
  * All calls on one GPU share its array: calls that overlap on one GPU (on
@@ -305,8 +306,8 @@ H3A_API int h3a_merge_heads(const h3a_merge_heads_args *args, void *stream);
  * of h3a_pack_qkv. Batch is 1 (the packed path's only case). Any even
  * rotary width up to head_dim, as for h3a_qknorm_rope; cos/sin 4-byte
  * aligned (a rotary width that is a multiple of 16 with 16-byte aligned
- * table rows takes the vectorised kernel, others an element-wise one with
- * the same results).
+ * table rows exchanges partners between lanes, others through LDS; same
+ * results).
  */
 typedef struct h3a_qknorm_rope_pack_args {
     int32_t abi_version;
@@ -495,10 +496,8 @@ H3A_API int h3a_attn_merge(const h3a_attn_merge_args *args, void *stream);
  * fusions.py:268-275); cos / sin fp32 (seqlen rows of table_stride >=
  * rotary_dim floats), 4-byte aligned. With rotary_dim a multiple of 32,
  * rotate_half_tables = 1 and 16-byte aligned table rows (table_stride a
- * multiple of 4), each lane holds its RoPE partners and only the tables'
- * first half is read; otherwise the partners come from the token's other
- * lanes through LDS and the tables are read at every rotated column (same
- * results). No workspace; nothing is allocated.
+ * multiple of 4) only the tables' first half is read, otherwise every rotated
+ * column (same results). No workspace; nothing is allocated.
  */
 #define H3A_PROJ_PLAIN 0
 #define H3A_PROJ_QKNORM_ROPE 1

@@ -180,6 +180,44 @@ def test_units_keep_rows_with_a_block_of_overflowed_scores(Sq, Sk, H, row, block
     assert_parity(out.cpu()[:, rows], lse.cpu()[:, :, rows], ref_out, ref_lse, f"{Sq}x{Sk} block {block}")
 
 
+# Scores that grow from block to block by far more than fp32 exponents hold
+# (every rescale taken), that shrink, and one key far above all others: units
+# of a dense and a packed call, ragged rows, and the pieces of a last round.
+@pytest.mark.parametrize("H, Sq, Sk, packed", [(2, 64, 700, False), (2, 64, 700, True), (40, 1296, 400, False), (20, 3500, 700, False)])
+@pytest.mark.parametrize("kind", ["rising", "falling", "peak"])
+def test_units_and_pieces_on_extreme_scores(H, Sq, Sk, packed, kind):
+    q, k, v = _qkv(1, Sq, Sk, H, Sq + Sk)
+    q[..., 0], k[..., 0] = 8.0, 0.0
+    ramp = torch.linspace(0, 3000, Sk).to(torch.bfloat16)  # scores up to 2,100
+    k[..., 0] = {"rising": ramp, "falling": ramp.flip(0), "peak": torch.eye(1, Sk)[0].roll(Sk // 2).to(torch.bfloat16) * 3000}[kind][:, None]
+    kw = dict(cu_seqlens_q=torch.tensor([0, Sq], dtype=torch.int32, device=DEV), max_seqlen_q=Sq,
+              cu_seqlens_k=torch.tensor([0, Sk], dtype=torch.int32, device=DEV)) if packed else {}
+    out, lse = flash_attn_func(q.to(DEV), k.to(DEV), v.to(DEV), **kw)
+    torch.cuda.synchronize()
+    h, rows = [0, H - 1], sorted({0, Sq // 2, max(0, Sq - Sq % 256 - 8), max(0, Sq - Sq % 256 - 1), Sq - 2, Sq - 1})
+    ref_out, ref_lse = sdpa_reference(q[:, rows][:, :, h], k[:, :, h], v[:, :, h])
+    m = (out.cpu()[:, rows][:, :, h].float() - ref_out).abs().max().item()
+    assert m <= 2e-2, m
+    # scores of thousands: their fp32 sum over 128 products carries 2^-24 of it a term
+    assert ((lse.cpu()[:, h][..., rows] - ref_lse).abs() <= 1e-3 + 2.0**-18 * ref_lse.abs()).all()
+
+
+# A NaN in one query row, and in one key: NaN where the row or the key takes part
+# and nowhere else, as from the tiles.
+@pytest.mark.parametrize("H, Sq, Sk, row", [(2, 64, 300, 5), (40, 1296, 100, 1290)])
+def test_nan_stays_in_its_rows(H, Sq, Sk, row):
+    q, k, v = (x.to(DEV) for x in _qkv(1, Sq, Sk, H, 11))
+    clean, _ = flash_attn_func(q, k, v)
+    q[0, row, 1, 7] = float("nan")
+    out, _ = flash_attn_func(q, k, v)
+    bad = torch.zeros((1, Sq, H), dtype=torch.bool, device=DEV)
+    bad[0, row, 1] = True
+    assert torch.isnan(out[bad]).all() and torch.equal(out[~bad], clean[~bad])
+    q[0, row, 1, 7], k[0, Sk // 2, 1, 3] = 0.0, float("nan")
+    out, _ = flash_attn_func(q, k, v)
+    assert torch.isnan(out[:, :, 1]).all() and torch.equal(out[:, :, 0], clean[:, :, 0])
+
+
 def test_packed_rows_up_to_the_tile_of_the_longest_segment():
     # max_seqlen_q counts in whole tiles of 256 rows on every route, units too
     q, k, v = (x.to(DEV) for x in _qkv(1, 330, 330, 2, 9))

@@ -2,9 +2,9 @@
 the reference's rounding order (the projection rounded to bf16, then the q/k
 RMSNorm + RoPE): plain sections and sections with the norm + RoPE epilogue,
 ragged token counts, half-width last tiles, rotary widths that are multiples
-of 32 (partners in the same lane, the tables' first half read) and any other
-even width or table form (partners from the token's other lanes, every
-rotated column read), more tiles than CUs (one workgroup per tile), the 480p
+of 16 (a lane holds both columns of a pair; of 32 in the rotate-half form: the
+tables' first half read) and any other even width or table alignment (partners
+from the token's other lanes, every rotated column read), more tiles than CUs (one workgroup per tile), the 480p
 rank and 40-head projection shapes (sampled rows), hipBLASLt's own linear,
 and the attention processor with fused projections and its fallback record."""
 

@@ -153,7 +153,7 @@ def test_fused_prologue_pack_equals_unfused(R, wdtype, heads, world):
     tc, ts = cos, sin
     if R == 96:
         # device tables with rows of 98 floats (not 16-byte rows), read in
-        # place: the element-wise kernel in the pack layout
+        # place: the form for any rotary width in the pack layout
         tc, ts = torch.zeros((rows, 98), device=DEV), torch.zeros((rows, 98), device=DEV)
         tc[:, :R], ts[:, :R] = cos.to(DEV), sin.to(DEV)
         tc, ts = tc[:, :R], ts[:, :R]
