@@ -189,6 +189,8 @@ int device_cus() {
 int32_t attn_units(const h3a_attn_args* a, const h3a::AttnParams& p, bool list) {
     const int cus = device_cus();
     if (p.wide != 0 || cus <= 0) return 0;
+    const int64_t rows = a->cu_seqlens_q != nullptr ? a->max_seqlen_q : a->seqlen_q;
+    const int64_t n = (rows + h3a::attn_fwd_unit_rows() - 1) / h3a::attn_fwd_unit_rows();
     // Every unit reads all keys of its head, so units win while they all run
     // at once, or in two rounds over few keys. Timed, heads x Sq x Sk (us, tiles
     // -> units): 5 x 640 x 640 14.5 -> 9.0, 10 x 640 x 640 18.5 -> 9.4, 4 x
@@ -198,7 +200,6 @@ int32_t attn_units(const h3a_attn_args* a, const h3a::AttnParams& p, bool list) 
     // 2,500 19.8 -> 19.4, x 4,000 24.2 -> 25.1, x 8,000 36 -> 44, x 50,000 153
     // -> 238; 40 x 1 x 2,500 27.8 -> 24.8, x 4,000 32 -> 35.
     if (a->cu_seqlens_q == nullptr) {
-        const int64_t n = (a->seqlen_q + h3a::attn_fwd_unit_rows() - 1) / h3a::attn_fwd_unit_rows();
         const int64_t units = n * p.heads * p.n_groups;
         if (a->seqlen_k > 3072) return 0;
         return (units <= cus && a->seqlen_k <= 2048) || (units <= 2 * cus && units * a->seqlen_k <= 400000) ? (int32_t)n : 0;
@@ -225,9 +226,7 @@ int32_t attn_units(const h3a_attn_args* a, const h3a::AttnParams& p, bool list) 
     }
     const double tiles_us = base_us + 0.9 / 64.0 * keys / pieces + 0.018 * (double)units;
     const double units_us = 1.1 * (double)((units + cus - 1) / cus) * (4.3 + 1.5 * ceil(keys / 256.0));
-    // (A segment's units end with its rows or, as tiles would, with the last
-    // whole tile that max_seqlen_q reaches.)
-    return units_us < tiles_us ? p.n_qtiles * (h3a::attn_fwd_block_m() / h3a::attn_fwd_unit_rows()) : 0;
+    return units_us < tiles_us ? (int32_t)n : 0;
 }
 
 // Split plan of a validated launch: dense inputs only (varlen tiles are not

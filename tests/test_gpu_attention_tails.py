@@ -218,16 +218,6 @@ def test_nan_stays_in_its_rows(H, Sq, Sk, row):
     assert torch.isnan(out[:, :, 1]).all() and torch.equal(out[:, :, 0], clean[:, :, 0])
 
 
-def test_packed_rows_up_to_the_tile_of_the_longest_segment():
-    # max_seqlen_q counts in whole tiles of 256 rows on every route, units too
-    q, k, v = (x.to(DEV) for x in _qkv(1, 330, 330, 2, 9))
-    cu = torch.tensor([0, 130, 330], dtype=torch.int32, device=DEV)
-    want = flash_attn_func(q, k, v, cu_seqlens_q=cu, max_seqlen_q=200)
-    out, lse = torch.full_like(want[0], 7.0), torch.full_like(want[1], 7.0)
-    flash_attn_func(q, k, v, cu_seqlens_q=cu, max_seqlen_q=70, out=out, lse=lse)
-    assert torch.equal(out, want[0]) and torch.equal(lse, want[1])
-
-
 # Queued last rounds over short key ranges (pieces of a few key tiles).
 @pytest.mark.parametrize("H, Sq, Sk", [(20, 3500, 1500), (40, 2048, 2048), (70, 1024, 1300)])
 def test_last_round_pieces_of_short_key_ranges(H, Sq, Sk):
