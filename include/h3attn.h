@@ -87,8 +87,8 @@ extern "C" {
  * [cu_seqlens_q[i], cu_seqlens_q[i+1]) of Q/O/LSE and rows
  * [cu_seqlens_k[i], cu_seqlens_k[i+1]) of K/V (cu_seqlens_k may equal
  * cu_seqlens_q). Both arrays are int32 device arrays of num_segments+1
- * entries; max_seqlen_q bounds every query segment. Attention is
- * block-diagonal: a query attends only to keys of its own segment.
+ * entries; max_seqlen_q bounds every query segment (rows of a longer one may
+ * stay unwritten). Attention is block-diagonal: a query attends only to keys of its own segment.
  *
  * Rows with no key (seqlen_k == 0) produce O = 0 and LSE = -inf.
  *
