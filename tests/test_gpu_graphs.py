@@ -139,3 +139,50 @@ def test_persistent_short_segment_launch_replays_in_a_graph(heads):
             )
             torch.cuda.synchronize()
             assert torch.equal(captured[0][:, a:e], alone[0]), replay
+
+
+def test_units_ragged_rows_and_short_pieces_replay_in_a_graph():
+    # short dense and packed calls as units (the packed segmentation changes
+    # between replays), ragged rows as units beside whole tiles, a last round
+    # over a short key range in pieces (fp32 partial results, counter reset by
+    # a recorded kernel), and the q/k prologue at a width through LDS
+    D = 128
+    q, k, v = (torch.empty((1, 600, 5, D), dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    q2, k2, v2 = (torch.empty((1, 1560, 40, D), dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    q3, k3, v3 = (torch.empty((1, 3500, 20, D), dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    w = torch.ones(D, dtype=torch.bfloat16, device=DEV)
+    ang = torch.randn((600, 126), device=DEV, generator=torch.Generator(device=DEV).manual_seed(1))
+    cos, sin = ang.cos(), ang.sin()
+    segmentations = ([0, 200, 400, 600], [0, 0, 300, 600], [0, 1, 33, 300], [0, 256, 257, 513], [0, 300, 300, 600])
+    cu = torch.tensor(segmentations[0], dtype=torch.int32, device=DEV)
+
+    def step():
+        qn, kn = fused_qk_norm_rope(q, k, w, w, cos, sin, 1e-5, 1e-6)
+        out = [qn, kn, *flash_attn_func(qn, kn, v)]
+        packed = torch.zeros_like(q)
+        packed_lse = torch.zeros((1, 5, 600), device=DEV)
+        flash_attn_func(q, k, v, cu_seqlens_q=cu, cu_seqlens_k=cu, max_seqlen_q=300, out=packed, lse=packed_lse)
+        return [*out, packed, packed_lse, *flash_attn_func(q2, k2, v2), *flash_attn_func(q3, k3, v3)]
+
+    inputs = [q, k, v, q2, k2, v2, q3, k3, v3]
+    _fill(inputs, 0)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    torch.cuda.synchronize()
+
+    for replay in range(4):
+        _fill(inputs, 300 + replay)
+        cu.copy_(torch.tensor(segmentations[replay + 1], dtype=torch.int32))
+        eager = [t.clone() for t in step()]
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for i, (got, want) in enumerate(zip(captured, eager)):
+            assert torch.equal(got, want), f"replay {replay}: output {i} differs from the eager launch"
